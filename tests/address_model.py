@@ -8,7 +8,7 @@ nothing on a GPU; the kernels' arithmetic is not computed, only where it
 goes. Cited lines are those of the kernel sources.
 
 Kernels covered (the FP8 and 2-byte pools share their addressing):
-- qk_norm_rope_store_kernel (qk_norm_rope.hip:55-111): q_out rows, cache rows
+- qk_norm_rope_store_kernel (qk_norm_rope.hip): q_out rows, cache rows
   by slot;
 - pack_metadata_kernel (metadata.hip:24-98): its output arrays;
 - decode_fast_kernel (head dims 64, 128, 256) with its inline work list or
@@ -158,12 +158,12 @@ def pow2ceil(x: int) -> int:
 
 
 # ---------------------------------------------------------------------------
-# Fused prologue (qk_norm_rope.hip:55-111)
+# Fused prologue (qk_norm_rope.hip)
 # ---------------------------------------------------------------------------
 
 def prologue(W: Writes, q_out: Buf, k_cache: Buf, v_cache: Buf, slots: np.ndarray, T: int, H: int,
              KV: int, num_blocks: int, bs: int, q_stride: int, fp8: bool, D: int = 128) -> None:
-    """One wave per (token, head) row; q rows to q_out, k / v rows by slot."""
+    """One workgroup per token; q rows to q_out, k / v rows by slot."""
     if T == 0:
         return
     t = np.arange(T, dtype=np.int64)

@@ -287,7 +287,7 @@ def test_planted_mistakes_are_reported():
 
 
 def test_head_dims_64_and_256():
-    """The fused prologue (two rows per wave at D 64, two rotate-half pairs
+    """The fused prologue (4, 8 or 16 lanes a row, eight rotate-half pairs
     per lane at D 256) and prefill at those head dims (prefill_kernel at 64,
     with its partials in the workspace the library sizes; the generic kernel
     at 256): every K/V row read and every store inside its buffer, over

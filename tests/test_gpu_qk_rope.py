@@ -136,8 +136,8 @@ def test_matches_composites(device, dtype, T, H, KV, pad):
 @pytest.mark.parametrize("T,H,KV,pad", [(1, 5, 1, 0), (37, 5, 1, 0), (130, 16, 4, 32),
                                         (257, 8, 2, 0)])
 def test_head_dims_64_and_256(device, dtype, hd, T, H, KV, pad):
-    """D 64: two rows per wave (an odd row count leaves the last wave half
-    idle); D 256: two rotate-half pairs per lane."""
+    """D 64: 4 lanes per row (an odd row count leaves lanes of the last wave
+    idle); D 256: 16 lanes per row."""
     print(f"qk_norm_rope_store D={hd} dtype={dtype} T={T} H={H} KV={KV} pad={pad}", flush=True)
     res, kc, vc, vref = _run(device, dtype, T, H, KV, pad=pad, seed=T + H + hd, D=hd)
     _check(res, kc, vc, vref, dtype, hd)
@@ -154,6 +154,35 @@ def test_norm_free_matches_composites(device, dtype, hd, T, H, KV, pad):
     res, kc, vc, vref = _run(device, dtype, T, H, KV, pad=pad, seed=T + H + hd + 1, D=hd,
                              norms=False)
     _check(res, kc, vc, vref, dtype, hd)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("H,KV", [(1, 1), (5, 1), (64, 8)])
+def test_off_16_byte_rows_match_aligned(device, hd, H, KV, fp8):
+    """Rows that do not start on 16 bytes take the element accesses: the same
+    bits as the 16-byte ones (each row's arithmetic is the same). 1 to 80 rows
+    per token: one pass of a part of a wave to several passes."""
+    dtype, T, nb, bs = torch.bfloat16, 19, 8, 16
+    print(f"qk_norm_rope_store unaligned D={hd} H={H} KV={KV} fp8={fp8}", flush=True)
+    qkv, qw, kw, slots, pos, inv_freq = _case(device, dtype, T, H, KV, nb, bs, seed=hd, D=hd)
+    width = (H + 2 * KV) * hd
+    odd = torch.zeros(T * (width + 3) + 1, dtype=dtype, device=device)[1:].view(T, width + 3)[:, :width]
+    odd.copy_(qkv)
+    assert odd.data_ptr() % 16 != 0 and odd.stride(0) % 8 != 0
+    got = []
+    for src in (qkv, odd):
+        cd = torch.uint8 if fp8 else dtype
+        kc = torch.full((nb, KV, bs, hd), 7, dtype=cd, device=device)
+        vc = kc.clone()
+        q = torch.empty(T, H, hd, dtype=dtype, device=device)
+        sc = torch.full((KV,), 1 / 16, device=device)
+        pk.qk_norm_rope_store(q, kc, vc, src, slots, pos, inv_freq, qw, kw, 1e-6,
+                              *((sc, sc) if fp8 else ()))
+        got.append((q, kc, vc))
+    torch.cuda.synchronize()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
 
 
 def test_one_norm_weight_is_refused(device):
