@@ -9,51 +9,55 @@
 // cache (the chunk's K/V are stored before the call, as the reference stores
 // them before attending, model_runner.py:146). For an empty prefix both agree.
 //
-// MI355X design (gfx950, v_mfma_f32_16x16x32_{bf16,f16}, wave64):
+// MI355X design (gfx950, v_mfma_f32_32x32x16_{bf16,f16}, wave64):
 //   head dim D = 64 or 128 (prefill_kernel<.., D, ..>; the other multiples
 //   of 32 up to 256 run prefill_generic_kernel below);
-//   workgroup = 8 waves = one (sequence, kv-head, head group, 64-row query
-//   tile, key split); wave w owns one query head and 32 query rows. Two waves
-//   per SIMD, 256 VGPRs each (MFMA operands stay in VGPRs). HW = gcd(G, 4)
-//   heads per workgroup, 4 / HW row tiles of 64 (G = 4: 4 heads x 64 rows).
-//   The 64-key K/V tile the workgroup gathers from the pool into LDS is read
-//   by all 8 waves (GQA and row reuse).
+//   workgroup = 8 waves = one (sequence, kv-head, tile of 256 rows, key part).
+//   Rows are (token, head) pairs of the kv head's G query heads, flattened as
+//   token * G + head: any G fills its tiles, and a wave's 32 rows span 32 / G
+//   tokens, so its causal range ends with the tile's. Two waves per SIMD, 256
+//   VGPRs each. All 8 waves read the 64-key K/V tiles that the workgroup
+//   gathers from the pool into LDS (GQA and row reuse).
 //   per step of 64 keys, each wave:
 //     S^T = K . Q^T   -- A = K rows from LDS, B = the wave's query rows, kept
 //                        in registers for the whole key loop;
-//     softmax          -- lane l holds 16 keys of query (mb*16 + l%16) of each
-//                        16-row block; the rest are in lanes l^16, l^32 (row
-//                        max / sum with v_permlane16/32_swap). Scale and max
-//                        subtraction are one FMA before exp2; the row sum is a
-//                        v_dot2 of the rounded P pair with (1, 1). The running
-//                        max is only moved (and O rescaled) when a row's new
-//                        max exceeds it by more than 2^kTau: P entries then
-//                        stay <= 2^kTau, exact in fp32 accumulation, and the
-//                        rescale is rare after the first step;
+//     softmax          -- lane l holds 32 keys of query row l % 32, lane l ^ 32
+//                        the others. Scale and reference are one FMA before
+//                        exp2; the row sum is a v_dot2 of the rounded P pair
+//                        with (1, 1). No maximum is taken in the usual step:
+//                        whether the reference must move is read off the packed
+//                        P values (past_bound), and only then the maxima are
+//                        taken, O rescaled and P formed again;
 //     O^T += V^T . P^T -- P^T is the S^T accumulator, already in B-operand
 //                        layout (packed with v_cvt_pk_bf16_f32); V stays
 //                        row-major in LDS like K, and the V^T A operand is two
 //                        ds_read_b64_tr_b16 (gfx950 transposing LDS read: in a
 //                        group of 16 lanes, lane j receives element j%4 of the
 //                        8-byte chunks addressed by lanes 4e + j/4, e = 0..3).
-//   The two waves of a SIMD are phase-shifted (one runs PV of the previous
-//   step before QK, the other after softmax), so one's softmax VALU work can
-//   run under the other's MFMAs. K/V loads run three steps ahead through a
-//   register ring, are copied into LDS (2 K, 3 V buffers) one step ahead, and
-//   keys past the visible range are clamped to the last visible key (a real,
-//   finite context row) and masked.
-//   Operand layouts of v_mfma_f32_16x16x32 (checked on the hardware):
-//     A[m = lane%16][k = 8*(lane/16) + e], B[k = 8*(lane/16) + e][n = lane%16],
-//     D[m = 4*(lane/16) + i][n = lane%16].
+//   K/V tiles load straight into LDS (global_load_lds, 16 bytes per lane),
+//   three steps ahead, with a swizzle in place of padded rows: no ring
+//   registers, no LDS stores. The two waves of a SIMD run half a step apart:
+//   one's MFMAs with the other's softmax. Keys past the visible range are
+//   clamped to the last visible key (a real, finite context row) and masked.
+//   Operand layouts of v_mfma_f32_32x32x16 (checked on the hardware):
+//     A[m = lane%32][k = 8*(lane/32) + e], B[k = 8*(lane/32) + e][n = lane%32],
+//     D[m = 8*(i/4) + 4*(lane/32) + i%4][n = lane%32].
 //
-// Key splits: a query tile whose key range is longer than ks_steps steps of 64
-// keys is cut into nsp <= splits_max ranges run by separate workgroups (the
-// tiles of a long prefix would otherwise run many times longer than the rest):
-// near-equal parts when the work list orders the items (at most 64 tiles),
-// else at multiples of ks_steps.
-// Each split publishes its unnormalised O, running max and row sum with
-// device-coherent stores, then takes a ticket from a per-tile counter; the last
-// of the nsp to arrive merges the others into its registers
+// What bounds it: power, then issue. 12000 tokens of 32 / 8 heads run at 3009
+// cycles per step against 2048 of MFMA, at 1.8 GHz (all-zero inputs, which draw
+// less, hold 2.4 GHz and take 0.76x the time): 1071 us = 1.10 PFLOP/s of useful
+// work, where a plain 8192^3 product reaches 1.47. Before (16x16x32 MFMAs, K/V
+// through a register ring, maxima in every step): 1383 us. A step without the
+// tile loads takes the same cycles at a higher clock; more operand reads ahead
+// (6 to 12) change nothing; the dot2 row sums cost 11 cycles each under the
+// other wave's MFMAs, 4 alone.
+//
+// Key splits: tiles are cut into nsp <= splits_max near-equal key parts run by
+// separate workgroups where that shortens the launch (prefill_item; in the
+// fixed order of very many tiles at ks_steps). Each part publishes its
+// unnormalised O, exponent reference and row sum with device-coherent stores,
+// then takes a ticket from a per-tile counter; the last of the nsp to arrive
+// merges the others into its registers
 //   M = max_j m_j,  L = sum_j l_j 2^(m_j - M),  O = sum_j O_j 2^(m_j - M) / L
 // writes the output and resets the counter to 0.
 #include <type_traits>
@@ -65,28 +69,36 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 8;        // waves per workgroup: 2 per SIMD
 constexpr int kThreads = 64 * kWaves;
-constexpr int kPairs = kWaves / 2;   // (head, 64-row tile) pairs, two 32-row waves each
-constexpr int kWaveRows = 32;    // query rows per wave
+constexpr int kWaveRows = 32;    // flattened (token, head) rows per wave
+constexpr int kTileRows = kWaves * kWaveRows;   // ... and per workgroup
 constexpr int kKT = 64;          // keys per step
-constexpr int kDepth = 3;        // K/V tiles in flight per workgroup
-// LDS row of the K and V tiles (elements) at head dim d: 72 dwords at 128,
-// 40 at 64 -- an 8-bank shift per row either way, so 16 rows of K read at one
-// column and 4 rows x 32 bytes of a transposing V read both hit distinct banks
-constexpr int lds_row(int d) { return d + 16; }
-constexpr int kMaxBlocksLds = 16384;  // block ids of one workgroup's key range kept in LDS (64 KB)
+constexpr int kBufK = 4;         // K tiles in LDS
+constexpr int kBufV = 5;         // V tiles in LDS
+constexpr int kListBlocks = 2048;     // blocks of the key range listed in LDS at a time (8 KB)
+constexpr int kMaxTableBlocks = 16384;  // widest block table accepted
+constexpr int kSchedMfma = 0x8, kSchedDsRead = 0x100;   // sched_group_barrier classes
+constexpr int kWaitVm0 = 0x0f70;       // s_waitcnt vmcnt(0), the other counters free
+constexpr float kNoRef = 3.402823466e38f;     // exponent offset of a row without a reference
 constexpr int kSplitSteps = 16;       // a key range longer than this many steps is split
 constexpr int kMaxSplits = 8;
-constexpr float kTau = 8.f;           // lazy-rescale threshold, log2 units
+constexpr int kAhead = 4;            // operand reads ahead of their MFMA
+constexpr int kSlots = 8;             // tiles per lane of the work list
+constexpr int kListTiles = 64 * kSlots;
+constexpr int kSmallDiv = 1 << 21;    // dividends small_div takes for any divisor
+constexpr int kMinPart = 4;           // shortest part the work list cuts (steps)
+constexpr int kItemSteps = 4;         // an item's prologue and output, in steps
+constexpr int kMergeSteps = 4;        // publishing and merging a part, in steps
 constexpr float kLog2e = 1.4426950408889634f;
-// partial record of one wave (32 rows of one head, one split) at head dim d,
-// floats: [nb*2 + mb][half][lane][2], nb < d / 16
+// partial record of one wave (32 rows, one split) at head dim d, floats:
+// [db*8 + i/2][lane][2] over the O^T accumulators, db < d / 32
 constexpr int rec_o(int d) { return d / 8 * 2 * 64 * 2; }
-constexpr int kRecML = 2 * 64 * 2;       // [mb][lane][m, l]
+constexpr int kRecML = 2 * 64 * 2;       // [lane][m, l] (half of it used)
 
 struct PrefillArgs {
   uint16_t* out;
@@ -101,9 +113,10 @@ struct PrefillArgs {
   float* part_ml;
   const float* k_scale;   // FP8 pools: per-kv-head scales (element = e4m3 byte * scale)
   const float* v_scale;
-  int num_seqs, num_kv_heads, group, hgroups, block_size, bs_shift, num_blocks, max_bps;
-  int tiles_max, subtiles, splits_max;   // subtiles: 32-row subtiles per sequence
-  int ks_steps, num_groups;              // key steps per split; (split, seq, kv-head) groups
+  int num_seqs, num_kv_heads, group, block_size, bs_shift, num_blocks, max_bps;
+  int tiles_max, subtiles, splits_max;   // subtiles: 32-row subtiles per (sequence, kv head)
+  int ks_steps;                          // key steps per split (fixed order)
+  int max_items;                         // items per kv head the grid has room for
   int num_cus;                           // compute units of the device (work-list sizing)
   float scale_log2;
   int64_t q_stride_token, q_stride_head, out_stride_token, out_stride_head;
@@ -118,6 +131,10 @@ struct Mfma<npd::BF16> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(V8, a),
                                                    __builtin_bit_cast(V8, b), c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(V8, a),
+                                                 __builtin_bit_cast(V8, b), c, 0, 0, 0);
+  }
 };
 template <>
 struct Mfma<npd::F16> {
@@ -126,7 +143,49 @@ struct Mfma<npd::F16> {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(V8, a),
                                                   __builtin_bit_cast(V8, b), c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x16 mma32(u32x4 a, u32x4 b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(V8, a),
+                                                 __builtin_bit_cast(V8, b), c, 0, 0, 0);
+  }
 };
+
+// When a row's reference moves. bf16: the reference sits kBias above the
+// maximum it was taken from, P is <= 2^-7 then, and a P of 2 or more (bit 14 of
+// any packed half; also inf and NaN) asks for a new one: one v_or3 per two
+// pairs. fp16 keeps its reference at the maximum (a bias would cost small P
+// their bits) and asks at P >= 2^8, by packed integer maxima. Either way a
+// reference moves when a score passed it by 2^8 and P stays exact enough: fp32
+// sums, relative rounding of the pair.
+template <class TT>
+struct Bound;
+template <>
+struct Bound<npd::BF16> {
+  static constexpr float kBias = 7.f, kMove = 0.f;
+};
+template <>
+struct Bound<npd::F16> {
+  static constexpr float kBias = 0.f, kMove = 7.f;
+};
+template <class TT, int KB>
+__device__ __forceinline__ bool past_bound(const u32x4 (&pb)[KB]) {
+  if constexpr (std::is_same<TT, npd::BF16>::value) {
+    uint32_t o = 0;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      o = o | pb[kb][0] | pb[kb][1];
+      o = o | pb[kb][2] | pb[kb][3];
+    }
+    return (o & 0x40004000u) != 0;
+  } else {
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+    us2 m = __builtin_bit_cast(us2, pb[0][0]);   // P >= 0: ordered as integers
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pb[kb][i]));
+    return m.x >= 0x5c00u || m.y >= 0x5c00u;   // 2^8
+  }
+}
 
 // Max / sum over the 4 key groups of a query row (lanes l, l^16, l^32, l^48).
 using npd::row_max4;
@@ -139,68 +198,129 @@ __device__ __forceinline__ u32x2 lds_read_tr(const uint16_t* p) {
   return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p)));
 }
 
-// The work item of this workgroup (every wave derives the same one): the
-// sequence s, its query tile t of TR rows, key split j of split length ks
-// steps, kv head kh and head group hg, and the sequence's first query row,
-// chunk length and context. eq: the tile's nsp = ceil(steps / ks) splits are
-// near-equal parts (the first steps % nsp one step longer) instead of ks-step
-// splits and a shorter last one. false: no item, the workgroup exits.
+// x / d for 0 <= x < 2^31, d > 0 and quotients below 2^21: the fp32 estimate
+// is off by at most one. A handful of instructions against some 35 of the
+// integer division.
+__device__ __forceinline__ int small_div(int x, int d) {
+  int q = (int)((float)x * __builtin_amdgcn_rcpf((float)d));
+  const int r = x - q * d;
+  return q + (r >= d ? 1 : 0) - (r < 0 ? 1 : 0);
+}
+
+// The work item of this workgroup, derived by its first wave: the sequence s,
+// its tile t of kTileRows flattened (token, head) rows, key part j of nsp, kv
+// head kh, the sequence's first query row, chunk length and context, the
+// tile's keys 0 .. nkeys - 1 and the part's steps st0 .. st1 - 1. false: no
+// item, the workgroup exits.
 struct Item {
-  int s, t, j, kh, hg, ks, q0, qlen, ctx;
-  bool eq;
+  int s, t, j, nsp, kh, q0, qlen, ctx, nkeys, st0, st1;
 };
-template <int TR>
+// one past the last position that tile t of a chunk sees
+__device__ __forceinline__ int tile_keys(const PrefillArgs& a, int t, int qlen, int ctx) {
+  const int fr = qlen * a.group, fe = (t + 1) * kTileRows;
+  const int last = fe >= fr ? qlen - 1   // position in the chunk of the tile's last row
+                            : (fe < kSmallDiv ? small_div(fe - 1, a.group) : (fe - 1) / a.group);
+  const int nk = ctx - qlen + last + 1;
+  return nk < 0 ? 0 : nk;
+}
 __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Item& it) {
-  int s, t, j, kh, hg, ks = a.ks_steps;
-  int q0, qlen, ctx;
+  int s, t, j, kh, nsp, nsteps, q0, qlen, ctx;
   const int cap = a.max_bps * a.block_size;
-  if (a.num_seqs * a.tiles_max <= 64) {
-    // Work list in longest-processing-time order, derived by every wave from
-    // the sequence lengths. Lane i stands for (sequence i / tiles_max, tile
-    // i % tiles_max) with n_i key steps. The split length ks is chosen so that
-    // the longest key range falls into equal parts no shorter than the
-    // average work per compute unit (and no shorter than the host's split,
-    // which sized the workspace); each tile's splits are near-equal parts. The
+  const int per_item = a.num_kv_heads;   // workgroups per (sequence, tile, part)
+  const int tiles = a.num_seqs * a.tiles_max;
+  if (tiles <= kListTiles) {
+    // Work list in longest-processing-time order, derived from the sequence
+    // lengths. Slot (k, lane) stands for tile index i = 64 k +
+    // lane: sequence i / tiles_max, tile i % tiles_max, n key steps. The
     // kv-head is the fastest-varying index and every count is a multiple of
     // the kv-head count, so with 8 kv-heads each XCD (workgroups go to XCDs
     // round-robin by blockIdx) serves one kv-head and its K/V stays in that
     // XCD's L2.
-    const int ls = lane / a.tiles_max, lt = lane - ls * a.tiles_max;
-    bool valid = ls < a.num_seqs;
-    int n = 0, c0 = 0, ql = 0, cx = 0;
-    if (valid) {
-      c0 = a.cu_seqlens_q[ls];
-      ql = a.cu_seqlens_q[ls + 1] - c0;
-      valid = lt * TR < ql;
-      if (valid) {
-        cx = a.context_lens[ls];
-        cx = cx < 0 ? 0 : (cx < cap ? cx : cap);
-        const int rw = (ql - lt * TR) < TR ? (ql - lt * TR) : TR;
-        int nk = cx - ql + lt * TR + rw;
-        nk = nk < 0 ? 0 : nk;
-        n = (nk + kKT - 1) / kKT;
+    int n[kSlots], c0[kSlots], ql[kSlots], cx[kSlots];
+    bool valid[kSlots];
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+      valid[k] = 64 * k + lane < tiles;
+      n[k] = c0[k] = ql[k] = cx[k] = 0;
+      if (64 * k < tiles && valid[k]) {
+        const int ls = small_div(64 * k + lane, a.tiles_max);
+        c0[k] = a.cu_seqlens_q[ls];
+        ql[k] = a.cu_seqlens_q[ls + 1];
+        cx[k] = a.context_lens[ls];
       }
     }
-    const int per_item = a.num_kv_heads * a.hgroups;   // workgroups per (sequence, tile, split)
-    const int tot = npd::wave_sum_i(n), nmax = npd::wave_max_i(n);   // DPP, wave-uniform
-    const int avg = (int)(((int64_t)tot * per_item + a.num_cus - 1) / a.num_cus);
-    int parts = avg > 0 ? nmax / avg : 1;
-    parts = parts < 1 ? 1 : parts;
-    const int ksd = __builtin_amdgcn_readfirstlane((nmax + parts - 1) / parts);
-    ks = ksd > ks ? ksd : ks;
-    // a tile of n steps runs as nsp = ceil(n / ks) near-equal parts: no short
-    // tail part that would pay a whole item's prologue and merge for a few
-    // steps. Items in longest-processing-time order: by part length (bucket
-    // len = ceil(n / nsp)), longest first; within a bucket by tile, part and
-    // then (kv-head, head group).
-    int nsp = (n + ks - 1) / ks;
-    nsp = nsp < 1 ? 1 : (nsp > a.splits_max ? a.splits_max : nsp);
-    if (!valid) nsp = 0;
-    const int len = valid ? (n + nsp - 1) / nsp : -1;
-    const int lenmax = npd::wave_max_i(len);
+    int tot = 0, nmax = 0, ntiles = 0;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k)
+      if (64 * k < tiles) {
+        const int lt = 64 * k + lane - small_div(64 * k + lane, a.tiles_max) * a.tiles_max;
+        ql[k] -= c0[k];
+        cx[k] = cx[k] < 0 ? 0 : (cx[k] < cap ? cx[k] : cap);
+        valid[k] = valid[k] && lt * kTileRows < ql[k] * a.group;
+        if (valid[k]) n[k] = (tile_keys(a, lt, ql[k], cx[k]) + kKT - 1) / kKT;
+        tot += npd::wave_sum_i(n[k]);   // DPP, wave-uniform
+        nmax = max(nmax, npd::wave_max_i(n[k]));
+        ntiles += __popcll(__ballot(valid[k]));
+      }
+    // Parts per tile: a tile of n steps runs as nsp = ceil(n / ks) near-equal
+    // parts (a short tail part would pay a whole item's prologue and merge for
+    // a few steps), ks = nmax / p for the p whose estimated time is least: the
+    // longest item where one round of the compute units takes them all, else
+    // their mean load plus a share of the longest item (what a greedy
+    // longest-first order leaves uneven; less with every further round). An
+    // item costs kItemSteps steps on top of its own, one that publishes and
+    // merges kMergeSteps more. Over 500 random batches of 1-6 chunks this ends
+    // within 0.2% of the best p's greedy schedule on average. Three rounds of
+    // whole tiles are not cut.
+    auto nsp_of = [&](int k, int step) {
+      const int p = small_div(n[k] + step - 1, step);
+      return !valid[k] ? 0 : (p < 1 ? 1 : (p > a.splits_max ? a.splits_max : p));
+    };
+    int ks = nmax < 1 ? 1 : nmax;
+    const int units = a.num_cus < per_item ? 1 : small_div(a.num_cus, per_item);
+    if (a.splits_max > 1 && ntiles < 3 * units) {
+      float best = 0.f;
+      for (int p = 1; p <= a.splits_max; ++p) {
+        const int kp = small_div(nmax + p - 1, p);
+        if (p > 1 && kp < kMinPart) break;
+        int sums = 0;   // parts, and parts of cut tiles (16 bits each: at most 8 * 512)
+#pragma unroll
+        for (int k = 0; k < kSlots; ++k)
+          if (64 * k < tiles) {
+            const int c = nsp_of(k, kp < 1 ? 1 : kp);
+            sums += npd::wave_sum_i(c + (c > 1 ? c << 16 : 0));
+          }
+        const int items = sums & 0xffff, cut = sums >> 16;
+        if (p > 1 && items > a.max_items) break;
+        const float longest = (float)(kp + kItemSteps + (p > 1 ? kMergeSteps : 0));
+        const float mean = (float)(tot + items * kItemSteps + cut * kMergeSteps) / units;
+        const float est = items <= units ? longest
+                                         : fmaxf(longest, mean + 0.35f * longest * (3 * units - items) / (2 * units));
+        if (p == 1 || est < 0.97f * best) best = est, ks = kp < 1 ? 1 : kp;
+      }
+    }
+    // Items by part length (bucket len = ceil(n / nsp)), longest first; within
+    // a bucket by tile, part and then kv-head.
+    int cut[kSlots], len[kSlots], lenmax = 0;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k) {
+      cut[k] = 0;
+      len[k] = -1;
+      if (64 * k < tiles) {
+        cut[k] = nsp_of(k, ks);
+        if (valid[k]) len[k] = small_div(n[k] + cut[k] - 1, cut[k]);
+        lenmax = max(lenmax, npd::wave_max_i(len[k]));
+      }
+    }
     // items in buckets >= b, non-increasing in b; item id is in the last
     // bucket b with from(b) > id (binary search over DPP wave sums)
-    auto from = [&](int b) -> int { return npd::wave_sum_i(len >= b ? nsp : 0) * per_item; };
+    auto from = [&](int b) -> int {
+      int c = 0;
+#pragma unroll
+      for (int k = 0; k < kSlots; ++k)
+        if (64 * k < tiles) c += npd::wave_sum_i(len[k] >= b ? cut[k] : 0);
+      return c * per_item;
+    };
     int id = blockIdx.x;
     if (id >= from(0)) return false;   // past the last item
     int lo = 0, hi = lenmax;
@@ -209,476 +329,543 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
       if (from(mid) > id) lo = mid; else hi = mid - 1;
     }
     id -= from(lo + 1);
-    // the tile of the bucket holding item id: walk the bucket's tiles (a
-    // wave-uniform loop over at most 64 lanes)
-    uint64_t m = __ballot(len == lo);
-    int sel = __builtin_ctzll(m);
-    for (;;) {
-      const int c = __builtin_amdgcn_readlane(nsp, sel) * per_item;
-      if (id < c || (m & (m - 1)) == 0) break;
-      id -= c;
-      m &= m - 1;
-      sel = __builtin_ctzll(m);
-    }
-    j = id / per_item;
-    id -= j * per_item;
-    const int rem = id;
-    kh = rem % a.num_kv_heads;
-    hg = rem / a.num_kv_heads;
-    s = __builtin_amdgcn_readfirstlane(sel / a.tiles_max);
-    t = __builtin_amdgcn_readfirstlane(sel - s * a.tiles_max);
-    j = __builtin_amdgcn_readfirstlane(j);
-    q0 = __builtin_amdgcn_readlane(c0, sel);
-    qlen = __builtin_amdgcn_readlane(ql, sel);
-    ctx = __builtin_amdgcn_readlane(cx, sel);
+    // the bucket's tile holding item id: the slot row by its sum, then the
+    // lane by an inclusive scan over the row
+    bool found = false;
+    s = t = j = kh = nsp = nsteps = q0 = qlen = ctx = 0;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k)
+      if (64 * k < tiles && !found) {
+        const int c = len[k] == lo ? cut[k] : 0;
+        const int sum = npd::wave_scan_i(c);
+        const int all = __builtin_amdgcn_readlane(sum, 63) * per_item;
+        if (id < all) {
+          const int sel = __builtin_ctzll(__ballot(sum * per_item > id));
+          nsp = __builtin_amdgcn_readlane(c, sel);
+          id -= (__builtin_amdgcn_readlane(sum, sel) - nsp) * per_item;
+          s = small_div(64 * k + sel, a.tiles_max);
+          t = 64 * k + sel - s * a.tiles_max;
+          nsteps = __builtin_amdgcn_readlane(n[k], sel);
+          q0 = __builtin_amdgcn_readlane(c0[k], sel);
+          qlen = __builtin_amdgcn_readlane(ql[k], sel);
+          ctx = __builtin_amdgcn_readlane(cx[k], sel);
+          found = true;
+        } else {
+          id -= all;
+        }
+      }
+    if (!found) return false;   // never: id is below from(lo)
+    j = small_div(id, per_item);
+    kh = id - j * per_item;
   } else {
-    // Unit = (split j, sequence, kv-head; tile t, head group). The units of
-    // one (j, s, kv-head) read the same K/V key range: they form a group that
-    // runs on one XCD at the same time (workgroups go to XCDs round-robin by
-    // blockIdx, so the group's blockIdx values are 8 apart and consecutive in
-    // that XCD's order), so K/V tiles come from that XCD's L2 after the first
-    // read. Within a group the last tile (the most keys) comes first.
-    const int gunits = a.tiles_max * a.hgroups;
-    const int xcd = blockIdx.x & 7, p = blockIdx.x >> 3;
-    const int gi = (p / gunits) * 8 + xcd;
-    if (gi >= a.num_groups) return false;
-    const int u = p - (p / gunits) * gunits;
-    t = a.tiles_max - 1 - u / a.hgroups;
-    hg = u - (u / a.hgroups) * a.hgroups;
-    kh = gi % a.num_kv_heads;
-    const int js = gi / a.num_kv_heads;
-    s = js % a.num_seqs;
-    j = js / a.num_seqs;
+    // Fixed order: key part, sequence, tile (the last, with the most keys,
+    // first), kv head. The kv head varies fastest, as above, so the tiles of a
+    // sequence that run together on an XCD read the same K/V.
+    const int id = blockIdx.x;
+    int u = id / per_item;
+    kh = id - u * per_item;
+    const int v = u / a.tiles_max;
+    t = a.tiles_max - 1 - (u - v * a.tiles_max);
+    j = v / a.num_seqs;
+    s = v - j * a.num_seqs;
     q0 = a.cu_seqlens_q[s];
     qlen = a.cu_seqlens_q[s + 1] - q0;
-    if (t * TR >= qlen) return false;
+    if (t * kTileRows >= qlen * a.group) return false;
     ctx = a.context_lens[s];
     ctx = ctx < 0 ? 0 : (ctx < cap ? ctx : cap);
+    nsteps = (tile_keys(a, t, qlen, ctx) + kKT - 1) / kKT;
+    nsp = (nsteps + a.ks_steps - 1) / a.ks_steps;
+    nsp = nsp < 1 ? 1 : (nsp > a.splits_max ? a.splits_max : nsp);
+    if (j >= nsp) return false;
   }
-
-  it = Item{s, t, j, kh, hg, ks, q0, qlen, ctx, a.num_seqs * a.tiles_max <= 64};
+  // near-equal parts, the first nsteps % nsp one step longer
+  const int base = small_div(nsteps, nsp), rem = nsteps - base * nsp;
+  const int st0 = j * base + (j < rem ? j : rem);
+  it = Item{s, t, j, nsp, kh, q0, qlen, ctx, tile_keys(a, t, qlen, ctx), st0,
+            st0 + base + (j < rem ? 1 : 0)};
   return true;
 }
 
+// LDS position of 16-byte chunk `chunk` of tile row `row` is chunk ^ swz(row):
+// rows are D * 2 bytes apart with no padding (the direct-to-LDS loads write
+// 1 KB runs), and the swizzle spreads both reads of a tile over all banks --
+// 32 rows at one chunk (K), 4 rows x 4 chunks (transposing V reads). Bits of a
+// row index above the fourth do not enter, so rows 16 apart share offsets.
+template <int D>
+__device__ __forceinline__ int swz(int row) {
+  if (D == 64)   // two rows per 256 bytes
+    return (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
+  return ((row & 3) << 2) | (((row >> 2) & 1) << 1) | ((row >> 3) & 1);
+}
+// chunk offset bits (bytes) that differ between rows r and r + 8
+template <int D>
+constexpr int swz8() { return D == 64 ? 32 : 16; }
+
+// 64 lanes x 16 bytes from base + off (per lane) straight into LDS at
+// lds .. lds + 1023, lane i at lds + 16 i. Counts in vmcnt; the caller waits.
+__device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t off, const void* base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :: "s"(lds), "v"(off), "s"(base) : "memory");
+}
+__device__ __forceinline__ void load_to_lds(uint32_t lds, const void* p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(lds), "v"(p) : "memory");
+}
+// All but the last L LDS accesses of this wave are done and at most N of its
+// direct-to-LDS loads are still in flight; then the workgroup's barrier.
+template <int N, int L = 0>
+__device__ __forceinline__ void wait_and_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(%1)\n\ts_barrier" :: "n"(N), "n"(L) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // kOff32: every K/V element of the pool lies within 4 GiB of the cache base,
-// so gather offsets are 32-bit. kF8: the pool holds OCP e4m3 bytes; a K/V
-// chunk is 8 bytes, converted exactly to four TT pairs when copied into LDS,
-// and the per-kv-head scales go into the score scale and the output.
-template <class TT, int D, int HW, bool kOff32, bool kF8>
+// so gather offsets are 32-bit. kF8: the pool holds OCP e4m3 bytes, converted
+// exactly to TT pairs on the way into LDS (through registers); the per-kv-head
+// scales go into the score scale and the output.
+template <class TT, int D, bool kOff32, bool kF8>
 __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   static_assert(D == 64 || D == 128, "head dims of this kernel");
-  constexpr int RT = kPairs / HW;                      // row tiles of 64 per workgroup
-  constexpr int TR = 64 * RT;                          // query rows per workgroup
-  constexpr int MB = kWaveRows / 16;                   // 16-row query blocks per wave
-  constexpr int NC = D / 32;                           // head-dim chunks of QK
-  constexpr int NB = D / 16;                           // 16-dim blocks of O
-  constexpr int kRow = lds_row(D);
+  constexpr int RB = 2 * D;                            // bytes of a tile row
+  constexpr int TB = kKT * RB;                         // bytes of a K or V tile
+  constexpr int NI = TB / (1024 * kWaves);             // 1 KB loads per wave and tile (D 128: 2)
+  constexpr int NC = D / 16;                           // head-dim chunks of QK
+  constexpr int NS = kKT / 32;                         // 32-key blocks of S
+  constexpr int KB = kKT / 16;                         // 16-key blocks of PV
+  constexpr int DB = D / 32;                           // 32-dim blocks of O
   constexpr int kRecO = rec_o(D);
-  __shared__ __attribute__((aligned(16))) uint16_t s_k[2][kKT * kRow];
-  __shared__ __attribute__((aligned(16))) uint16_t s_v[3][kKT * kRow];
-  __shared__ int s_blk[kMaxBlocksLds];
+  static_assert(NI * 1024 * kWaves == TB, "tile shape");
+  __shared__ __attribute__((aligned(1024))) char s_k[kBufK * TB];
+  __shared__ __attribute__((aligned(1024))) char s_v[kBufV * TB];
+  __shared__ int s_row[kListBlocks];   // first K/V row of each block of the key range
   __shared__ int s_ticket;
+  __shared__ Item s_item;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int g = lane >> 4, r = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int hf = lane >> 5, c32 = lane & 31;
 
-  Item it;
-  if (!prefill_item<TR>(a, lane, it)) return;
-  const int s = it.s, t = it.t, j = it.j, kh = it.kh, hg = it.hg, ks = it.ks;
-  const int q0 = it.q0, qlen = it.qlen, ctx = it.ctx;
-
-  const int prefix = ctx - qlen;                       // position of query row 0
-  const int rows = (qlen - t * TR) < TR ? (qlen - t * TR) : TR;
-  const int pos0 = prefix + t * TR;                    // position of the tile's first row
-  int nkeys = pos0 + rows;                             // keys 0 .. last row's position
-  nkeys = nkeys < 0 ? 0 : nkeys;
-  const int nsteps = (nkeys + kKT - 1) / kKT;
-  // grid order: split j covers steps [j*ks, (j+1)*ks) -- the same keys for
-  // every tile of the sequence -- the last split runs to the end of the
-  // tile's range; work list: near-equal parts
-  int nsp = (nsteps + ks - 1) / ks;
-  nsp = nsp < 1 ? 1 : (nsp > a.splits_max ? a.splits_max : nsp);
-  if (j >= nsp) return;
-  int st0, st1;
-  if (it.eq) {   // near-equal parts, the first nsteps % nsp one step longer
-    const int base = nsteps / nsp, rem = nsteps - base * nsp;
-    st0 = j * base + (j < rem ? j : rem);
-    st1 = st0 + base + (j < rem ? 1 : 0);
-  } else {
-    st0 = j * ks;
-    st1 = j == nsp - 1 ? nsteps : st0 + ks;
+  // The first wave derives the item: eight waves sharing the SIMDs for the same
+  // answer took 5.1 us where this takes 4.4 (32 tiles, four part counts tried).
+  if (wave == 0) {
+    Item it{};
+    it.nsp = 0;
+    prefill_item(a, lane, it);
+    if (lane == 0) s_item = it;
   }
+  __syncthreads();
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  const int nsp = uni(s_item.nsp);
+  if (nsp == 0) return;   // no item
+  const int s = uni(s_item.s), t = uni(s_item.t), j = uni(s_item.j), kh = uni(s_item.kh);
+  const int q0 = uni(s_item.q0), qlen = uni(s_item.qlen), ctx = uni(s_item.ctx), G = a.group;
+  const int nkeys = uni(s_item.nkeys), st0 = uni(s_item.st0), st1 = uni(s_item.st1);
 
-  // wave -> (head of the group, row tile, half of the row tile)
-  const int pair = wave >> 1, half = wave & 1;
-  const int wr = pair / HW;
-  const int h = kh * a.group + hg * HW + (pair - wr * HW);
-  const int wsub = (t * RT + wr) * 2 + half;           // 32-row subtile index in the sequence
-  const int wrow0 = wsub * kWaveRows;                  // this wave's first row
-  const int wpos0 = prefix + wrow0;
+  // flattened rows f = token * G + head: the tile's 256, this wave's 32 and
+  // this lane's one (clamped to the chunk's last; outputs past it are not stored)
+  const int prefix = ctx - qlen;                       // position of the chunk's first token
+  const int frows = qlen * G;
+  const int wsub = t * kWaves + wave;                  // 32-row subtile of the (sequence, kv head)
+  const int f0 = wsub * kWaveRows;
+  const bool row_ok = f0 + c32 < frows;
+  const int f = row_ok ? f0 + c32 : frows - 1;
+  const int tok = frows < kSmallDiv ? small_div(f, G) : f / G;
+  const int h = kh * G + (f - tok * G);
+  const int pos = prefix + tok;                        // this lane's query position
+  const int wpos0 = __builtin_amdgcn_readfirstlane(pos);
+  const int wpos1 = __builtin_amdgcn_readlane(pos, 31);   // the wave's first and last position
   const int bs = a.block_size;
-  const int kbeg = st0 * kKT;
   const int kend = st1 * kKT < nkeys ? st1 * kKT : nkeys;
-  const int blk0 = kbeg / bs;
-  const int nblk = kend > kbeg ? (kend + bs - 1) / bs - blk0 : 0;
 
+  uint16_t* op = a.out + (int64_t)(q0 + tok) * a.out_stride_token + (int64_t)h * a.out_stride_head;
   if (st0 >= st1) {
     // no key at all (every row of the tile sits before position 0): zero rows
+    if (row_ok)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const int row = wrow0 + mb * 16 + r;
-      if (row >= qlen) continue;
-      uint16_t* op = a.out + (int64_t)(q0 + row) * a.out_stride_token + (int64_t)h * a.out_stride_head;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) *reinterpret_cast<u32x2*>(op + nb * 16 + g * 4) = u32x2{0, 0};
-    }
+      for (int e = 0; e < D / 8; ++e) *reinterpret_cast<u32x2*>(op + e * 8 + hf * 4) = u32x2{0, 0};
     return;
   }
 
-  // block ids of the split's key range -> LDS (clamped into the pool); the
-  // host guarantees max_bps <= kMaxBlocksLds, so the whole range fits
-  for (int e = tid; e < nblk; e += kThreads) {
-    int bid = a.block_tables[(int64_t)s * a.max_bps + blk0 + e];
-    s_blk[e] = bid < 0 ? 0 : (bid >= a.num_blocks ? a.num_blocks - 1 : bid);
+  // the lane's query row as B operands: qb[c] = Q[row][c*16 + 8 hf .. +8]
+  u32x4 qb[NC];
+  {
+    const uint16_t* qp = a.q + (int64_t)(q0 + tok) * a.q_stride_token +
+                         (int64_t)h * a.q_stride_head + hf * 8;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) qb[c] = *reinterpret_cast<const u32x4*>(qp + c * 16);
   }
 
-  // the wave's query rows as B operands: qb[mb][c] = Q[row mb*16 + r][c*32 + 8g .. +8].
-  // Rows past the chunk read its last row (their outputs are never stored):
-  // unconditional loads keep the compiler's count of loads in flight exact.
-  u32x4 qb[MB][NC];
+  // Tile loads. 2-byte pools: 1 KB run e of this wave's NI covers tile bytes
+  // (wave * NI + e) * 1024 ..; lane i's 16 bytes are the chunk that the swizzle
+  // puts at byte 16 i of the run. FP8 pools: through registers, NF loads of
+  // F8B bytes (F8B / 8 chunks) per thread. Keys past the split's range are
+  // clamped to its last key: a real, finite context row that the causal mask
+  // removes (only keys past the tile's last position are clamped).
+  constexpr int F8B = D == 64 ? 8 : 16;
+  constexpr int LROW = kF8 ? D / F8B : RB / 16;        // lanes per row
+  constexpr int NR = kF8 ? kKT * D / (kThreads * F8B) : NI;
+  static_assert(!kF8 || NR * kThreads * F8B == kKT * D, "FP8 tile shape");
+  int lrow[NR], lcol[NR];   // tile row and source column (bytes) of this lane's loads
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    int row = wrow0 + mb * 16 + r;
-    row = row < qlen ? row : qlen - 1;
-    const uint16_t* qp = a.q + (int64_t)(q0 + row) * a.q_stride_token +
-                         (int64_t)h * a.q_stride_head + g * 8;
-#pragma unroll
-    for (int c = 0; c < NC; ++c) qb[mb][c] = *reinterpret_cast<const u32x4*>(qp + c * 32);
+  for (int e = 0; e < NR; ++e) {
+    if (kF8) {
+      lrow[e] = (tid + kThreads * e) / LROW;
+      lcol[e] = (tid + kThreads * e) % LROW * F8B;
+    } else {
+      const int o = (wave * NI + e) * 1024 + lane * 16;
+      lrow[e] = o / RB;
+      lcol[e] = ((o % RB / 16) ^ swz<D>(lrow[e])) * 16;
+    }
   }
-  __syncthreads();
-
-  // K/V tile loaders: chunk tid + 512e (8 elements) of the 64-key tile, i.e.
-  // key tid / CPR + KPP * e, column chunk tid % CPR. Loads run kDepth steps
-  // ahead through a register ring (slot = step % kDepth): one tile in flight
-  // per CU leaves a step waiting on memory latency.
-  constexpr int CPR = D / 8;                           // 8-element chunks per row
-  constexpr int KPP = kThreads / CPR;                  // keys per load pass
-  constexpr int kPer = kKT / KPP;                      // 2 at D 128, 1 at D 64
-  static_assert(kPer * KPP == kKT, "tile shape");
-  typedef typename std::conditional<kF8, u32x2, u32x4>::type raw_t;   // 8 elements
-  raw_t kst[kDepth][kPer], vst[kDepth][kPer];
-  const int col = tid % CPR;
-  // Every fetch issues the same loads, so the compiler's count of loads in
-  // flight stays exact and its waits cover only the slot being used: tokens
-  // past the split's range are clamped to its last key. Such keys only occur
-  // past the tile's last row (the causal mask removes them) and hold real
-  // context rows, so their V is finite and P = 0 cancels it.
-  auto fetch = [&](int step, raw_t* ks, raw_t* vs) {
+  int blk0 = 0;   // first block of the list in s_row
+  // pool row of tile row lrow[e] of step `step` (< 2^31, host check)
+  auto pool_row = [&](int step, int e) {
+    int tk = step * kKT + lrow[e];
+    tk = tk < kend ? tk : kend - 1;
+    const int lb = a.bs_shift >= 0 ? tk >> a.bs_shift : tk / bs;
+    return s_row[lb - blk0] + (tk - (a.bs_shift >= 0 ? lb << a.bs_shift : lb * bs));
+  };
+  const uint32_t lds_k = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)s_k;
+  const uint32_t lds_v = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)s_v;
+  typedef uint32_t raw16 __attribute__((ext_vector_type(F8B / 4), aligned(8)));
+  struct Raw {
+    raw16 k[kF8 ? NR : 1], v[kF8 ? NR : 1];
+  };
+  int rows[NR];   // pool rows of the tile loaded next
+  auto find_rows = [&](int step) {
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      int tok = step * kKT + tid / CPR + KPP * e;
-      tok = tok < kend ? tok : kend - 1;
-      const int lb = a.bs_shift >= 0 ? tok >> a.bs_shift : tok / bs;
-      const int blk = s_blk[lb - blk0];
-      const int row = (blk * a.num_kv_heads + kh) * bs + (tok - lb * bs);   // < 2^31 (host check)
-      if constexpr (kF8) {   // D-byte rows, 8-byte chunks
-        const char* kb = reinterpret_cast<const char*>(a.k_cache);
-        const char* vb = reinterpret_cast<const char*>(a.v_cache);
-        if (kOff32) {
-          const uint32_t off = (uint32_t)row * (uint32_t)D + (uint32_t)col * 8u;
-          ks[e] = *reinterpret_cast<const u32x2*>(kb + off);
-          vs[e] = *reinterpret_cast<const u32x2*>(vb + off);
-        } else {
-          const int64_t off = (int64_t)row * D + col * 8;
-          ks[e] = *reinterpret_cast<const u32x2*>(kb + off);
-          vs[e] = *reinterpret_cast<const u32x2*>(vb + off);
-        }
-      } else if (kOff32) {
-        const uint32_t off = (uint32_t)row * (uint32_t)(2 * D) + (uint32_t)col * 16u;
-        ks[e] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(a.k_cache) + off);
-        vs[e] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(a.v_cache) + off);
+    for (int e = 0; e < NR; ++e) rows[e] = pool_row(step, e);
+  };
+  // 2-byte pools: the tile of `rows` into LDS buffers kb, vb
+  auto load = [&](int kb, int vb) {
+#pragma unroll
+    for (int e = 0; e < NR; ++e) {
+      const uint32_t run = (uint32_t)(wave * NI + e) * 1024u;
+      if (kOff32) {
+        const uint32_t off = (uint32_t)rows[e] * (uint32_t)RB + (uint32_t)lcol[e];
+        load_to_lds(lds_k + kb * TB + run, off, a.k_cache);
+        load_to_lds(lds_v + vb * TB + run, off, a.v_cache);
       } else {
-        const int64_t idx = (int64_t)row * CPR + col;
-        ks[e] = a.k_cache[idx];
-        vs[e] = a.v_cache[idx];
+        const int64_t off = (int64_t)rows[e] * RB + lcol[e];
+        load_to_lds(lds_k + kb * TB + run, reinterpret_cast<const char*>(a.k_cache) + off);
+        load_to_lds(lds_v + vb * TB + run, reinterpret_cast<const char*>(a.v_cache) + off);
       }
     }
   };
-  auto pairs = [](raw_t w) -> u32x4 {
-    if constexpr (kF8)
-      return u32x4{npd::e4m3x2_to<TT, false>(w.x), npd::e4m3x2_to<TT, true>(w.x),
-                   npd::e4m3x2_to<TT, false>(w.y), npd::e4m3x2_to<TT, true>(w.y)};
-    else
-      return w;
-  };
-  auto stash = [&](int kbuf, int vbuf, const raw_t* ks, const raw_t* vs) {
+  // FP8 pools: the tile of `rows` into registers; registers into LDS
+  auto fetch = [&](Raw& r) {
 #pragma unroll
-    for (int e = 0; e < kPer; ++e) {
-      const int kk = tid / CPR + KPP * e;
-      *reinterpret_cast<u32x4*>(&s_k[kbuf][kk * kRow + col * 8]) = pairs(ks[e]);
-      *reinterpret_cast<u32x4*>(&s_v[vbuf][kk * kRow + col * 8]) = pairs(vs[e]);
+    for (int e = 0; e < NR; ++e) {
+      const int64_t off = kOff32 ? (int64_t)((uint32_t)rows[e] * (uint32_t)D + (uint32_t)lcol[e])
+                                 : (int64_t)rows[e] * D + lcol[e];
+      r.k[e] = *reinterpret_cast<const raw16*>(reinterpret_cast<const char*>(a.k_cache) + off);
+      r.v[e] = *reinterpret_cast<const raw16*>(reinterpret_cast<const char*>(a.v_cache) + off);
     }
   };
+  auto stash = [&](const Raw& r, int kb, int vb) {
+#pragma unroll
+    for (int e = 0; e < NR; ++e)
+#pragma unroll
+      for (int x = 0; x < F8B / 8; ++x) {
+        const int at = lrow[e] * RB + (((lcol[e] / 8 + x) ^ swz<D>(lrow[e])) << 4);
+        auto put = [&](char* tile, const raw16& w) {
+          *reinterpret_cast<u32x4*>(tile + at) =
+              u32x4{npd::e4m3x2_to<TT, false>(w[2 * x]), npd::e4m3x2_to<TT, true>(w[2 * x]),
+                    npd::e4m3x2_to<TT, false>(w[2 * x + 1]), npd::e4m3x2_to<TT, true>(w[2 * x + 1])};
+        };
+        put(s_k + kb * TB, r.k[e]);
+        put(s_v + vb * TB, r.v[e]);
+      }
+  };
 
-  f32x4 oacc[NB][MB];   // O^T[d = nb*16 + 4g + i][q = mb*16 + r]
+  f32x16 oacc[DB];   // O^T[d = db*32 + 8*(i/4) + 4 hf + i%4][row c32]
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) oacc[nb][mb] = f32x4{0, 0, 0, 0};
-  float mrow[MB], nmref[MB], lrow[MB];   // running max (log2 units), -max or 0, row sum
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    mrow[mb] = -INFINITY;
-    nmref[mb] = 0.f;
-    lrow[mb] = 0.f;
-  }
+    for (int i = 0; i < 16; ++i) oacc[db][i] = 0.f;
+  // reference of the row's exponents (log2 units; -inf: none yet), what is
+  // added to the scaled scores (-mref; large before the first reference, so
+  // that any visible score asks for one), and the row sum of this lane's keys
+  float mref = -INFINITY, nmref = kNoRef, lsum = 0.f;
   const float c2 = kF8 ? a.scale_log2 * a.k_scale[kh] : a.scale_log2;
   const float oscale = kF8 ? a.v_scale[kh] : 1.f;
 
+  const int kofs = c32 * RB + ((hf ^ swz<D>(c32)) << 4);
+  // K operand x of a step: head-dim chunk x / NS of 32-key block x % NS
+  auto read_k = [&](int kb, int x) {
+    return *reinterpret_cast<const u32x4*>(s_k + ((kb * TB + kofs) ^ (x / NS << 5)) + x % NS * 32 * RB);
+  };
+  auto qk = [&](int kb, const u32x4 (&kpre)[kAhead], f32x16 (&sacc)[NS]) {
 #pragma unroll
-  for (int d = 0; d < kDepth; ++d) fetch(st0 + d, kst[d], vst[d]);
-  stash(0, 0, kst[0], vst[0]);
-  __syncthreads();
-
-  // Step pieces. qk: S^T of step `step` from K buffer kbuf; softmax: P of
-  // that step into pb (moves the running max and rescales O when needed);
-  // pv: O^T += V^T . P^T from V buffer vbuf.
-  f32x4 sacc[4][MB];   // S^T[key = n*16 + 4g + i][q = mb*16 + r]
-  auto qk = [&](int kbuf) {
-    const uint16_t* kt = s_k[kbuf];
-    // S^T = K . Q^T
+    for (int n = 0; n < NS; ++n)
 #pragma unroll
-    for (int n = 0; n < 4; ++n)
+      for (int i = 0; i < 16; ++i) sacc[n][i] = 0.f;
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) sacc[n][mb] = f32x4{0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        const u32x4 ka = *reinterpret_cast<const u32x4*>(&kt[(n * 16 + r) * kRow + c * 32 + g * 8]);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) sacc[n][mb] = Mfma<TT>::mma(ka, qb[mb][c], sacc[n][mb]);
-      }
+    for (int x = 0; x < NS * NC; ++x) {
+      const u32x4 ka = x < kAhead ? kpre[x] : read_k(kb, x);
+      sacc[x % NS] = Mfma<TT>::mma32(ka, qb[x / NS], sacc[x % NS]);
     }
   };
-  auto softmax = [&](int step, u32x4 (&pb)[2][MB]) {
+  auto softmax = [&](int step, f32x16 (&sacc)[NS], u32x4 (&pb)[KB]) {
     const int key0 = step * kKT;
-    // causal mask, lazy-max softmax
-    const bool diag = key0 + kKT - 1 > wpos0;   // some key here is after some row
-    float v[MB][16];
-    float mxs[MB];
-    bool need = false;
+    if (__builtin_expect(key0 + kKT - 1 > wpos0, 0)) {   // some key here is after some row
+      const int lim = pos - key0 - 4 * hf;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
+      for (int n = 0; n < NS; ++n)
 #pragma unroll
-      for (int n = 0; n < 4; ++n)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[mb][n * 4 + i] = sacc[n][mb][i];
+        for (int i = 0; i < 16; ++i)
+          if (n * 32 + 8 * (i >> 2) + (i & 3) > lim) sacc[n][i] = -INFINITY;
     }
-    if (diag) {
+    // P = 2^(s*c - m), packed: pb[kb] is the B operand of keys kb*16 .. +16 in
+    // slots e < 4 -> key 4 hf + e, e >= 4 -> 8 + 4 hf + e - 4
+    auto expo = [&]() {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        // key n*16 + 4g + i of this step is visible to the row iff n*16 + i <= lim
-        const int lim = wpos0 + mb * 16 + r - key0 - 4 * g;
+      for (int n = 0; n < NS; ++n)
 #pragma unroll
-        for (int n = 0; n < 4; ++n)
+        for (int i = 0; i < 16; i += 2)
+          pb[n * 2 + (i >> 3)][(i & 7) >> 1] =
+              TT::pack2(__builtin_amdgcn_exp2f(fmaf(sacc[n][i], c2, nmref)),
+                        __builtin_amdgcn_exp2f(fmaf(sacc[n][i + 1], c2, nmref)));
+    };
+    expo();
+    // The reference moves only when an exponential grew past a bound, read off
+    // the packed values: the maximum is taken in that rare case only.
+    if (__builtin_expect(__ballot(past_bound<TT, KB>(pb)) != 0, 0)) {
+      float mx = fmaxf(fmaxf(sacc[0][0], sacc[0][1]), sacc[0][2]);
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (n * 16 + i > lim) v[mb][n * 4 + i] = -INFINITY;
-      }
+      for (int e = 3; e + 1 < 16 * NS; e += 2)
+        mx = fmaxf(fmaxf(mx, sacc[e >> 4][e & 15]), sacc[(e + 1) >> 4][(e + 1) & 15]);
+      mx = npd::half_max(fmaxf(mx, sacc[NS - 1][15])) * c2;
+      const bool nd = mx > mref + Bound<TT>::kMove;
+      const float mnew = nd ? mx + Bound<TT>::kBias : mref;
+      const float alpha = nd ? __builtin_amdgcn_exp2f(mref - mnew) : 1.f;   // 0 from -inf
+#pragma unroll
+      for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+      lsum *= alpha;
+      mref = mnew;
+      nmref = mnew == -INFINITY ? kNoRef : -mnew;
+      expo();
     }
+    float ps[4] = {lsum, 0.f, 0.f, 0.f};   // four short chains
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      // a chain of three-operand maxima (v_max3_f32: two values per instruction)
-      float mx = fmaxf(fmaxf(v[mb][0], v[mb][1]), v[mb][2]);
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int e = 3; e < 15; e += 2) mx = fmaxf(fmaxf(mx, v[mb][e]), v[mb][e + 1]);
-      mx = row_max4(fmaxf(mx, v[mb][15]));
-      mxs[mb] = mx * c2;
-      need = need || (mxs[mb] > mrow[mb] + kTau);
-    }
-    if (__ballot(need) != 0) {
-      // a row whose max moved past the threshold takes the new max as its
-      // reference; alpha = 0 from the initial -inf (O and l are still 0)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        const bool nd = mxs[mb] > mrow[mb] + kTau;
-        const float mnew = nd ? mxs[mb] : mrow[mb];
-        const float alpha = nd ? __builtin_amdgcn_exp2f(mrow[mb] - mnew) : 1.f;
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) oacc[nb][mb] *= alpha;
-        lrow[mb] *= alpha;
-        mrow[mb] = mnew;
-        nmref[mb] = mnew == -INFINITY ? 0.f : -mnew;
-      }
-    }
-    // P = 2^(s*c - m), packed; pb[kc][mb] is the B operand of keys kc*32 .. +32:
-    // slots e<4 -> key kc*32 + 4g + e, e>=4 -> kc*32 + 16 + 4g + e - 4
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      uint32_t packed[8];
-#pragma unroll
-      for (int e = 0; e < 16; e += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(fmaf(v[mb][e], c2, nmref[mb]));
-        const float p1 = __builtin_amdgcn_exp2f(fmaf(v[mb][e + 1], c2, nmref[mb]));
-        const uint32_t u = TT::pack2(p0, p1);
-        lrow[mb] = TT::dot2(u, TT::kOne2, lrow[mb]);
-        packed[e / 2] = u;
-      }
-      pb[0][mb] = u32x4{packed[0], packed[1], packed[2], packed[3]};
-      pb[1][mb] = u32x4{packed[4], packed[5], packed[6], packed[7]};
-    }
+      for (int i = 0; i < 4; ++i) ps[i] = TT::dot2(pb[kb][i], TT::kOne2, ps[i]);
+    lsum = (ps[0] + ps[1]) + (ps[2] + ps[3]);
   };
-  auto pv = [&](int vbuf, const u32x4 (&pb)[2][MB]) {
-    // O^T += V^T . P^T ; A = V^T[d = nb*16 + r][keys kc*32 + {4g..4g+3, 16+4g..16+4g+3}]
-    // transposing reads: lane r of group g addresses key (.. + 4g + r/4),
-    // dims nb*16 + 4*(r%4) .. +3, and receives dim nb*16 + r of keys +0..3
-    const uint16_t* vlane = s_v[vbuf] + (g * 4 + (r >> 2)) * kRow + 4 * (r & 3);
+  // O^T += V^T . P^T ; A = V^T[d = db*32 + c32][keys as pb's slots]: two
+  // transposing reads, in each of which lane i of a group of 16 addresses key
+  // i/4 (+ 4 hf) and dims 16*(group & 1) + 4*(i%4) .. +3
+  const int vrow = 4 * hf + ((lane & 15) >> 2);
+  const int vofs = vrow * RB + (((((lane >> 4) & 1) * 2 + ((lane & 3) >> 1)) ^ swz<D>(vrow)) << 4) +
+                   (lane & 1) * 8;
+  auto pv = [&](int vb, const u32x4 (&pb)[KB]) {
+    const int vt = vb * TB + vofs;
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-        const u32x2 lo = lds_read_tr(vlane + (kc * 32) * kRow + nb * 16);
-        const u32x2 hi = lds_read_tr(vlane + (kc * 32 + 16) * kRow + nb * 16);
-        const u32x4 va = u32x4{lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) oacc[nb][mb] = Mfma<TT>::mma(va, pb[kc][mb], oacc[nb][mb]);
+      for (int db = 0; db < DB; ++db) {
+        const int at = vt ^ (db << 6);
+        const u32x2 lo = lds_read_tr(reinterpret_cast<const uint16_t*>(s_v + at + kb * 16 * RB));
+        const u32x2 hi = lds_read_tr(
+            reinterpret_cast<const uint16_t*>(s_v + (at ^ swz8<D>()) + (kb * 16 + 8) * RB));
+        oacc[db] = Mfma<TT>::mma32(u32x4{lo.x, lo.y, hi.x, hi.y}, pb[kb], oacc[db]);
       }
-    }
   };
 
-  // Two waves share each SIMD (waves w and w + 4). Group A (waves 0-3) runs
-  // a step as QK -> softmax -> PV; group B (waves 4-7) runs the PV of the
-  // previous step first, then QK -> softmax, so that one wave's softmax (VALU)
-  // runs while the other's MFMAs do. K tiles use two LDS buffers; V tiles
-  // three, because group B still reads step j - 1's V in step j.
-  // Register ring slot SL holds this step's tile (already in LDS); it is
-  // refilled with step + kDepth, and slot SL + 1 (the next step's tile) is
-  // copied into LDS at the end of the step.
+  // Order of the interval's LDS reads and MFMAs (NS * NC QK, then KB * DB PV):
+  // operand reads stay kAhead MFMAs ahead (the first kAhead K operands were
+  // read before the barrier), so that none waits on LDS latency. Left to itself
+  // the compiler keeps one pair of K reads in flight.
+  auto interleave = [&]() {
+    constexpr int kQ = NS * NC, kP = KB * DB;
+#pragma unroll
+    for (int i = 0; i < kQ - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < kP; ++i) {
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 0);
+      __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(kSchedMfma, kAhead, 0);
+  };
+  // Two waves share each SIMD (waves w and w + 4), kept half a step apart: in
+  // every interval between two barriers one of them runs its MFMAs (QK of its
+  // step and PV of the step before), the other its softmax.
+  //   interval       2i                2i + 1
+  //   waves 0-3   QK(i), PV(i-1)     softmax(i)
+  //   waves 4-7   softmax(i-1)       QK(i), PV(i-1)
+  // Each wave starts its share of tile i + 3 before softmax(i), in interval
+  // 2i + 1 at the earliest, into the buffers of K tile i - 1 and V tile i - 2
+  // (4 K, 5 V buffers), last read in interval 2i - 1. Its share of tile i + 2
+  // has landed when its softmax(i) is done (interval 2i + 1 or 2i + 2), so the
+  // whole tile has when a wave reads its first K operands ahead of step i + 2,
+  // at the end of interval 2i + 3 or 2i + 4.
   const bool late = wave >= kWaves / 2;
-  u32x4 pb[2][MB];
-  bool pending = false;   // group B: pb holds the P of a step whose PV is due
-  auto step_body = [&](int step, auto slot) {
-    constexpr int SL = decltype(slot)::value;
-    constexpr int SN = (SL + 1) % kDepth;
-    const int rel = step - st0;
-    fetch(step + kDepth, kst[SL], vst[SL]);   // past st1: clamped, never used
-    // some row of the wave sees a key here (always so with one row tile)
-    const bool active = RT == 1 || step * kKT <= wpos0 + kWaveRows - 1;
-    if (!late) {
-      if (active) {
-        qk(rel & 1);
-        softmax(step, pb);
-        pv(rel % 3, pb);
-      }
-    } else {
-      if (pending) pv((rel + 2) % 3, pb);
-      pending = active;
-      if (active) {
-        qk(rel & 1);
-        softmax(step, pb);
-      }
+  const int list_steps = (int)((int64_t)(kListBlocks - 2) * bs / kKT);   // steps the list covers
+  const int seg = list_steps < 1 ? 1 : list_steps;
+  for (int sb = st0; sb < st1; sb += seg) {
+    const int n = (sb + seg < st1 ? sb + seg : st1) - sb;
+    // first rows of the blocks of this segment's keys (ids clamped into the pool)
+    auto div_bs = [&](int x) { return a.bs_shift >= 0 ? x >> a.bs_shift : x / bs; };
+    blk0 = div_bs(sb * kKT);
+    const int ke = (sb + n) * kKT < kend ? (sb + n) * kKT : kend;
+    const int nblk = div_bs(ke - 1) + 1 - blk0;
+    if (sb != st0) __syncthreads();   // the last segment's reads are done
+    for (int e = tid; e < nblk; e += kThreads) {
+      int bid = a.block_tables[(int64_t)s * a.max_bps + blk0 + e];
+      bid = bid < 0 ? 0 : (bid >= a.num_blocks ? a.num_blocks - 1 : bid);
+      s_row[e] = (bid * a.num_kv_heads + kh) * bs;
     }
-    // K buffer (rel + 1) & 1 and V buffer (rel + 1) % 3 were last read in
-    // step - 1 (group B's PV of step - 2 included), which every wave finished
-    // before that step's barrier. Written even after the last step (nobody
-    // reads it then): an unconditional copy keeps the compiler's load
-    // accounting exact on every path.
-    stash((rel + 1) & 1, (rel + 1) % 3, kst[SN], vst[SN]);
+    // nothing of the compiler's own loads stays in flight: its waits inside
+    // the loop would cover the tile loads too
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
     __syncthreads();
-  };
-  // full rounds of the ring in the loop; the 0-2 remaining steps after it, so
-  // that every path back to the loop head has run all three slots
-  static_assert(kDepth == 3, "the unrolled ring below has three slots");
-  int step = st0;
-  for (; step + kDepth <= st1; step += kDepth) {
-    step_body(step, std::integral_constant<int, 0>{});
-    step_body(step + 1, std::integral_constant<int, 1>{});
-    step_body(step + 2, std::integral_constant<int, 2>{});
-  }
-  if (step < st1) step_body(step, std::integral_constant<int, 0>{});
-  if (step + 1 < st1) step_body(step + 1, std::integral_constant<int, 1>{});
-  if (late && pending) pv((st1 - 1 - st0) % 3, pb);
-
-  // row sums over the 4 lanes of a row
+    // P of the step before the segment: none. Its V tile (the last buffer) is
+    // zeroed too, so that the first interval's PV adds nothing.
+    u32x4 pb[KB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) lrow[mb] = row_sum4(lrow[mb]);
+    for (int e = 0; e < KB; ++e) pb[e] = u32x4{0, 0, 0, 0};
+    for (int e = tid; e < TB / 16; e += kThreads)
+      *reinterpret_cast<u32x4*>(s_v + (kBufV - 1) * TB + e * 16) = u32x4{0, 0, 0, 0};
+    // steps in which some row of this wave sees a key (the causal mask only
+    // ever ends a wave's steps): later ones it spends in the barriers
+    int nact = wpos1 < sb * kKT ? 0 : wpos1 / kKT - sb + 1;
+    nact = nact < n ? nact : n;
+    Raw raw;   // FP8: the bytes of the tile stashed next
+    if constexpr (kF8) {
+      Raw r1, r2;
+      find_rows(sb);
+      fetch(raw);
+      if (n > 1) { find_rows(sb + 1); fetch(r1); }
+      if (n > 2) { find_rows(sb + 2); fetch(r2); }
+      stash(raw, 0, 0);
+      if (n > 1) stash(r1, 1, 1);
+      if (n > 2) stash(r2, 2, 2);
+      if (n > 3) { find_rows(sb + 3); fetch(raw); }
+      wait_and_barrier<63>();
+    } else {
+      find_rows(sb);
+      load(0, 0);
+      if (n > 1) { find_rows(sb + 1); load(1, 1); }
+      if (n > 2) { find_rows(sb + 2); load(2, 2); }
+      if (n > 3) find_rows(sb + 3);
+      if (n > 2) wait_and_barrier<2 * NR>(); else wait_and_barrier<0>();   // tiles 0 and 1
+    }
+    // buffers of the step's tile, of V tile i - 1 and of tile i + 3
+    int kb = 0, vb = 0, vp = kBufV - 1, kb3 = 3, vb3 = 3;
+    // the first K operands of step i + 1, read ahead of its barrier; and tile
+    // i + 2 has landed, i + 3 may be in flight
+    u32x4 kpre[kAhead];
+    auto softmax_done = [&](int i) {
+      if (i + 1 < n)
+#pragma unroll
+        for (int x = 0; x < kAhead; ++x) kpre[x] = read_k(kb, x);
+      if (!kF8 && i + 3 < n) wait_and_barrier<2 * NR, kAhead>();
+      else wait_and_barrier<kF8 ? 63 : 0, kAhead>();
+    };
+    auto next_tile = [&](int i) {   // tile i + 3, and the rows (FP8: the bytes) of tile i + 4
+      if (i + 3 < n) {
+        if constexpr (kF8) stash(raw, kb3, vb3); else load(kb3, vb3);
+        if (i + 4 < n) {
+          find_rows(sb + i + 4);
+          if constexpr (kF8) fetch(raw);
+        }
+      }
+      kb = (kb + 1) & 3;
+      kb3 = (kb3 + 1) & 3;
+      vp = vb;
+      vb = vb == kBufV - 1 ? 0 : vb + 1;
+      vb3 = vb3 == kBufV - 1 ? 0 : vb3 + 1;
+    };
+    static_assert(kBufK == 4 && kBufV == 5, "buffer rotation");
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x) kpre[x] = read_k(kb, x);
+    if (late) wait_and_barrier<63>();
+    int i = 0;
+    for (; i < nact; ++i) {
+      f32x16 sacc[NS];   // S^T[key = n*32 + 8*(i/4) + 4 hf + i%4][row c32]
+      __builtin_amdgcn_s_setprio(1);
+      qk(kb, kpre, sacc);
+      pv(vp, pb);
+      interleave();
+      wait_and_barrier<63>();
+      __builtin_amdgcn_s_setprio(0);
+      next_tile(i);
+      softmax(sb + i, sacc, pb);
+      softmax_done(i);
+    }
+    pv(vp, pb);
+    for (; i < n; ++i) {
+      wait_and_barrier<63>();
+      next_tile(i);
+      softmax_done(i);
+    }
+    if (!late) wait_and_barrier<63>();   // as many barriers as waves 4-7
+  }
+
+  float l = npd::half_sum(lsum);   // the row's keys are in lanes c32 and c32 + 32
 
   if (nsp > 1) {
     // publish this split's partial (register order: every store is 512
     // contiguous bytes), then the last split of the tile to arrive merges
-    const int H = a.num_kv_heads * a.group;
-    const int64_t rec = (((int64_t)s * a.subtiles + wsub) * H + h) * a.splits_max;
+    const int64_t rec = (((int64_t)s * a.num_kv_heads + kh) * a.subtiles + wsub) * a.splits_max;
     {
       float* po = a.part_o + (rec + j) * kRecO + lane * 2;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const int idx = nb * MB + mb;
-          npd::st_coherent2(po + (idx * 2) * 128, oacc[nb][mb][0], oacc[nb][mb][1]);
-          npd::st_coherent2(po + (idx * 2 + 1) * 128, oacc[nb][mb][2], oacc[nb][mb][3]);
-        }
-      float* pm = a.part_ml + (rec + j) * kRecML + lane * 2;
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) npd::st_coherent2(pm + mb * 128, mrow[mb], lrow[mb]);
+        for (int i = 0; i < 8; ++i)
+          npd::st_coherent2(po + (db * 8 + i) * 128, oacc[db][2 * i], oacc[db][2 * i + 1]);
+      npd::st_coherent2(a.part_ml + (rec + j) * kRecML + lane * 2, mref, l);
     }
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);   // every store of this wave has completed
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
-    const int64_t cidx = (((int64_t)s * a.tiles_max + t) * a.num_kv_heads + kh) * a.hgroups + hg;
+    const int64_t cidx = ((int64_t)s * a.tiles_max + t) * a.num_kv_heads + kh;
     if (tid == 0)
       s_ticket = __hip_atomic_fetch_add(a.counters + cidx, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (s_ticket != nsp - 1) return;
     for (int jj = 0; jj < nsp; ++jj) {
       if (jj == j) continue;
-      const float* pm = a.part_ml + (rec + jj) * kRecML + lane * 2;
-      float wa[MB], wb[MB];
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb) {
-        float mp, lp;
-        npd::ld_coherent2(pm + mb * 128, mp, lp);
-        const float mm = fmaxf(mrow[mb], mp);
-        wa[mb] = mrow[mb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mrow[mb] - mm);
-        wb[mb] = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mm);
-        lrow[mb] = lrow[mb] * wa[mb] + lp * wb[mb];
-        mrow[mb] = mm;
-      }
+      float mp, lp;
+      npd::ld_coherent2(a.part_ml + (rec + jj) * kRecML + lane * 2, mp, lp);
+      const float mm = fmaxf(mref, mp);
+      const float wa = mref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mref - mm);
+      const float wb = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mm);
+      l = l * wa + lp * wb;
+      mref = mm;
       const float* po = a.part_o + (rec + jj) * kRecO + lane * 2;
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          const int idx = nb * MB + mb;
-          float x0, x1, x2, x3;
-          npd::ld_coherent2(po + (idx * 2) * 128, x0, x1);
-          npd::ld_coherent2(po + (idx * 2 + 1) * 128, x2, x3);
-          oacc[nb][mb] = oacc[nb][mb] * wa[mb] + f32x4{x0, x1, x2, x3} * wb[mb];
+        for (int i = 0; i < 8; ++i) {
+          float x0, x1;
+          npd::ld_coherent2(po + (db * 8 + i) * 128, x0, x1);
+          oacc[db][2 * i] = oacc[db][2 * i] * wa + x0 * wb;
+          oacc[db][2 * i + 1] = oacc[db][2 * i + 1] * wa + x1 * wb;
         }
     }
     if (tid == 0) __hip_atomic_store(a.counters + cidx, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // normalise and store: lane writes d = nb*16 + 4g .. +3 of query row mb*16 + r
+  // normalise and store: lane writes d = db*32 + 8e + 4 hf .. +3 of its row
+  if (!row_ok) return;
+  const float inv = (l > 0.f && pos >= 0) ? oscale / l : 0.f;
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int row = wrow0 + mb * 16 + r;
-    if (row >= qlen) continue;
-    const float l = lrow[mb];
-    const float inv = (l > 0.f && wpos0 + mb * 16 + r >= 0) ? oscale / l : 0.f;
-    uint16_t* op = a.out + (int64_t)(q0 + row) * a.out_stride_token + (int64_t)h * a.out_stride_head;
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const f32x4 o = oacc[nb][mb];
+    for (int e = 0; e < 4; ++e) {
       u32x2 w;
-      w.x = TT::pack2(o[0] * inv, o[1] * inv);
-      w.y = TT::pack2(o[2] * inv, o[3] * inv);
-      *reinterpret_cast<u32x2*>(op + nb * 16 + g * 4) = w;
+      w.x = TT::pack2(oacc[db][4 * e] * inv, oacc[db][4 * e + 1] * inv);
+      w.y = TT::pack2(oacc[db][4 * e + 2] * inv, oacc[db][4 * e + 3] * inv);
+      *reinterpret_cast<u32x2*>(op + db * 32 + e * 8 + hf * 4) = w;
     }
-  }
 }
 
 // Every head dim but 64 and 128 (multiples of 32 from 32 to 256): at 256 the
@@ -911,31 +1098,24 @@ int launch_generic(int64_t head_dim, const PrefillArgs& a, int64_t grid, hipStre
   return npd::check_launch(name);
 }
 
-template <class TT, int D, bool kOff32, bool kF8>
-int launch(int hw, const PrefillArgs& a, int64_t grid, hipStream_t st, const char* name) {
-  switch (hw) {
-    case 1: hipLaunchKernelGGL((prefill_kernel<TT, D, 1, kOff32, kF8>), dim3((unsigned)grid), dim3(kThreads), 0, st, a); break;
-    case 2: hipLaunchKernelGGL((prefill_kernel<TT, D, 2, kOff32, kF8>), dim3((unsigned)grid), dim3(kThreads), 0, st, a); break;
-    case 4: hipLaunchKernelGGL((prefill_kernel<TT, D, 4, kOff32, kF8>), dim3((unsigned)grid), dim3(kThreads), 0, st, a); break;
-    default: return npd::fail(NPD_E_INVALID, "%s: heads per workgroup %d", name, hw);
+template <class TT, bool kF8>
+int launch_dt(int64_t head_dim, bool off32, const PrefillArgs& a, int64_t grid, hipStream_t st,
+              const char* name) {
+  const dim3 g((unsigned)grid), b(kThreads);
+  if (head_dim == 64) {
+    if (off32) hipLaunchKernelGGL((prefill_kernel<TT, 64, true, kF8>), g, b, 0, st, a);
+    else hipLaunchKernelGGL((prefill_kernel<TT, 64, false, kF8>), g, b, 0, st, a);
+  } else {
+    if (off32) hipLaunchKernelGGL((prefill_kernel<TT, 128, true, kF8>), g, b, 0, st, a);
+    else hipLaunchKernelGGL((prefill_kernel<TT, 128, false, kF8>), g, b, 0, st, a);
   }
   return npd::check_launch(name);
 }
 
-template <class TT, bool kF8>
-int launch_dt(int64_t head_dim, bool off32, int hw, const PrefillArgs& a, int64_t grid,
-              hipStream_t st, const char* name) {
-  if (head_dim == 64)
-    return off32 ? launch<TT, 64, true, kF8>(hw, a, grid, st, name)
-                 : launch<TT, 64, false, kF8>(hw, a, grid, st, name);
-  return off32 ? launch<TT, 128, true, kF8>(hw, a, grid, st, name)
-               : launch<TT, 128, false, kF8>(hw, a, grid, st, name);
-}
-
 // Workspace: [counter region (kCounterBytes) | O partials | (m, l) partials].
-// Sized for the most records any head group / row tiling of these shapes can
-// address: a sequence has tiles_max * (4 / HW) * 2 <= ceil(max_q_len / 32) + 7
-// subtiles of 32 rows.
+// Sized for the most records any group size can address: a (sequence, kv head)
+// of G heads has 8 * ceil(max_q_len * G / 256) <= G * (ceil(max_q_len / 32) + 7)
+// subtiles of 32 flattened rows.
 struct Layout {
   int splits, ks_steps;
   int64_t o_off, ml_off, total;
@@ -1006,12 +1186,11 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
     return fail(NPD_E_INVALID, "%s: num_heads %lld is not a multiple of num_kv_heads %lld", name,
                 (long long)num_heads, (long long)num_kv_heads);
   const int64_t g = num_heads / num_kv_heads;
-  const int hw = (g % 4 == 0) ? 4 : (g % 2 == 0 ? 2 : 1);   // gcd(g, 4)
   if (num_blocks * block_size * num_kv_heads > INT32_MAX || max_blocks_per_seq * block_size > INT32_MAX)
     return fail(NPD_E_INVALID, "%s: pool exceeds int32 row indexing", name);
-  if (!generic && max_blocks_per_seq > kMaxBlocksLds)
+  if (!generic && max_blocks_per_seq > kMaxTableBlocks)
     return fail(NPD_E_INVALID, "%s: block tables wider than %d blocks are not supported", name,
-                kMaxBlocksLds);
+                kMaxTableBlocks);
   if (q_stride_token % 8 || q_stride_head % 8 || out_stride_token % 4 || out_stride_head % 4 ||
       q_stride_token < 0 || q_stride_head < 0 || out_stride_token < 0 || out_stride_head < 0)
     return fail(NPD_E_ALIGN, "%s: query strides must be multiples of 8 elements, out strides of 4",
@@ -1070,14 +1249,27 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
       return fail(NPD_E_ALIGN, "%s: workspace must be 256-byte aligned", name);
   }
-  const int rt = kPairs / hw;
-  const int64_t tiles = (max_q_len + 64LL * rt - 1) / (64LL * rt);
-  const int64_t hgroups = g / hw;
-  if (L.total > 0 && num_seqs * tiles * num_kv_heads * (g / hw) > kMaxCounters)
+  if (max_q_len * g > INT32_MAX - kTileRows)
+    return fail(NPD_E_INVALID, "%s: too many query rows", name);
+  const int64_t tiles = (max_q_len * g + kTileRows - 1) / kTileRows;
+  if (L.total > 0 && num_seqs * tiles * num_kv_heads > kMaxCounters)
     return fail(NPD_E_INVALID, "%s: too many query tiles for the %lld merge counters", name,
                 (long long)kMaxCounters);
-  const int64_t groups = (int64_t)L.splits * num_seqs * num_kv_heads;
-  const int64_t grid = (groups + 7) / 8 * 8 * tiles * hgroups;
+  // Up to kListTiles (sequence, tile) pairs the kernel cuts key ranges by the
+  // work it finds. More run whole, in a fixed order, unless they leave compute
+  // units idle (many short chunks on long prefixes).
+  const bool list = num_seqs * tiles <= kListTiles;
+  const bool whole = !list && total_q * num_heads >= 2LL * device_cus() * kTileRows;
+  const int splits = whole ? 1 : L.splits;
+  // Grid: the tiles there can be (a chunk's last tile may be part full), or
+  // two rounds of the compute units where the kernel may cut that many parts;
+  // a workgroup without an item ends after the work list.
+  const int64_t whole_tiles = num_seqs * tiles < total_q * g / kTileRows + num_seqs
+                                  ? num_seqs * tiles : total_q * g / kTileRows + num_seqs;
+  const int64_t two_rounds = (2LL * device_cus() + num_kv_heads - 1) / num_kv_heads;
+  const int64_t max_items = !list ? splits * num_seqs * tiles
+                            : splits > 1 && whole_tiles < two_rounds ? two_rounds : whole_tiles;
+  const int64_t grid = max_items * num_kv_heads;
   if (grid > INT32_MAX) return fail(NPD_E_INVALID, "%s: too many tiles", name);
 
   PrefillArgs a;
@@ -1097,16 +1289,15 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   a.num_seqs = (int)num_seqs;
   a.num_kv_heads = (int)num_kv_heads;
   a.group = (int)g;
-  a.hgroups = (int)hgroups;
   a.block_size = (int)block_size;
   a.bs_shift = (block_size & (block_size - 1)) == 0 ? __builtin_ctzll((unsigned long long)block_size) : -1;
   a.num_blocks = (int)num_blocks;
   a.max_bps = (int)max_blocks_per_seq;
   a.tiles_max = (int)tiles;
-  a.subtiles = (int)(tiles * rt * 2);
-  a.splits_max = L.splits;
+  a.subtiles = (int)(tiles * kWaves);
+  a.splits_max = splits;
   a.ks_steps = L.ks_steps;
-  a.num_groups = (int)groups;
+  a.max_items = (int)max_items;
   a.num_cus = device_cus();
   a.scale_log2 = scale * kLog2e;
   a.q_stride_token = q_stride_token;
@@ -1117,10 +1308,10 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   const int64_t elt = fp8 ? 1 : 2;
   const bool off32 = num_blocks * num_kv_heads * block_size * head_dim * elt <= (int64_t)UINT32_MAX;
   if (dtype == NPD_DTYPE_BF16)
-    return fp8 ? launch_dt<BF16, true>(head_dim, off32, hw, a, grid, st, name)
-               : launch_dt<BF16, false>(head_dim, off32, hw, a, grid, st, name);
-  return fp8 ? launch_dt<F16, true>(head_dim, off32, hw, a, grid, st, name)
-             : launch_dt<F16, false>(head_dim, off32, hw, a, grid, st, name);
+    return fp8 ? launch_dt<BF16, true>(head_dim, off32, a, grid, st, name)
+               : launch_dt<BF16, false>(head_dim, off32, a, grid, st, name);
+  return fp8 ? launch_dt<F16, true>(head_dim, off32, a, grid, st, name)
+             : launch_dt<F16, false>(head_dim, off32, a, grid, st, name);
 }
 
 }  // namespace

@@ -15,11 +15,11 @@ Kernels covered (the FP8 and 2-byte pools share their addressing):
   decode_schedule_kernel's, decode_fast_item's output, partial, group-slot,
   (m, l) and counter stores, merge_unit_fast's reads and stores, and the
   dynamic LDS of pass 1-3;
-- prefill_kernel's work list / fixed grid (prefill_attention.hip:164-288),
-  its zero rows, partial records, counters and output rows (:290-660);
+- prefill_kernel's work list / fixed grid (prefill_item), its zero rows,
+  partial records, counters, block list and output rows (prefill_attention.hip);
 - copy_blocks_kernel (copy_blocks.hip:15-29).
 Host-side choices (partition, grid, workspace layout) are restated from the
-entry points (decode_attention.hip:1192-1512, prefill_attention.hip:686-851);
+entry points (decode_attention.hip, prefill_attention.hip);
 the workspace sizes are asked of the built library itself.
 """
 from __future__ import annotations
@@ -86,7 +86,10 @@ def ring_of(D: int, G: int = 1, fp8: bool = False) -> int:
 KT = 64
 SPLIT_STEPS = 16
 MAX_SPLITS = 8
-MAX_BLOCKS_LDS = 16384
+TILE_ROWS = 256        # kTileRows: flattened (token, head) rows per workgroup
+LIST_TILES = 512       # kListTiles: tiles the in-kernel work list orders
+LIST_BLOCKS = 2048     # kListBlocks: blocks listed in LDS at a time
+MIN_PART, ITEM_STEPS, MERGE_STEPS = 4, 4, 4
 REC_ML = 2 * 64 * 2
 
 
@@ -552,29 +555,28 @@ class PrefillLaunch:
     max_bps: int
     max_q_len: int
     max_ctx: int
-    hw: int = 4
-    rt: int = 1
+    rt: int = 1          # 64-token blocks per tile (groups of 1, 2, 4 heads)
+    hgroups: int = 1     # every head of a kv head is in the tile
     tiles: int = 0
-    hgroups: int = 0
     splits: int = 1
     ks_steps: int = SPLIT_STEPS
     o_off: int = 0
     ml_off: int = 0
     total: int = 0
     grid: int = 0
-    groups: int = 0
+    max_items: int = 0
     subtiles: int = 0
     num_cus: int = 256
 
 
 def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
-                 D: int = 128) -> PrefillLaunch:
+                 D: int = 128, total_q: int | None = None) -> PrefillLaunch:
     """prefill_layout and prefill_impl (prefill_attention.hip), head dims 64
-    and 128 (prefill_kernel)."""
+    and 128 (prefill_kernel). total_q: S * max_q_len unless given."""
     assert D in (64, 128)
     L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus)
     g = H // KV
-    L.hw = 4 if g % 4 == 0 else (2 if g % 2 == 0 else 1)
+    tq = S * max_q_len if total_q is None else total_q
     if max_ctx > 0:
         steps = _ceil(max_ctx, KT)
         ks = max(_ceil(steps, MAX_SPLITS), SPLIT_STEPS)
@@ -588,146 +590,144 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
         L.o_off = K_COUNTER_BYTES
         L.ml_off = L.o_off + nrec * rec_o(D) * 4
         L.total = L.ml_off + nrec * REC_ML * 4
-    L.rt = 4 // L.hw
-    L.tiles = _ceil(max_q_len, 64 * L.rt)
-    L.hgroups = g // L.hw
-    L.groups = L.splits * S * KV
-    L.grid = _ceil(L.groups, 8) * 8 * L.tiles * L.hgroups
-    L.subtiles = L.tiles * L.rt * 2
+    L.rt = 4 // g
+    L.tiles = _ceil(max_q_len * g, TILE_ROWS)
+    L.subtiles = L.tiles * 8
+    in_list = S * L.tiles <= LIST_TILES
+    if not in_list and tq * H >= 2 * num_cus * TILE_ROWS:
+        L.splits = 1
+    whole = min(S * L.tiles, tq * g // TILE_ROWS + S)
+    two = _ceil(2 * num_cus, KV)
+    if not in_list:
+        L.max_items = L.splits * S * L.tiles
+    else:
+        L.max_items = two if L.splits > 1 and whole < two else whole
+    L.grid = L.max_items * KV
     return L
+
+
+def tile_keys(G: int, t: int, qlen: int, ctx: int) -> int:
+    """Keys that tile t of a chunk sees."""
+    last = min((t + 1) * TILE_ROWS, qlen * G) - 1
+    return max(ctx - qlen + last // G + 1, 0)
 
 
 def prefill_items(L: PrefillLaunch, cu: np.ndarray, ctx_lens: np.ndarray):
     """(s, t, j, kh, hg, q0, qlen, ctx, ks, eq) per running workgroup
-    (prefill_attention.hip:170-288)."""
-    TR = 64 * L.rt
+    (prefill_item); hg is 0 and eq (near-equal parts) True for every one."""
     cap = L.max_bps * L.bs
+    G = L.H // L.KV
     items = []
-    if L.S * L.tiles <= 64:
-        lane = np.arange(64)
-        ls, lt = lane // L.tiles, lane % L.tiles
-        valid = ls < L.S
-        c0 = np.zeros(64, np.int64)
-        ql = np.zeros(64, np.int64)
-        cx = np.zeros(64, np.int64)
-        n = np.zeros(64, np.int64)
-        for i in np.flatnonzero(valid):
-            c0[i] = cu[ls[i]]
-            ql[i] = cu[ls[i] + 1] - c0[i]
-            if lt[i] * TR < ql[i]:
-                cx[i] = min(max(int(ctx_lens[ls[i]]), 0), cap)
-                rw = min(ql[i] - lt[i] * TR, TR)
-                nk = max(0, cx[i] - ql[i] + lt[i] * TR + rw)
-                n[i] = _ceil(nk, KT)
-            else:
-                valid[i] = False
-        per_item = L.KV * L.hgroups
-        tot, nmax = int(n.sum()), int(n.max())
-        avg = _ceil(tot * per_item, L.num_cus)
-        parts = max(nmax // avg if avg > 0 else 1, 1)
-        ks = max(_ceil(nmax, parts), L.ks_steps)
-        # near-equal parts per tile; items by part length (longest first),
-        # then tile, part, (kv-head, head group)
-        nsp = np.where(valid, np.clip(_ceil(n, ks), 1, L.splits), 0)
-        ln = np.where(valid, _ceil(n, np.maximum(nsp, 1)), -1)
-        lenmax = int(ln.max())
-        frm = [int(nsp[ln >= b].sum()) * per_item for b in range(lenmax + 2)]
+    tiles = L.S * L.tiles
+    if tiles <= LIST_TILES:
+        n = np.zeros(tiles, np.int64)
+        valid = np.zeros(tiles, bool)
+        seq = [(int(cu[s]), int(cu[s + 1] - cu[s]), min(max(int(ctx_lens[s]), 0), cap))
+               for s in range(L.S)]
+        for i in range(tiles):
+            c0, ql, cx = seq[i // L.tiles]
+            valid[i] = (i % L.tiles) * TILE_ROWS < ql * G
+            if valid[i]:
+                n[i] = _ceil(tile_keys(G, i % L.tiles, ql, cx), KT)
+        tot, nmax, ntiles = int(n.sum()), int(n.max(initial=0)), int(valid.sum())
+
+        def cut_of(step):
+            return np.where(valid, np.clip(_ceil(n, step), 1, L.splits), 0)
+
+        ks = max(nmax, 1)
+        units = max(L.num_cus // L.KV, 1)
+        if L.splits > 1 and ntiles < 3 * units:
+            best = 0.0
+            for p in range(1, L.splits + 1):
+                kp = _ceil(nmax, p)
+                if p > 1 and kp < MIN_PART:
+                    break
+                c = cut_of(max(kp, 1))
+                cnt, cut = int(c.sum()), int(c[c > 1].sum())
+                if p > 1 and cnt > L.max_items:
+                    break
+                longest = kp + ITEM_STEPS + (MERGE_STEPS if p > 1 else 0)
+                mean = (tot + cnt * ITEM_STEPS + cut * MERGE_STEPS) / units
+                est = longest if cnt <= units else max(
+                    longest, mean + 0.35 * longest * (3 * units - cnt) / (2 * units))
+                if p == 1 or est < 0.97 * best:
+                    best, ks = est, max(kp, 1)
+        cut = cut_of(ks)
+        ln = np.where(valid, _ceil(n, np.maximum(cut, 1)), -1)
+        frm = [int(cut[ln >= b].sum()) * L.KV for b in range(int(ln.max(initial=-1)) + 2)]
         for bid in range(L.grid):
-            idv = bid
-            if idv >= frm[0]:
+            if not frm or bid >= frm[0]:
                 continue
-            lo = max(b for b in range(lenmax + 1) if frm[b] > idv)
-            idv -= frm[lo + 1]
-            lanes = np.flatnonzero(ln == lo)
-            if len(lanes) == 0:
+            lo = max(b for b in range(len(frm) - 1) if frm[b] > bid)
+            idv = bid - frm[lo + 1]
+            sel = None
+            for i in np.flatnonzero(ln == lo):   # slot rows, then lanes: index order
+                if idv < int(cut[i]) * L.KV:
+                    sel = int(i)
+                    break
+                idv -= int(cut[i]) * L.KV
+            if sel is None:
                 items.append(None)
                 continue
-            sel = int(lanes[0])
-            for k, l in enumerate(lanes):
-                sel = int(l)
-                c = int(nsp[l]) * per_item
-                if idv < c or k == len(lanes) - 1:
-                    break
-                idv -= c
-            j = idv // per_item
-            rem = idv - j * per_item
-            kh, hg = rem % L.KV, rem // L.KV
-            items.append((sel // L.tiles, sel % L.tiles, j, kh, hg, int(c0[sel]), int(ql[sel]),
-                          int(cx[sel]), ks, True))
+            c0, ql, cx = seq[sel // L.tiles]
+            items.append((sel // L.tiles, sel % L.tiles, idv // L.KV, idv % L.KV, 0, c0, ql, cx, ks,
+                          True))
         return items
-    gunits = L.tiles * L.hgroups
     for bid in range(L.grid):
-        xcd, p = bid & 7, bid >> 3
-        gi = (p // gunits) * 8 + xcd
-        if gi >= L.groups:
-            continue
-        u = p - (p // gunits) * gunits
-        t = L.tiles - 1 - u // L.hgroups
-        hg = u - (u // L.hgroups) * L.hgroups
-        kh = gi % L.KV
-        js = gi // L.KV
-        s = js % L.S
-        j = js // L.S
+        u, kh = divmod(bid, L.KV)
+        v, tr = divmod(u, L.tiles)
+        t = L.tiles - 1 - tr
+        j, s = divmod(v, L.S)
         q0 = int(cu[s])
         qlen = int(cu[s + 1]) - q0
-        if t * TR >= qlen:
+        if t * TILE_ROWS >= qlen * G:
             continue
         ctx = min(max(int(ctx_lens[s]), 0), cap)
-        items.append((s, t, j, kh, hg, q0, qlen, ctx, L.ks_steps, False))
+        items.append((s, t, j, kh, 0, q0, qlen, ctx, L.ks_steps, True))
     return items
 
 
 def prefill(W: Writes, L: PrefillLaunch, out: Buf, ws: Buf, cu: np.ndarray, ctx_lens: np.ndarray,
             out_stride_token: int, out_stride_head: int, D: int = 128) -> None:
-    TR = 64 * L.rt
     G = L.H // L.KV
     for it in prefill_items(L, cu, ctx_lens):
         if it is None:
             W.errors.append("prefill: a workgroup derived no tile (empty ballot)")
             continue
-        s, t, j, kh, hg, q0, qlen, ctx, ks, eq = it
+        s, t, j, kh, _, q0, qlen, ctx, ks, _ = it
         W.index([s], L.S, "prefill sequence")
-        prefix = ctx - qlen
-        rows = min(qlen - t * TR, TR)
-        pos0 = prefix + t * TR
-        nkeys = max(pos0 + rows, 0)
+        nkeys = tile_keys(G, t, qlen, ctx)
         nsteps = _ceil(nkeys, KT)
         nsp = min(max(_ceil(nsteps, ks), 1), L.splits)
         if j >= nsp:
             continue
-        if eq:   # near-equal parts, the first nsteps % nsp one step longer
-            base, rm = divmod(nsteps, nsp)
-            st0 = j * base + min(j, rm)
-            st1 = st0 + base + (1 if j < rm else 0)
-        else:
-            st0 = j * ks
-            st1 = nsteps if j == nsp - 1 else st0 + ks
-        kbeg = st0 * KT
+        base, rm = divmod(nsteps, nsp)   # near-equal parts
+        st0 = j * base + min(j, rm)
+        st1 = st0 + base + (1 if j < rm else 0)
         kend = min(st1 * KT, nkeys)
-        blk0 = kbeg // L.bs
-        nblk = _ceil(kend, L.bs) - blk0 if kend > kbeg else 0
-        W.index([nblk - 1] if nblk else [], MAX_BLOCKS_LDS, "prefill block ids in LDS")
-        W.index([blk0 + nblk - 1] if nblk else [], L.max_bps, "prefill block-table column")
+        seg = max((LIST_BLOCKS - 2) * L.bs // KT, 1)   # steps whose blocks the list holds
+        for sb in range(st0, st1, seg):
+            se = min(sb + seg, st1)
+            blk0 = sb * KT // L.bs
+            nblk = (min(se * KT, kend) - 1) // L.bs + 1 - blk0
+            W.index([nblk - 1], LIST_BLOCKS, "prefill block list in LDS")
+            W.index([blk0 + nblk - 1], L.max_bps, "prefill block-table column")
         for wave in range(8):
-            pair, half = wave >> 1, wave & 1
-            wr = pair // L.hw
-            h = kh * G + hg * L.hw + (pair - wr * L.hw)
-            wsub = (t * L.rt + wr) * 2 + half
-            wrow0 = wsub * WAVE_ROWS
-            r = np.arange(WAVE_ROWS) + wrow0
-            r = r[r < qlen]
-            lo = ((q0 + r) * out_stride_token + h * out_stride_head) * 2
+            wsub = t * 8 + wave
+            f = np.arange(WAVE_ROWS) + wsub * WAVE_ROWS
+            f = f[f < qlen * G]
+            lo = ((q0 + f // G) * out_stride_token + (kh * G + f % G) * out_stride_head) * 2
             W.add(out, lo, lo + 2 * D, "prefill output rows")
             if st0 >= st1 or nsp <= 1:
                 continue
-            rec = ((s * L.subtiles + wsub) * L.H + h) * L.splits
+            rec = ((s * L.KV + kh) * L.subtiles + wsub) * L.splits
             W.index([wsub], L.subtiles, "prefill subtile")
             for jj in (j, 0, nsp - 1):
                 o = L.o_off + (rec + jj) * rec_o(D) * 4
                 W.add(ws, o, o + rec_o(D) * 4, "prefill partial O")
                 o = L.ml_off + (rec + jj) * REC_ML * 4
                 W.add(ws, o, o + REC_ML * 4, "prefill partial (m, l)")
-            cidx = ((s * L.tiles + t) * L.KV + kh) * L.hgroups + hg
+            cidx = (s * L.tiles + t) * L.KV + kh
             W.index([cidx], K_MAX_COUNTERS, "prefill merge counter")
 
 

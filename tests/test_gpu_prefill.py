@@ -255,3 +255,53 @@ def test_head_dims_64_and_256_zero_rows_and_decode(device, hd):
     pk.paged_attention_forward(dec, q[-1:].contiguous(), kc, vc, bt, ctx, scale, 16, mb)
     torch.cuda.synchronize()
     assert max_abs(full[-1:], f32(dec).astype(np.float64)) <= ATOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("G,kvh", [(3, 2), (5, 1), (7, 2), (16, 1)])
+def test_flattened_rows_across_tiles(device, dtype, G, kvh):
+    """Tiles of 256 (token, head) rows that start and end inside a token, the
+    last rows of a chunk on a tile's first, and one token's heads alone."""
+    print(f"prefill flattened rows G={G} dtype={dtype}", flush=True)
+    chunks = [256 // G + 1, 1, 512 // G, 150]
+    args = make_case(device, [0, 333, 64, 1100], chunks, H=G * kvh, kvh=kvh, dtype=dtype, seed=G)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    check(run(*args, 0.09), q, kc, vc, bt, cu, ctx, 0.09)
+
+
+@pytest.mark.parametrize("S,longest", [(70, 60), (40, 700), (180, 200)])
+def test_many_tiles(device, S, longest):
+    """More than 64 (sequence, tile) pairs: 70 one-tile sequences, 40 x 11 in
+    the work list's further slots, 180 x 4 in the fixed order (cut key ranges:
+    the longest context is past 1024)."""
+    print(f"prefill many tiles S={S} longest={longest}", flush=True)
+    rng = np.random.default_rng(S)
+    chunks = [longest] + [int(x) for x in rng.integers(1, 24, S - 1)]
+    prefixes = [0, 1200] + [int(x) for x in rng.integers(0, 80, S - 2)]
+    args = make_case(device, prefixes, chunks, H=8, kvh=2, seed=S)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    check(run(*args, 0.1), q, kc, vc, bt, cu, ctx, 0.1)
+
+
+def test_block_list_in_segments(device):
+    """Blocks of one token: the block list in LDS is refilled along the key
+    range (2046 blocks at a time)."""
+    args = make_case(device, [4500, 0], [33, 20], H=4, kvh=1, bs=1, seed=11)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    check(run(*args, 0.1), q, kc, vc, bt, cu, ctx, 0.1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_exponent_reference_moves(device, dtype):
+    """Scores that climb by far more than 2^8 along the keys (the exponent
+    reference moves several times), that fall, and that start far below zero."""
+    args = make_case(device, [300, 300, 300], [40, 40, 40], H=4, kvh=1, dtype=dtype, seed=5)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    bs = kc.size(2)
+    ramp = torch.linspace(0, 1, 340, device=device)
+    for s, r in enumerate((6 * ramp, 6 - 6 * ramp, -8 + 4 * ramp)):
+        for i in range(340):
+            b = int(bt[s, i // bs])
+            kc[b, 0, i % bs] = (kc[b, 0, i % bs].float() * 0.2 + r[i]).to(dtype)
+    q.copy_((q.float() * 0.2 + 1.0).to(dtype))
+    check(run(*args, 0.12), q, kc, vc, bt, cu, ctx, 0.12)
