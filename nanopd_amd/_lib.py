@@ -96,8 +96,16 @@ def check(rc: int) -> None:
         raise NpdError(f"nanopd error {rc}: {msg}")
 
 
+_fns: dict = {}   # the library's functions by name, looked up once
+
+
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc != 0:
+        check(rc)
 
 
 def exported_symbols() -> list[str]:

@@ -21,6 +21,7 @@ There is no CPU or PyTorch fallback: without the built library every op raises.
 """
 from __future__ import annotations
 
+import functools
 import threading
 from typing import NamedTuple, Sequence
 
@@ -41,37 +42,50 @@ def _fail(msg: str) -> None:
     raise RuntimeError(msg)
 
 
-def _check(cond: bool, msg: str) -> None:
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def _dtype_code(t: torch.Tensor, what: str) -> int:
     code = _DTYPES.get(t.dtype)
-    _check(code is not None, f"{what}: dtype {t.dtype} not supported (float16 / bfloat16)")
+    if not (code is not None):
+        _fail(f"{what}: dtype {t.dtype} not supported (float16 / bfloat16)")
     return code
 
 
 def _int32(t: torch.Tensor, what: str) -> None:
-    _check(isinstance(t, torch.Tensor), f"{what} must be a tensor")
-    _check(t.dtype == torch.int32, f"{what} must be int32 (got {t.dtype})")
+    if not (isinstance(t, torch.Tensor)):
+        _fail(f"{what} must be a tensor")
+    if not (t.dtype == torch.int32):
+        _fail(f"{what} must be int32 (got {t.dtype})")
 
 
+# The checks of an op run on every call, ahead of a launch that takes a few
+# microseconds: they compare plain ints (a torch.device object per tensor costs
+# as much as a kernel argument block) and format a message only to raise it.
 def _same_device(dev: torch.device, *ts: torch.Tensor) -> None:
+    idx = dev.index if dev.type == "cuda" else -1
     for t in ts:
-        _check(t.device == dev, f"tensor on {t.device}, expected {dev}")
+        if t.get_device() != idx:
+            _fail(f"tensor on {t.device}, expected {dev}")
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(dev: torch.device) -> int:
+    """The current stream's handle (without a torch Stream object where torch
+    hands it out as it is)."""
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _cache_checks(k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
-    _check(k_cache.dim() == 4 and v_cache.dim() == 4,
-           "caches must be [num_blocks, num_kv_heads, block_size, head_dim]")
-    _check(k_cache.shape == v_cache.shape, "k_cache and v_cache shapes differ")
-    _check(k_cache.dtype == v_cache.dtype, "k_cache and v_cache dtypes differ")
-    _check(k_cache.is_contiguous() and v_cache.is_contiguous(), "caches must be contiguous")
+    if not (k_cache.dim() == 4 and v_cache.dim() == 4):
+        _fail("caches must be [num_blocks, num_kv_heads, block_size, head_dim]")
+    if not (k_cache.shape == v_cache.shape):
+        _fail("k_cache and v_cache shapes differ")
+    if not (k_cache.dtype == v_cache.dtype):
+        _fail("k_cache and v_cache dtypes differ")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        _fail("caches must be contiguous")
 
 
 # ---------------------------------------------------------------------------
@@ -91,19 +105,24 @@ def paged_kv_store(k_cache: torch.Tensor, v_cache: torch.Tensor, k_src: torch.Te
     ``(k_cache, v_cache, k_src[1, kvh, T, D], v_src, block_table[nb], start_pos: int)``,
     is accepted too and means positions ``start_pos + t`` on a shared table.
     """
-    _check(isinstance(k_src, torch.Tensor) and k_src.is_cuda, "k src is must be on CUDA")
-    _check(isinstance(v_src, torch.Tensor) and v_src.is_cuda, "v src is must be on CUDA")
+    if not (isinstance(k_src, torch.Tensor) and k_src.is_cuda):
+        _fail("k src is must be on CUDA")
+    if not (isinstance(v_src, torch.Tensor) and v_src.is_cuda):
+        _fail("v src is must be on CUDA")
     if isinstance(positions, int):
-        _check(k_src.dim() == 4 and k_src.size(0) == 1 and v_src.dim() == 4,
-               "start-position form needs k_src/v_src of shape [1, kvh, T, D]")
+        if not (k_src.dim() == 4 and k_src.size(0) == 1 and v_src.dim() == 4):
+            _fail("start-position form needs k_src/v_src of shape [1, kvh, T, D]")
         _int32(block_tables, "block_table")
-        _check(block_tables.dim() == 1, "start-position form needs a 1-D block table")
+        if not (block_tables.dim() == 1):
+            _fail("start-position form needs a 1-D block table")
         k_src, v_src = k_src[0], v_src[0]
         n = k_src.size(1)
         positions = torch.arange(positions, positions + n, dtype=torch.int32, device=k_src.device)
         block_tables = block_tables.unsqueeze(0).expand(n, -1).contiguous()
-    _check(k_src.dim() == 3, "k_src must be [num_kv_heads, num_tokens, head_dim]")
-    _check(v_src.shape == k_src.shape, "k_src and v_src shapes differ")
+    if not (k_src.dim() == 3):
+        _fail("k_src must be [num_kv_heads, num_tokens, head_dim]")
+    if not (v_src.shape == k_src.shape):
+        _fail("k_src and v_src shapes differ")
     _cache_checks(k_cache, v_cache)
     _int32(block_tables, "block_tables")
     _int32(positions, "positions")
@@ -111,14 +130,17 @@ def paged_kv_store(k_cache: torch.Tensor, v_cache: torch.Tensor, k_src: torch.Te
     _same_device(dev, v_src, k_cache, v_cache, block_tables, positions)
     kvh, n, d = k_src.shape
     num_blocks, ckvh, bs, cd = k_cache.shape
-    _check(ckvh == kvh and cd == d, f"source [{kvh}, {n}, {d}] does not match cache {tuple(k_cache.shape)}")
-    _check(k_src.dtype == k_cache.dtype and v_src.dtype == k_cache.dtype, "source/cache dtype mismatch")
+    if not (ckvh == kvh and cd == d):
+        _fail(f"source [{kvh}, {n}, {d}] does not match cache {tuple(k_cache.shape)}")
+    if not (k_src.dtype == k_cache.dtype and v_src.dtype == k_cache.dtype):
+        _fail("source/cache dtype mismatch")
     code = _dtype_code(k_cache, "paged_kv_store")
-    _check(block_tables.dim() == 2 and block_tables.size(0) >= n,
-           "block_tables must be [num_tokens, max_blocks_per_seq]")
-    _check(block_tables.is_contiguous(), "block_tables must be contiguous")
-    _check(positions.dim() == 1 and positions.numel() >= n and positions.is_contiguous(),
-           "positions must be a contiguous [num_tokens] tensor")
+    if not (block_tables.dim() == 2 and block_tables.size(0) >= n):
+        _fail("block_tables must be [num_tokens, max_blocks_per_seq]")
+    if not (block_tables.is_contiguous()):
+        _fail("block_tables must be contiguous")
+    if not (positions.dim() == 1 and positions.numel() >= n and positions.is_contiguous()):
+        _fail("positions must be a contiguous [num_tokens] tensor")
     if n == 0:
         return
     if k_src.stride(2) != 1 or v_src.stride() != k_src.stride():
@@ -138,21 +160,27 @@ def paged_kv_store_slots(k_cache: torch.Tensor, v_cache: torch.Tensor, k_src: to
     int32 [num_tokens], ``slot = block * block_size + offset``; negative slots
     are skipped.
     """
-    _check(isinstance(k_src, torch.Tensor) and k_src.is_cuda, "k src is must be on CUDA")
-    _check(isinstance(v_src, torch.Tensor) and v_src.is_cuda, "v src is must be on CUDA")
-    _check(k_src.dim() == 3, "k_src must be [num_tokens, num_kv_heads, head_dim]")
-    _check(v_src.shape == k_src.shape, "k_src and v_src shapes differ")
+    if not (isinstance(k_src, torch.Tensor) and k_src.is_cuda):
+        _fail("k src is must be on CUDA")
+    if not (isinstance(v_src, torch.Tensor) and v_src.is_cuda):
+        _fail("v src is must be on CUDA")
+    if not (k_src.dim() == 3):
+        _fail("k_src must be [num_tokens, num_kv_heads, head_dim]")
+    if not (v_src.shape == k_src.shape):
+        _fail("k_src and v_src shapes differ")
     _cache_checks(k_cache, v_cache)
     _int32(slot_mapping, "slot_mapping")
     dev = k_src.device
     _same_device(dev, v_src, k_cache, v_cache, slot_mapping)
     n, kvh, d = k_src.shape
     num_blocks, ckvh, bs, cd = k_cache.shape
-    _check(ckvh == kvh and cd == d, "source does not match cache shape")
-    _check(k_src.dtype == k_cache.dtype and v_src.dtype == k_cache.dtype, "source/cache dtype mismatch")
+    if not (ckvh == kvh and cd == d):
+        _fail("source does not match cache shape")
+    if not (k_src.dtype == k_cache.dtype and v_src.dtype == k_cache.dtype):
+        _fail("source/cache dtype mismatch")
     code = _dtype_code(k_cache, "paged_kv_store_slots")
-    _check(slot_mapping.dim() == 1 and slot_mapping.numel() >= n and slot_mapping.is_contiguous(),
-           "slot_mapping must be a contiguous [num_tokens] tensor")
+    if not (slot_mapping.dim() == 1 and slot_mapping.numel() >= n and slot_mapping.is_contiguous()):
+        _fail("slot_mapping must be a contiguous [num_tokens] tensor")
     if n == 0:
         return
     if k_src.stride(2) != 1 or v_src.stride() != k_src.stride():
@@ -167,16 +195,17 @@ FP8_DTYPES = (torch.uint8, torch.float8_e4m3fn)
 
 def _fp8_cache_checks(k_cache: torch.Tensor, v_cache: torch.Tensor, k_scale: torch.Tensor,
                       v_scale: torch.Tensor) -> None:
-    _check(k_cache.dim() == 4 and v_cache.dim() == 4 and k_cache.shape == v_cache.shape,
-           "fp8 caches must be [num_blocks, num_kv_heads, block_size, head_dim]")
-    _check(k_cache.dtype in FP8_DTYPES and v_cache.dtype == k_cache.dtype,
-           "fp8 caches must be torch.float8_e4m3fn (or uint8 holding e4m3 bytes)")
-    _check(k_cache.is_contiguous() and v_cache.is_contiguous(), "caches must be contiguous")
+    if not (k_cache.dim() == 4 and v_cache.dim() == 4 and k_cache.shape == v_cache.shape):
+        _fail("fp8 caches must be [num_blocks, num_kv_heads, block_size, head_dim]")
+    if not (k_cache.dtype in FP8_DTYPES and v_cache.dtype == k_cache.dtype):
+        _fail("fp8 caches must be torch.float8_e4m3fn (or uint8 holding e4m3 bytes)")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        _fail("caches must be contiguous")
     kvh = k_cache.size(1)
     for sc, nm in ((k_scale, "k_scale"), (v_scale, "v_scale")):
-        _check(isinstance(sc, torch.Tensor) and sc.dtype == torch.float32 and sc.dim() == 1
-               and sc.numel() == kvh and sc.is_contiguous(),
-               f"{nm} must be a contiguous float32 [num_kv_heads] tensor")
+        if not (isinstance(sc, torch.Tensor) and sc.dtype == torch.float32 and sc.dim() == 1
+                and sc.numel() == kvh and sc.is_contiguous()):
+            _fail(f"{nm} must be a contiguous float32 [num_kv_heads] tensor")
 
 
 def paged_kv_store_slots_fp8(k_cache: torch.Tensor, v_cache: torch.Tensor, k_src: torch.Tensor,
@@ -185,20 +214,23 @@ def paged_kv_store_slots_fp8(k_cache: torch.Tensor, v_cache: torch.Tensor, k_src
     """:func:`paged_kv_store_slots` into an FP8 (OCP e4m3) pool with
     per-kv-head scales (no reference counterpart; its caches are fp16):
     byte = e4m3(clamp(x / scale[h], -448, 448)), round to nearest even."""
-    _check(isinstance(k_src, torch.Tensor) and k_src.is_cuda, "k src is must be on CUDA")
-    _check(k_src.dim() == 3 and v_src.shape == k_src.shape,
-           "k_src / v_src must be [num_tokens, num_kv_heads, head_dim]")
+    if not (isinstance(k_src, torch.Tensor) and k_src.is_cuda):
+        _fail("k src is must be on CUDA")
+    if not (k_src.dim() == 3 and v_src.shape == k_src.shape):
+        _fail("k_src / v_src must be [num_tokens, num_kv_heads, head_dim]")
     _fp8_cache_checks(k_cache, v_cache, k_scale, v_scale)
     _int32(slot_mapping, "slot_mapping")
     dev = k_src.device
     _same_device(dev, v_src, k_cache, v_cache, slot_mapping, k_scale, v_scale)
     n, kvh, d = k_src.shape
     num_blocks, ckvh, bs, cd = k_cache.shape
-    _check(ckvh == kvh and cd == d, "source does not match cache shape")
-    _check(v_src.dtype == k_src.dtype, "k_src / v_src dtypes differ")
+    if not (ckvh == kvh and cd == d):
+        _fail("source does not match cache shape")
+    if not (v_src.dtype == k_src.dtype):
+        _fail("k_src / v_src dtypes differ")
     code = _dtype_code(k_src, "paged_kv_store_slots_fp8")
-    _check(slot_mapping.dim() == 1 and slot_mapping.numel() >= n and slot_mapping.is_contiguous(),
-           "slot_mapping must be a contiguous [num_tokens] tensor")
+    if not (slot_mapping.dim() == 1 and slot_mapping.numel() >= n and slot_mapping.is_contiguous()):
+        _fail("slot_mapping must be a contiguous [num_tokens] tensor")
     if n == 0:
         return
     if k_src.stride(2) != 1 or v_src.stride() != k_src.stride():
@@ -234,6 +266,7 @@ def _decode_workspace(dev: torch.device, stream: int, need: int, kind: str = "de
         return ws
 
 
+@functools.lru_cache(maxsize=1024)
 def attention_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
                               block_size: int, max_num_blocks_per_seq: int) -> int:
     return int(_lib.load().npd_paged_attention_workspace_size(
@@ -254,9 +287,12 @@ def paged_attention_forward(out: torch.Tensor, query: torch.Tensor, key_cache: t
     zero-filled before its first use, replaces the cached per-stream one; calls
     that share a workspace must run in stream order.
     """
-    _check(isinstance(query, torch.Tensor) and query.is_cuda, "query is must be on CUDA")
-    _check(query.dim() == 3, "query must be [num seqs, num_heads, head_size]")
-    _check(key_cache.dim() == 4, "key_cache must be [num_blocks, num_kv_heads, block_size, head_size]")
+    if not (isinstance(query, torch.Tensor) and query.is_cuda):
+        _fail("query is must be on CUDA")
+    if not (query.dim() == 3):
+        _fail("query must be [num seqs, num_heads, head_size]")
+    if not (key_cache.dim() == 4):
+        _fail("key_cache must be [num_blocks, num_kv_heads, block_size, head_size]")
     _int32(block_tables, "block_tables")
     _int32(seq_lens, "seq_lens")
     _cache_checks(key_cache, value_cache)
@@ -264,19 +300,26 @@ def paged_attention_forward(out: torch.Tensor, query: torch.Tensor, key_cache: t
     _same_device(dev, out, key_cache, value_cache, block_tables, seq_lens)
     s, h, d = query.shape
     num_blocks, kvh, bs, cd = key_cache.shape
-    _check(cd == d, f"head_dim {d} does not match cache head_dim {cd}")
-    _check(int(block_size) == bs, f"block_size {block_size} does not match cache block size {bs}")
-    _check(h % kvh == 0, f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
-    _check(out.shape == query.shape and out.dtype == query.dtype, "out must match query")
-    _check(query.dtype == key_cache.dtype, "query/cache dtype mismatch")
+    if not (cd == d):
+        _fail(f"head_dim {d} does not match cache head_dim {cd}")
+    if not (int(block_size) == bs):
+        _fail(f"block_size {block_size} does not match cache block size {bs}")
+    if not (h % kvh == 0):
+        _fail(f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
+    if not (out.shape == query.shape and out.dtype == query.dtype):
+        _fail("out must match query")
+    if not (query.dtype == key_cache.dtype):
+        _fail("query/cache dtype mismatch")
     code = _dtype_code(query, "paged_attention_forward")
     mb = int(max_num_blocks_per_seq)
-    _check(block_tables.dim() == 2 and block_tables.size(0) >= s and block_tables.size(1) == mb,
-           "block_tables must be [num_seqs, max_num_blocks_per_seq]")
-    _check(block_tables.is_contiguous(), "block_tables must be contiguous")
-    _check(seq_lens.dim() == 1 and seq_lens.numel() >= s and seq_lens.is_contiguous(),
-           "seq_lens must be a contiguous [num_seqs] tensor")
-    _check(query.stride(2) == 1 and out.stride(2) == 1, "head_dim must be the contiguous dim")
+    if not (block_tables.dim() == 2 and block_tables.size(0) >= s and block_tables.size(1) == mb):
+        _fail("block_tables must be [num_seqs, max_num_blocks_per_seq]")
+    if not (block_tables.is_contiguous()):
+        _fail("block_tables must be contiguous")
+    if not (seq_lens.dim() == 1 and seq_lens.numel() >= s and seq_lens.is_contiguous()):
+        _fail("seq_lens must be a contiguous [num_seqs] tensor")
+    if not (query.stride(2) == 1 and out.stride(2) == 1):
+        _fail("head_dim must be the contiguous dim")
     if s == 0:
         return
     need = attention_workspace_bytes(s, h, kvh, d, bs, mb)
@@ -285,8 +328,8 @@ def paged_attention_forward(out: torch.Tensor, query: torch.Tensor, key_cache: t
     if need > 0:
         if workspace is None:
             workspace = _decode_workspace(dev, stream, need)
-        _check(workspace.numel() * workspace.element_size() >= need,
-               f"workspace of {need} bytes needed")
+        if not (workspace.numel() * workspace.element_size() >= need):
+            _fail(f"workspace of {need} bytes needed")
         ws_ptr = workspace.data_ptr()
     _lib.call("npd_paged_attention", out.data_ptr(), query.data_ptr(), key_cache.data_ptr(),
               value_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(), s, h, kvh, d,
@@ -303,8 +346,10 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
     """:func:`paged_attention_forward` over an FP8 pool written by
     :func:`paged_kv_store_slots_fp8`: K = e4m3(byte) * k_scale[kv head], V
     likewise. query/out fp16 or bf16; head_dim 128; block_size 16 or 32."""
-    _check(isinstance(query, torch.Tensor) and query.is_cuda, "query is must be on CUDA")
-    _check(query.dim() == 3, "query must be [num seqs, num_heads, head_size]")
+    if not (isinstance(query, torch.Tensor) and query.is_cuda):
+        _fail("query is must be on CUDA")
+    if not (query.dim() == 3):
+        _fail("query must be [num seqs, num_heads, head_size]")
     _fp8_cache_checks(key_cache, value_cache, k_scale, v_scale)
     _int32(block_tables, "block_tables")
     _int32(seq_lens, "seq_lens")
@@ -312,18 +357,24 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
     _same_device(dev, out, key_cache, value_cache, block_tables, seq_lens, k_scale, v_scale)
     s, h, d = query.shape
     num_blocks, kvh, bs, cd = key_cache.shape
-    _check(cd == d, f"head_dim {d} does not match cache head_dim {cd}")
-    _check(int(block_size) == bs, f"block_size {block_size} does not match cache block size {bs}")
-    _check(h % kvh == 0, f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
-    _check(out.shape == query.shape and out.dtype == query.dtype, "out must match query")
+    if not (cd == d):
+        _fail(f"head_dim {d} does not match cache head_dim {cd}")
+    if not (int(block_size) == bs):
+        _fail(f"block_size {block_size} does not match cache block size {bs}")
+    if not (h % kvh == 0):
+        _fail(f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
+    if not (out.shape == query.shape and out.dtype == query.dtype):
+        _fail("out must match query")
     code = _dtype_code(query, "paged_attention_forward_fp8")
     mb = int(max_num_blocks_per_seq)
-    _check(block_tables.dim() == 2 and block_tables.size(0) >= s and block_tables.size(1) == mb,
-           "block_tables must be [num_seqs, max_num_blocks_per_seq]")
-    _check(block_tables.is_contiguous(), "block_tables must be contiguous")
-    _check(seq_lens.dim() == 1 and seq_lens.numel() >= s and seq_lens.is_contiguous(),
-           "seq_lens must be a contiguous [num_seqs] tensor")
-    _check(query.stride(2) == 1 and out.stride(2) == 1, "head_dim must be the contiguous dim")
+    if not (block_tables.dim() == 2 and block_tables.size(0) >= s and block_tables.size(1) == mb):
+        _fail("block_tables must be [num_seqs, max_num_blocks_per_seq]")
+    if not (block_tables.is_contiguous()):
+        _fail("block_tables must be contiguous")
+    if not (seq_lens.dim() == 1 and seq_lens.numel() >= s and seq_lens.is_contiguous()):
+        _fail("seq_lens must be a contiguous [num_seqs] tensor")
+    if not (query.stride(2) == 1 and out.stride(2) == 1):
+        _fail("head_dim must be the contiguous dim")
     if s == 0:
         return
     need = attention_workspace_bytes(s, h, kvh, d, bs, mb)
@@ -332,8 +383,8 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
     if need > 0:
         if workspace is None:
             workspace = _decode_workspace(dev, stream, need)
-        _check(workspace.numel() * workspace.element_size() >= need,
-               f"workspace of {need} bytes needed")
+        if not (workspace.numel() * workspace.element_size() >= need):
+            _fail(f"workspace of {need} bytes needed")
         ws_ptr = workspace.data_ptr()
     _lib.call("npd_paged_attention_fp8", out.data_ptr(), query.data_ptr(), key_cache.data_ptr(),
               value_cache.data_ptr(), block_tables.data_ptr(), seq_lens.data_ptr(),
@@ -346,6 +397,7 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
 # Chunked prefill attention
 # ---------------------------------------------------------------------------
 
+@functools.lru_cache(maxsize=1024)
 def prefill_workspace_bytes(num_seqs: int, total_q: int, num_heads: int, head_dim: int,
                             max_q_len: int, max_context_len: int) -> int:
     return int(_lib.load().npd_paged_prefill_workspace_size(
@@ -355,8 +407,10 @@ def prefill_workspace_bytes(num_seqs: int, total_q: int, num_heads: int, head_di
 def _prefill(out, query, key_cache, value_cache, block_tables, cu_seqlens_q, context_lens, scale,
              block_size, max_num_blocks_per_seq, max_q_len, max_context_len, workspace,
              fp8_scales):
-    _check(isinstance(query, torch.Tensor) and query.is_cuda, "query is must be on CUDA")
-    _check(query.dim() == 3, "query must be [total_q, num_heads, head_size]")
+    if not (isinstance(query, torch.Tensor) and query.is_cuda):
+        _fail("query is must be on CUDA")
+    if not (query.dim() == 3):
+        _fail("query must be [total_q, num_heads, head_size]")
     _int32(block_tables, "block_tables")
     _int32(cu_seqlens_q, "cu_seqlens_q")
     _int32(context_lens, "context_lens")
@@ -369,22 +423,29 @@ def _prefill(out, query, key_cache, value_cache, block_tables, cu_seqlens_q, con
                  *(fp8_scales or ()))
     tq, h, d = query.shape
     num_blocks, kvh, bs, cd = key_cache.shape
-    _check(cd == d, f"head_dim {d} does not match cache head_dim {cd}")
-    _check(int(block_size) == bs, f"block_size {block_size} does not match cache block size {bs}")
-    _check(h % kvh == 0, f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
-    _check(out.shape == query.shape and out.dtype == query.dtype, "out must match query")
+    if not (cd == d):
+        _fail(f"head_dim {d} does not match cache head_dim {cd}")
+    if not (int(block_size) == bs):
+        _fail(f"block_size {block_size} does not match cache block size {bs}")
+    if not (h % kvh == 0):
+        _fail(f"num_heads {h} is not a multiple of num_kv_heads {kvh}")
+    if not (out.shape == query.shape and out.dtype == query.dtype):
+        _fail("out must match query")
     if fp8_scales is None:
-        _check(query.dtype == key_cache.dtype, "query/cache dtype mismatch")
+        if not (query.dtype == key_cache.dtype):
+            _fail("query/cache dtype mismatch")
     code = _dtype_code(query, "paged_prefill_attention")
     ns = cu_seqlens_q.numel() - 1
     mb = int(max_num_blocks_per_seq)
-    _check(ns >= 0 and cu_seqlens_q.dim() == 1 and cu_seqlens_q.is_contiguous(),
-           "cu_seqlens_q must be a contiguous [num_seqs + 1] tensor")
-    _check(context_lens.dim() == 1 and context_lens.numel() >= ns and context_lens.is_contiguous(),
-           "context_lens must be a contiguous [num_seqs] tensor")
-    _check(block_tables.dim() == 2 and block_tables.size(0) >= ns and block_tables.size(1) == mb
-           and block_tables.is_contiguous(), "block_tables must be [num_seqs, max_num_blocks_per_seq]")
-    _check(query.stride(2) == 1 and out.stride(2) == 1, "head_dim must be the contiguous dim")
+    if not (ns >= 0 and cu_seqlens_q.dim() == 1 and cu_seqlens_q.is_contiguous()):
+        _fail("cu_seqlens_q must be a contiguous [num_seqs + 1] tensor")
+    if not (context_lens.dim() == 1 and context_lens.numel() >= ns and context_lens.is_contiguous()):
+        _fail("context_lens must be a contiguous [num_seqs] tensor")
+    if not (block_tables.dim() == 2 and block_tables.size(0) >= ns and block_tables.size(1) == mb
+            and block_tables.is_contiguous()):
+        _fail("block_tables must be [num_seqs, max_num_blocks_per_seq]")
+    if not (query.stride(2) == 1 and out.stride(2) == 1):
+        _fail("head_dim must be the contiguous dim")
     if ns == 0 or tq == 0:
         return
     mctx = int(max_context_len) if max_context_len is not None else mb * bs
@@ -394,8 +455,8 @@ def _prefill(out, query, key_cache, value_cache, block_tables, cu_seqlens_q, con
     if need > 0:
         if workspace is None:
             workspace = _decode_workspace(dev, stream, need, "prefill")
-        _check(workspace.numel() * workspace.element_size() >= need,
-               f"workspace of {need} bytes needed")
+        if not (workspace.numel() * workspace.element_size() >= need):
+            _fail(f"workspace of {need} bytes needed")
         ws_ptr = workspace.data_ptr()
     ptrs = (out.data_ptr(), query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
             block_tables.data_ptr(), cu_seqlens_q.data_ptr(), context_lens.data_ptr())
@@ -464,19 +525,20 @@ def copy_blocks(k_cache: torch.Tensor, v_cache: torch.Tensor, block_pairs) -> No
     if k_cache.dtype in FP8_DTYPES and v_cache.dtype == k_cache.dtype:
         # a block copy moves bytes: a 1-byte pool is passed as 2-byte
         # elements, half as many per row (head_dim is even)
-        _check(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.size(-1) % 2 == 0,
-               "fp8 caches must be contiguous with an even head_dim")
+        if not (k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.size(-1) % 2 == 0):
+            _fail("fp8 caches must be contiguous with an even head_dim")
         k_cache = k_cache.view(torch.uint8).view(torch.bfloat16)
         v_cache = v_cache.view(torch.uint8).view(torch.bfloat16)
     _cache_checks(k_cache, v_cache)
     dev = k_cache.device
-    _check(k_cache.is_cuda, "caches must be on CUDA")
+    if not (k_cache.is_cuda):
+        _fail("caches must be on CUDA")
     if not isinstance(block_pairs, torch.Tensor):
         block_pairs = torch.tensor(list(block_pairs), dtype=torch.int32).reshape(-1, 2).to(dev)
     _int32(block_pairs, "block_pairs")
     _same_device(dev, block_pairs)
-    _check(block_pairs.dim() == 2 and block_pairs.size(1) == 2 and block_pairs.is_contiguous(),
-           "block_pairs must be a contiguous [N, 2] tensor")
+    if not (block_pairs.dim() == 2 and block_pairs.size(1) == 2 and block_pairs.is_contiguous()):
+        _fail("block_pairs must be a contiguous [N, 2] tensor")
     n = block_pairs.size(0)
     if n == 0:
         return
@@ -489,19 +551,22 @@ def copy_blocks(k_cache: torch.Tensor, v_cache: torch.Tensor, block_pairs) -> No
 def _block_list(block_table, dev: torch.device) -> torch.Tensor:
     if isinstance(block_table, torch.Tensor):
         _int32(block_table, "block_table")
-        _check(block_table.dim() == 1 and block_table.is_contiguous(),
-               "block_table must be a contiguous 1-D int32 tensor")
+        if not (block_table.dim() == 1 and block_table.is_contiguous()):
+            _fail("block_table must be a contiguous 1-D int32 tensor")
         _same_device(dev, block_table)
         return block_table
     return torch.tensor(list(block_table), dtype=torch.int32).to(dev)
 
 
 def _pool_checks(k_cache: torch.Tensor, v_cache: torch.Tensor, what: str) -> None:
-    _check(k_cache.is_cuda, f"{what}: caches must be on CUDA")
-    _check(k_cache.dim() == 5 and v_cache.shape == k_cache.shape,
-           f"{what}: caches must be [num_layers, num_blocks, num_kv_heads, block_size, head_dim]")
-    _check(k_cache.dtype == v_cache.dtype, f"{what}: k_cache and v_cache dtypes differ")
-    _check(k_cache.is_contiguous() and v_cache.is_contiguous(), f"{what}: caches must be contiguous")
+    if not (k_cache.is_cuda):
+        _fail(f"{what}: caches must be on CUDA")
+    if not (k_cache.dim() == 5 and v_cache.shape == k_cache.shape):
+        _fail(f"{what}: caches must be [num_layers, num_blocks, num_kv_heads, block_size, head_dim]")
+    if not (k_cache.dtype == v_cache.dtype):
+        _fail(f"{what}: k_cache and v_cache dtypes differ")
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        _fail(f"{what}: caches must be contiguous")
 
 
 def extract_kv(k_cache: torch.Tensor, v_cache: torch.Tensor, block_table,
@@ -523,8 +588,8 @@ def extract_kv(k_cache: torch.Tensor, v_cache: torch.Tensor, block_table,
     if out_v is None:
         out_v = torch.empty(shape, dtype=k_cache.dtype, device=dev)
     for o in (out_k, out_v):
-        _check(tuple(o.shape) == shape and o.dtype == k_cache.dtype and o.is_contiguous(),
-               f"extract_kv: wire buffers must be contiguous {list(shape)} of the cache dtype")
+        if not (tuple(o.shape) == shape and o.dtype == k_cache.dtype and o.is_contiguous()):
+            _fail(f"extract_kv: wire buffers must be contiguous {list(shape)} of the cache dtype")
         _same_device(dev, o)
     block_bytes = k_cache[0, 0].numel() * k_cache.element_size()
     _lib.call("npd_kv_gather_blocks", k_cache.data_ptr(), v_cache.data_ptr(), L, nb, block_bytes,
@@ -543,8 +608,8 @@ def load_kv(k_cache: torch.Tensor, v_cache: torch.Tensor, block_table, wire_k: t
     L, nb = k_cache.shape[:2]
     shape = (L, ids.numel()) + tuple(k_cache.shape[2:])
     for w in (wire_k, wire_v):
-        _check(tuple(w.shape) == shape and w.dtype == k_cache.dtype and w.is_contiguous(),
-               f"load_kv: wire buffers must be contiguous {list(shape)} of the cache dtype")
+        if not (tuple(w.shape) == shape and w.dtype == k_cache.dtype and w.is_contiguous()):
+            _fail(f"load_kv: wire buffers must be contiguous {list(shape)} of the cache dtype")
         _same_device(dev, w)
     block_bytes = k_cache[0, 0].numel() * k_cache.element_size()
     _lib.call("npd_kv_scatter_blocks", k_cache.data_ptr(), v_cache.data_ptr(), L, nb, block_bytes,
@@ -580,32 +645,37 @@ def qk_norm_rope_store(q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     else:
         _cache_checks(k_cache, v_cache)
     dev = qkv.device
-    _check(qkv.is_cuda, "qkv must be on CUDA")
-    _check((q_norm_weight is None) == (k_norm_weight is None),
-           "pass both norm weights (Qwen3) or neither (Qwen2 / Llama)")
+    if not (qkv.is_cuda):
+        _fail("qkv must be on CUDA")
+    if not ((q_norm_weight is None) == (k_norm_weight is None)):
+        _fail("pass both norm weights (Qwen3) or neither (Qwen2 / Llama)")
     norms = [w for w in (q_norm_weight, k_norm_weight) if w is not None]
     _same_device(dev, q_out, k_cache, v_cache, slot_mapping, positions, inv_freq, *norms)
     _int32(slot_mapping, "slot_mapping")
     _int32(positions, "positions")
     num_blocks, kvh, bs, d = k_cache.shape
-    _check(q_out.dim() == 3 and q_out.size(2) == d, "q_out must be [num_tokens, num_heads, head_dim]")
+    if not (q_out.dim() == 3 and q_out.size(2) == d):
+        _fail("q_out must be [num_tokens, num_heads, head_dim]")
     t, h = q_out.size(0), q_out.size(1)
-    _check(qkv.dim() == 2 and qkv.size(0) == t and qkv.size(1) == (h + 2 * kvh) * d,
-           "qkv must be [num_tokens, (num_heads + 2 * num_kv_heads) * head_dim]")
-    _check(qkv.stride(1) == 1, "qkv rows must be contiguous")
-    _check(q_out.stride(2) == 1 and q_out.stride(1) == d, "q_out heads must be contiguous")
+    if not (qkv.dim() == 2 and qkv.size(0) == t and qkv.size(1) == (h + 2 * kvh) * d):
+        _fail("qkv must be [num_tokens, (num_heads + 2 * num_kv_heads) * head_dim]")
+    if not (qkv.stride(1) == 1):
+        _fail("qkv rows must be contiguous")
+    if not (q_out.stride(2) == 1 and q_out.stride(1) == d):
+        _fail("q_out heads must be contiguous")
     for x in (q_out, qkv, *norms):
-        _check(x.dtype == (qkv.dtype if fp8 else k_cache.dtype),
-               "qkv / q_out / norm weights must have one dtype (the cache dtype of a 2-byte pool)")
-    _check(all(w.numel() == d and w.is_contiguous() for w in norms),
-           "norm weights must be contiguous [head_dim]")
+        if not (x.dtype == (qkv.dtype if fp8 else k_cache.dtype)):
+            _fail("qkv / q_out / norm weights must have one dtype (the cache dtype of a 2-byte pool)")
+    if not (all(w.numel() == d and w.is_contiguous() for w in norms)):
+        _fail("norm weights must be contiguous [head_dim]")
     qw = q_norm_weight.data_ptr() if norms else None
     kw = k_norm_weight.data_ptr() if norms else None
-    _check(inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
-           and inv_freq.is_contiguous(), "inv_freq must be contiguous float32 [head_dim / 2]")
+    if not (inv_freq.dtype == torch.float32 and inv_freq.numel() == d // 2
+            and inv_freq.is_contiguous()):
+        _fail("inv_freq must be contiguous float32 [head_dim / 2]")
     for x, nm in ((slot_mapping, "slot_mapping"), (positions, "positions")):
-        _check(x.dim() == 1 and x.numel() >= t and x.is_contiguous(),
-               f"{nm} must be a contiguous [num_tokens] tensor")
+        if not (x.dim() == 1 and x.numel() >= t and x.is_contiguous()):
+            _fail(f"{nm} must be a contiguous [num_tokens] tensor")
     code = _dtype_code(qkv if fp8 else k_cache, "qk_norm_rope_store")
     if t == 0:
         return
