@@ -10,13 +10,15 @@
 // them before attending, model_runner.py:146). For an empty prefix both agree.
 //
 // MI355X design (gfx950, v_mfma_f32_32x32x16_{bf16,f16}, wave64):
-//   head dim D = 64 or 128 (prefill_kernel<.., D, ..>; the other multiples
-//   of 32 up to 256 run prefill_generic_kernel below);
-//   workgroup = 8 waves = one (sequence, kv-head, tile of 256 rows, key part).
+//   head dim D = 64, 128 or 256 (prefill_kernel<.., D, ..>; the other multiples
+//   of 32 up to 224 run prefill_generic_kernel below);
+//   workgroup = 8 waves = one (sequence, kv-head, tile of 256 rows, key part)
+//   -- 4 waves and 128 rows, without the half-step shift below, at head dim 256
+//   (32 keys per step, no key parts) and for few tiles at 128.
 //   Rows are (token, head) pairs of the kv head's G query heads, flattened as
 //   token * G + head: any G fills its tiles, and a wave's 32 rows span 32 / G
-//   tokens, so its causal range ends with the tile's. Two waves per SIMD, 256
-//   VGPRs each. All 8 waves read the 64-key K/V tiles that the workgroup
+//   tokens, so its causal range ends with the tile's. With 8
+//   waves, two share a SIMD, 256 VGPRs each. All 8 waves read the 64-key K/V tiles that the workgroup
 //   gathers from the pool into LDS (GQA and row reuse).
 //   per step of 64 keys, each wave:
 //     S^T = K . Q^T   -- A = K rows from LDS, B = the wave's query rows, kept
@@ -73,11 +75,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kWaves = 8;        // waves per workgroup: 2 per SIMD
-constexpr int kThreads = 64 * kWaves;
 constexpr int kWaveRows = 32;    // flattened (token, head) rows per wave
-constexpr int kTileRows = kWaves * kWaveRows;   // ... and per workgroup
+constexpr int tile_rows(int nw) { return nw * kWaveRows; }   // ... and per workgroup of nw waves
 constexpr int kKT = 64;          // keys per step
+// ... of prefill_kernel at head dim d: 32 at 256, so that its tiles (16 KB) and
+// accumulators fit
+constexpr int step_keys(int d) { return d == 256 ? 32 : kKT; }
 constexpr int kBufK = 4;         // K tiles in LDS
 constexpr int kBufV = 5;         // V tiles in LDS
 constexpr int kListBlocks = 2048;     // blocks of the key range listed in LDS at a time (8 KB)
@@ -87,7 +90,7 @@ constexpr int kWaitVm0 = 0x0f70;       // s_waitcnt vmcnt(0), the other counters
 constexpr float kNoRef = 3.402823466e38f;     // exponent offset of a row without a reference
 constexpr int kSplitSteps = 16;       // a key range longer than this many steps is split
 constexpr int kMaxSplits = 8;
-constexpr int kAhead = 4;            // operand reads ahead of their MFMA
+constexpr int kAhead = 4;             // LDS operand reads ahead of their MFMA
 constexpr int kSlots = 8;             // tiles per lane of the work list
 constexpr int kListTiles = 64 * kSlots;
 constexpr int kSmallDiv = 1 << 21;    // dividends small_div takes for any divisor
@@ -208,7 +211,7 @@ __device__ __forceinline__ int small_div(int x, int d) {
 }
 
 // The work item of this workgroup, derived by its first wave: the sequence s,
-// its tile t of kTileRows flattened (token, head) rows, key part j of nsp, kv
+// its tile t of TR flattened (token, head) rows, key part j of nsp, kv
 // head kh, the sequence's first query row, chunk length and context, the
 // tile's keys 0 .. nkeys - 1 and the part's steps st0 .. st1 - 1. false: no
 // item, the workgroup exits.
@@ -216,13 +219,15 @@ struct Item {
   int s, t, j, nsp, kh, q0, qlen, ctx, nkeys, st0, st1;
 };
 // one past the last position that tile t of a chunk sees
+template <int TR>
 __device__ __forceinline__ int tile_keys(const PrefillArgs& a, int t, int qlen, int ctx) {
-  const int fr = qlen * a.group, fe = (t + 1) * kTileRows;
+  const int fr = qlen * a.group, fe = (t + 1) * TR;
   const int last = fe >= fr ? qlen - 1   // position in the chunk of the tile's last row
                             : (fe < kSmallDiv ? small_div(fe - 1, a.group) : (fe - 1) / a.group);
   const int nk = ctx - qlen + last + 1;
   return nk < 0 ? 0 : nk;
 }
+template <int TR, int KT>
 __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Item& it) {
   int s, t, j, kh, nsp, nsteps, q0, qlen, ctx;
   const int cap = a.max_bps * a.block_size;
@@ -256,8 +261,8 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
         const int lt = 64 * k + lane - small_div(64 * k + lane, a.tiles_max) * a.tiles_max;
         ql[k] -= c0[k];
         cx[k] = cx[k] < 0 ? 0 : (cx[k] < cap ? cx[k] : cap);
-        valid[k] = valid[k] && lt * kTileRows < ql[k] * a.group;
-        if (valid[k]) n[k] = (tile_keys(a, lt, ql[k], cx[k]) + kKT - 1) / kKT;
+        valid[k] = valid[k] && lt * TR < ql[k] * a.group;
+        if (valid[k]) n[k] = (tile_keys<TR>(a, lt, ql[k], cx[k]) + KT - 1) / KT;
         tot += npd::wave_sum_i(n[k]);   // DPP, wave-uniform
         nmax = max(nmax, npd::wave_max_i(n[k]));
         ntiles += __popcll(__ballot(valid[k]));
@@ -370,10 +375,10 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
     s = v - j * a.num_seqs;
     q0 = a.cu_seqlens_q[s];
     qlen = a.cu_seqlens_q[s + 1] - q0;
-    if (t * kTileRows >= qlen * a.group) return false;
+    if (t * TR >= qlen * a.group) return false;
     ctx = a.context_lens[s];
     ctx = ctx < 0 ? 0 : (ctx < cap ? ctx : cap);
-    nsteps = (tile_keys(a, t, qlen, ctx) + kKT - 1) / kKT;
+    nsteps = (tile_keys<TR>(a, t, qlen, ctx) + KT - 1) / KT;
     nsp = (nsteps + a.ks_steps - 1) / a.ks_steps;
     nsp = nsp < 1 ? 1 : (nsp > a.splits_max ? a.splits_max : nsp);
     if (j >= nsp) return false;
@@ -381,7 +386,7 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
   // near-equal parts, the first nsteps % nsp one step longer
   const int base = small_div(nsteps, nsp), rem = nsteps - base * nsp;
   const int st0 = j * base + (j < rem ? j : rem);
-  it = Item{s, t, j, nsp, kh, q0, qlen, ctx, tile_keys(a, t, qlen, ctx), st0,
+  it = Item{s, t, j, nsp, kh, q0, qlen, ctx, tile_keys<TR>(a, t, qlen, ctx), st0,
             st0 + base + (j < rem ? 1 : 0)};
   return true;
 }
@@ -420,22 +425,26 @@ __device__ __forceinline__ void wait_and_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// NW: waves per workgroup, 8 (two per SIMD, 256 registers each) or 4 (one per
+// SIMD, up to 512: head dim 256 keeps O in accumulation registers).
 // kOff32: every K/V element of the pool lies within 4 GiB of the cache base,
 // so gather offsets are 32-bit. kF8: the pool holds OCP e4m3 bytes, converted
 // exactly to TT pairs on the way into LDS (through registers); the per-kv-head
 // scales go into the score scale and the output.
-template <class TT, int D, bool kOff32, bool kF8>
-__global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
-  static_assert(D == 64 || D == 128, "head dims of this kernel");
+template <class TT, int D, int NW, bool kOff32, bool kF8>
+__global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
+  static_assert(D == 64 || D == 128 || D == 256, "head dims of this kernel");
+  constexpr int KT = step_keys(D);                     // keys per step
+  constexpr int NT = 64 * NW;                          // threads
   constexpr int RB = 2 * D;                            // bytes of a tile row
-  constexpr int TB = kKT * RB;                         // bytes of a K or V tile
-  constexpr int NI = TB / (1024 * kWaves);             // 1 KB loads per wave and tile (D 128: 2)
+  constexpr int TB = KT * RB;                         // bytes of a K or V tile
+  constexpr int NI = TB / (1024 * NW);             // 1 KB loads per wave and tile (D 128: 2)
   constexpr int NC = D / 16;                           // head-dim chunks of QK
-  constexpr int NS = kKT / 32;                         // 32-key blocks of S
-  constexpr int KB = kKT / 16;                         // 16-key blocks of PV
+  constexpr int NS = KT / 32;                         // 32-key blocks of S
+  constexpr int KB = KT / 16;                         // 16-key blocks of PV
   constexpr int DB = D / 32;                           // 32-dim blocks of O
   constexpr int kRecO = rec_o(D);
-  static_assert(NI * 1024 * kWaves == TB, "tile shape");
+  static_assert(NI * 1024 * NW == TB, "tile shape");
   __shared__ __attribute__((aligned(1024))) char s_k[kBufK * TB];
   __shared__ __attribute__((aligned(1024))) char s_v[kBufV * TB];
   __shared__ int s_row[kListBlocks];   // first K/V row of each block of the key range
@@ -451,7 +460,7 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   if (wave == 0) {
     Item it{};
     it.nsp = 0;
-    prefill_item(a, lane, it);
+    prefill_item<tile_rows(NW), KT>(a, lane, it);
     if (lane == 0) s_item = it;
   }
   __syncthreads();
@@ -466,7 +475,7 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   // this lane's one (clamped to the chunk's last; outputs past it are not stored)
   const int prefix = ctx - qlen;                       // position of the chunk's first token
   const int frows = qlen * G;
-  const int wsub = t * kWaves + wave;                  // 32-row subtile of the (sequence, kv head)
+  const int wsub = t * NW + wave;                  // 32-row subtile of the (sequence, kv head)
   const int f0 = wsub * kWaveRows;
   const bool row_ok = f0 + c32 < frows;
   const int f = row_ok ? f0 + c32 : frows - 1;
@@ -476,7 +485,7 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   const int wpos0 = __builtin_amdgcn_readfirstlane(pos);
   const int wpos1 = __builtin_amdgcn_readlane(pos, 31);   // the wave's first and last position
   const int bs = a.block_size;
-  const int kend = st1 * kKT < nkeys ? st1 * kKT : nkeys;
+  const int kend = st1 * KT < nkeys ? st1 * KT : nkeys;
 
   uint16_t* op = a.out + (int64_t)(q0 + tok) * a.out_stride_token + (int64_t)h * a.out_stride_head;
   if (st0 >= st1) {
@@ -504,14 +513,14 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   // removes (only keys past the tile's last position are clamped).
   constexpr int F8B = D == 64 ? 8 : 16;
   constexpr int LROW = kF8 ? D / F8B : RB / 16;        // lanes per row
-  constexpr int NR = kF8 ? kKT * D / (kThreads * F8B) : NI;
-  static_assert(!kF8 || NR * kThreads * F8B == kKT * D, "FP8 tile shape");
+  constexpr int NR = kF8 ? KT * D / (NT * F8B) : NI;
+  static_assert(!kF8 || NR * NT * F8B == KT * D, "FP8 tile shape");
   int lrow[NR], lcol[NR];   // tile row and source column (bytes) of this lane's loads
 #pragma unroll
   for (int e = 0; e < NR; ++e) {
     if (kF8) {
-      lrow[e] = (tid + kThreads * e) / LROW;
-      lcol[e] = (tid + kThreads * e) % LROW * F8B;
+      lrow[e] = (tid + NT * e) / LROW;
+      lcol[e] = (tid + NT * e) % LROW * F8B;
     } else {
       const int o = (wave * NI + e) * 1024 + lane * 16;
       lrow[e] = o / RB;
@@ -521,7 +530,7 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   int blk0 = 0;   // first block of the list in s_row
   // pool row of tile row lrow[e] of step `step` (< 2^31, host check)
   auto pool_row = [&](int step, int e) {
-    int tk = step * kKT + lrow[e];
+    int tk = step * KT + lrow[e];
     tk = tk < kend ? tk : kend - 1;
     const int lb = a.bs_shift >= 0 ? tk >> a.bs_shift : tk / bs;
     return s_row[lb - blk0] + (tk - (a.bs_shift >= 0 ? lb << a.bs_shift : lb * bs));
@@ -608,8 +617,8 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
     }
   };
   auto softmax = [&](int step, f32x16 (&sacc)[NS], u32x4 (&pb)[KB]) {
-    const int key0 = step * kKT;
-    if (__builtin_expect(key0 + kKT - 1 > wpos0, 0)) {   // some key here is after some row
+    const int key0 = step * KT;
+    if (__builtin_expect(key0 + KT - 1 > wpos0, 0)) {   // some key here is after some row
       const int lim = pos - key0 - 4 * hf;
 #pragma unroll
       for (int n = 0; n < NS; ++n)
@@ -704,18 +713,18 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
   // has landed when its softmax(i) is done (interval 2i + 1 or 2i + 2), so the
   // whole tile has when a wave reads its first K operands ahead of step i + 2,
   // at the end of interval 2i + 3 or 2i + 4.
-  const bool late = wave >= kWaves / 2;
-  const int list_steps = (int)((int64_t)(kListBlocks - 2) * bs / kKT);   // steps the list covers
+  const bool late = NW == 8 && wave >= NW / 2;
+  const int list_steps = (int)((int64_t)(kListBlocks - 2) * bs / KT);   // steps the list covers
   const int seg = list_steps < 1 ? 1 : list_steps;
   for (int sb = st0; sb < st1; sb += seg) {
     const int n = (sb + seg < st1 ? sb + seg : st1) - sb;
     // first rows of the blocks of this segment's keys (ids clamped into the pool)
     auto div_bs = [&](int x) { return a.bs_shift >= 0 ? x >> a.bs_shift : x / bs; };
-    blk0 = div_bs(sb * kKT);
-    const int ke = (sb + n) * kKT < kend ? (sb + n) * kKT : kend;
+    blk0 = div_bs(sb * KT);
+    const int ke = (sb + n) * KT < kend ? (sb + n) * KT : kend;
     const int nblk = div_bs(ke - 1) + 1 - blk0;
     if (sb != st0) __syncthreads();   // the last segment's reads are done
-    for (int e = tid; e < nblk; e += kThreads) {
+    for (int e = tid; e < nblk; e += NT) {
       int bid = a.block_tables[(int64_t)s * a.max_bps + blk0 + e];
       bid = bid < 0 ? 0 : (bid >= a.num_blocks ? a.num_blocks - 1 : bid);
       s_row[e] = (bid * a.num_kv_heads + kh) * bs;
@@ -729,11 +738,11 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
     u32x4 pb[KB];
 #pragma unroll
     for (int e = 0; e < KB; ++e) pb[e] = u32x4{0, 0, 0, 0};
-    for (int e = tid; e < TB / 16; e += kThreads)
+    for (int e = tid; e < TB / 16; e += NT)
       *reinterpret_cast<u32x4*>(s_v + (kBufV - 1) * TB + e * 16) = u32x4{0, 0, 0, 0};
     // steps in which some row of this wave sees a key (the causal mask only
     // ever ends a wave's steps): later ones it spends in the barriers
-    int nact = wpos1 < sb * kKT ? 0 : wpos1 / kKT - sb + 1;
+    int nact = wpos1 < sb * KT ? 0 : wpos1 / KT - sb + 1;
     nact = nact < n ? nact : n;
     Raw raw;   // FP8: the bytes of the tile stashed next
     if constexpr (kF8) {
@@ -868,9 +877,8 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
     }
 }
 
-// Every head dim but 64 and 128 (multiples of 32 from 32 to 256): at 256 the
-// tiles and register ring of prefill_kernel would need about 174 KB of LDS
-// and 336 VGPRs. One workgroup of 4 waves per
+// The head dims whose rows are not a power of two of 16-byte chunks (32, 96,
+// 160, 192, 224). One workgroup of 4 waves per
 // (sequence, query head, 64-row query tile); wave w owns query rows
 // 16w .. 16w + 15 of the tile. Per step of 64 keys the workgroup copies the kv
 // head's K and V rows into LDS (keys past the visible range clamped to the
@@ -883,8 +891,8 @@ __global__ __launch_bounds__(kThreads) void prefill_kernel(PrefillArgs a) {
 //                      the transposing LDS read, P^T from the S^T layout).
 // The operand layouts, the P packing and the normalisation (the row sum adds
 // the rounded P values) are those of prefill_kernel. The next step's K/V
-// chunks load into registers during the step (two workgroups per CU at 254
-// VGPRs); the workgroups of one (sequence, kv head) share K/V through one
+// chunks load into registers during the step (two workgroups per CU, at most
+// 246 VGPRs); the workgroups of one (sequence, kv head) share K/V through one
 // XCD's L2 rather than one LDS tile, and there are no key splits. Rows with no
 // visible key are written as zeros.
 template <class TT, int D, bool kF8>
@@ -895,7 +903,7 @@ __global__ __launch_bounds__(256, 2) void prefill_generic_kernel(PrefillArgs a) 
   constexpr int NPASS = kKT * CPR / kGT;        // chunks of the 64-key tile per thread
   constexpr int NC = D / 32;                    // head-dim chunks of QK
   constexpr int NB = D / 16;                    // 16-dim blocks of O
-  static_assert(D % 32 == 0 && D >= 32 && D <= 256, "head dims of this kernel");
+  static_assert(D % 32 == 0 && D >= 32 && D < 256, "head dims of this kernel");
   static_assert(NPASS * kGT == kKT * CPR && RW % 8 == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint16_t s_k[kKT * RW];
   __shared__ __attribute__((aligned(16))) uint16_t s_v[kKT * RW];
@@ -1092,30 +1100,32 @@ int launch_generic(int64_t head_dim, const PrefillArgs& a, int64_t grid, hipStre
     case 160: hipLaunchKernelGGL((prefill_generic_kernel<TT, 160, kF8>), g, b, 0, st, a); break;
     case 192: hipLaunchKernelGGL((prefill_generic_kernel<TT, 192, kF8>), g, b, 0, st, a); break;
     case 224: hipLaunchKernelGGL((prefill_generic_kernel<TT, 224, kF8>), g, b, 0, st, a); break;
-    case 256: hipLaunchKernelGGL((prefill_generic_kernel<TT, 256, kF8>), g, b, 0, st, a); break;
     default: return npd::fail(NPD_E_INVALID, "%s: head_dim %lld", name, (long long)head_dim);
   }
   return npd::check_launch(name);
 }
 
+template <class TT, int D, int NW, bool kF8>
+void launch_d(bool off32, const PrefillArgs& a, int64_t grid, hipStream_t st) {
+  const dim3 g((unsigned)grid), b(64 * NW);
+  if (off32) hipLaunchKernelGGL((prefill_kernel<TT, D, NW, true, kF8>), g, b, 0, st, a);
+  else hipLaunchKernelGGL((prefill_kernel<TT, D, NW, false, kF8>), g, b, 0, st, a);
+}
+
 template <class TT, bool kF8>
-int launch_dt(int64_t head_dim, bool off32, const PrefillArgs& a, int64_t grid, hipStream_t st,
-              const char* name) {
-  const dim3 g((unsigned)grid), b(kThreads);
-  if (head_dim == 64) {
-    if (off32) hipLaunchKernelGGL((prefill_kernel<TT, 64, true, kF8>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((prefill_kernel<TT, 64, false, kF8>), g, b, 0, st, a);
-  } else {
-    if (off32) hipLaunchKernelGGL((prefill_kernel<TT, 128, true, kF8>), g, b, 0, st, a);
-    else hipLaunchKernelGGL((prefill_kernel<TT, 128, false, kF8>), g, b, 0, st, a);
-  }
+int launch_dt(int64_t head_dim, int waves, bool off32, const PrefillArgs& a, int64_t grid,
+              hipStream_t st, const char* name) {
+  if (head_dim == 256) launch_d<TT, 256, 4, kF8>(off32, a, grid, st);
+  else if (head_dim == 64) launch_d<TT, 64, 8, kF8>(off32, a, grid, st);
+  else if (waves == 8) launch_d<TT, 128, 8, kF8>(off32, a, grid, st);
+  else launch_d<TT, 128, 4, kF8>(off32, a, grid, st);
   return npd::check_launch(name);
 }
 
 // Workspace: [counter region (kCounterBytes) | O partials | (m, l) partials].
 // Sized for the most records any group size can address: a (sequence, kv head)
 // of G heads has 8 * ceil(max_q_len * G / 256) <= G * (ceil(max_q_len / 32) + 7)
-// subtiles of 32 flattened rows.
+// subtiles of 32 flattened rows (no more with 4-wave tiles).
 struct Layout {
   int splits, ks_steps;
   int64_t o_off, ml_off, total;
@@ -1151,7 +1161,7 @@ extern "C" int64_t npd_paged_prefill_workspace_size(int64_t num_seqs, int64_t to
                                                     int64_t num_heads, int64_t head_dim,
                                                     int64_t max_q_len, int64_t max_context_len) {
   (void)total_q;
-  // head dims other than 64 and 128 (prefill_generic_kernel) need no workspace
+  // head dims other than 64 and 128 are not cut and need no workspace
   if (head_dim != 64 && head_dim != 128) return 0;
   return prefill_layout(num_seqs, num_heads, head_dim, max_q_len, max_context_len).total;
 }
@@ -1179,16 +1189,16 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   if (head_dim < 32 || head_dim > 256 || head_dim % 32 != 0)
     return fail(NPD_E_INVALID, "%s: head_dim %lld is not a multiple of 32 in [32, 256]", name,
                 (long long)head_dim);
-  // head dims 64 and 128: prefill_kernel (key splits, shared K/V tiles);
-  // every other one: prefill_generic_kernel
-  const bool generic = head_dim != 64 && head_dim != 128;
+  // head dims 64, 128 and 256: prefill_kernel (256 without key splits: its
+  // callers bring no workspace); every other one: prefill_generic_kernel
+  const bool generic = head_dim != 64 && head_dim != 128 && head_dim != 256;
   if (num_heads % num_kv_heads != 0)
     return fail(NPD_E_INVALID, "%s: num_heads %lld is not a multiple of num_kv_heads %lld", name,
                 (long long)num_heads, (long long)num_kv_heads);
   const int64_t g = num_heads / num_kv_heads;
   if (num_blocks * block_size * num_kv_heads > INT32_MAX || max_blocks_per_seq * block_size > INT32_MAX)
     return fail(NPD_E_INVALID, "%s: pool exceeds int32 row indexing", name);
-  if (!generic && max_blocks_per_seq > kMaxTableBlocks)
+  if ((head_dim == 64 || head_dim == 128) && max_blocks_per_seq > kMaxTableBlocks)
     return fail(NPD_E_INVALID, "%s: block tables wider than %d blocks are not supported", name,
                 kMaxTableBlocks);
   if (q_stride_token % 8 || q_stride_head % 8 || out_stride_token % 4 || out_stride_head % 4 ||
@@ -1241,7 +1251,8 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
     return fp8 ? launch_generic<F16, true>(head_dim, a, grid, st, name)
                : launch_generic<F16, false>(head_dim, a, grid, st, name);
   }
-  const Layout L = prefill_layout(num_seqs, num_heads, head_dim, max_q_len, max_context_len);
+  const Layout L = head_dim == 256 ? Layout{1, 1 << 30, 0, 0, 0}
+                                   : prefill_layout(num_seqs, num_heads, head_dim, max_q_len, max_context_len);
   if (L.total > 0) {
     if (!workspace || workspace_bytes < L.total)
       return fail(NPD_E_WORKSPACE, "%s: workspace of %lld bytes needed, %lld given", name,
@@ -1249,9 +1260,24 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
       return fail(NPD_E_ALIGN, "%s: workspace must be 256-byte aligned", name);
   }
-  if (max_q_len * g > INT32_MAX - kTileRows)
+  if (max_q_len * g > INT32_MAX - 256)
     return fail(NPD_E_INVALID, "%s: too many query rows", name);
-  const int64_t tiles = (max_q_len * g + kTileRows - 1) / kTileRows;
+  // most tiles of tr rows there can be (a chunk's last one may be part full)
+  auto tiles_of = [&](int64_t tr) {
+    const int64_t by_max = num_seqs * ((max_q_len * g + tr - 1) / tr), by_rows = total_q * g / tr + num_seqs;
+    return by_max < by_rows ? by_max : by_rows;
+  };
+  // Tiles of 256 rows (8 waves, two per SIMD: one's softmax under the other's
+  // MFMAs), or of 128 (4 waves): at head dim 256, whose accumulators and
+  // queries need more than the 256 registers of two waves per SIMD (4 / 8
+  // waves: two chunks of 4096 tokens 425 / 463 us, 500 tokens 35 / 64 us), and
+  // at 128 where the 256-row tiles take half the compute units at most (500
+  // tokens of 32 / 8 heads 23.4 / 25.9 us, 64 on a prefix of 6000 43.0 / 50.8).
+  // Head dim 64 gains nothing from it (17.9 / 18.1 us).
+  const bool few = tiles_of(tile_rows(8)) * num_kv_heads * 2 <= device_cus();
+  const int waves = head_dim == 256 || (head_dim == 128 && few) ? 4 : 8;
+  const int64_t tr = tile_rows(waves);
+  const int64_t tiles = (max_q_len * g + tr - 1) / tr;
   if (L.total > 0 && num_seqs * tiles * num_kv_heads > kMaxCounters)
     return fail(NPD_E_INVALID, "%s: too many query tiles for the %lld merge counters", name,
                 (long long)kMaxCounters);
@@ -1259,13 +1285,11 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   // work it finds. More run whole, in a fixed order, unless they leave compute
   // units idle (many short chunks on long prefixes).
   const bool list = num_seqs * tiles <= kListTiles;
-  const bool whole = !list && total_q * num_heads >= 2LL * device_cus() * kTileRows;
+  const bool whole = !list && total_q * num_heads >= 2LL * device_cus() * tr;
   const int splits = whole ? 1 : L.splits;
-  // Grid: the tiles there can be (a chunk's last tile may be part full), or
-  // two rounds of the compute units where the kernel may cut that many parts;
+  // Grid: the tiles there can be, or two rounds of the compute units where the kernel may cut that many parts;
   // a workgroup without an item ends after the work list.
-  const int64_t whole_tiles = num_seqs * tiles < total_q * g / kTileRows + num_seqs
-                                  ? num_seqs * tiles : total_q * g / kTileRows + num_seqs;
+  const int64_t whole_tiles = tiles_of(tr);
   const int64_t two_rounds = (2LL * device_cus() + num_kv_heads - 1) / num_kv_heads;
   const int64_t max_items = !list ? splits * num_seqs * tiles
                             : splits > 1 && whole_tiles < two_rounds ? two_rounds : whole_tiles;
@@ -1294,7 +1318,7 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   a.num_blocks = (int)num_blocks;
   a.max_bps = (int)max_blocks_per_seq;
   a.tiles_max = (int)tiles;
-  a.subtiles = (int)(tiles * kWaves);
+  a.subtiles = (int)(tiles * waves);
   a.splits_max = splits;
   a.ks_steps = L.ks_steps;
   a.max_items = (int)max_items;
@@ -1308,10 +1332,10 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   const int64_t elt = fp8 ? 1 : 2;
   const bool off32 = num_blocks * num_kv_heads * block_size * head_dim * elt <= (int64_t)UINT32_MAX;
   if (dtype == NPD_DTYPE_BF16)
-    return fp8 ? launch_dt<BF16, true>(head_dim, off32, a, grid, st, name)
-               : launch_dt<BF16, false>(head_dim, off32, a, grid, st, name);
-  return fp8 ? launch_dt<F16, true>(head_dim, off32, a, grid, st, name)
-             : launch_dt<F16, false>(head_dim, off32, a, grid, st, name);
+    return fp8 ? launch_dt<BF16, true>(head_dim, waves, off32, a, grid, st, name)
+               : launch_dt<BF16, false>(head_dim, waves, off32, a, grid, st, name);
+  return fp8 ? launch_dt<F16, true>(head_dim, waves, off32, a, grid, st, name)
+             : launch_dt<F16, false>(head_dim, waves, off32, a, grid, st, name);
 }
 
 }  // namespace

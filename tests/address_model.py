@@ -86,7 +86,6 @@ def ring_of(D: int, G: int = 1, fp8: bool = False) -> int:
 KT = 64
 SPLIT_STEPS = 16
 MAX_SPLITS = 8
-TILE_ROWS = 256        # kTileRows: flattened (token, head) rows per workgroup
 LIST_TILES = 512       # kListTiles: tiles the in-kernel work list orders
 LIST_BLOCKS = 2048     # kListBlocks: blocks listed in LDS at a time
 MIN_PART, ITEM_STEPS, MERGE_STEPS = 4, 4, 4
@@ -567,17 +566,30 @@ class PrefillLaunch:
     max_items: int = 0
     subtiles: int = 0
     num_cus: int = 256
+    waves: int = 8       # per workgroup
+    kt: int = KT         # keys per step
+
+    @property
+    def rows(self) -> int:
+        return self.waves * WAVE_ROWS
 
 
 def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
-                 D: int = 128, total_q: int | None = None) -> PrefillLaunch:
-    """prefill_layout and prefill_impl (prefill_attention.hip), head dims 64
-    and 128 (prefill_kernel). total_q: S * max_q_len unless given."""
-    assert D in (64, 128)
-    L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus)
+                 D: int = 128, total_q: int | None = None, waves: int = 8) -> PrefillLaunch:
+    """prefill_layout and prefill_impl (prefill_attention.hip), head dims 64,
+    128 and 256 (prefill_kernel). total_q: S * max_q_len unless given; waves:
+    per workgroup, 8, or 4 (head dim 256, and 128 where 256-row tiles take half
+    the compute units at most)."""
+    assert D in (64, 128, 256)
+    if D == 256:
+        waves = 4
+    L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus, waves=waves,
+                      kt=32 if D == 256 else KT)
     g = H // KV
     tq = S * max_q_len if total_q is None else total_q
-    if max_ctx > 0:
+    if D == 256:
+        L.ks_steps = 1 << 30   # whole key ranges
+    elif max_ctx > 0:
         steps = _ceil(max_ctx, KT)
         ks = max(_ceil(steps, MAX_SPLITS), SPLIT_STEPS)
         L.ks_steps = ks
@@ -591,12 +603,12 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
         L.ml_off = L.o_off + nrec * rec_o(D) * 4
         L.total = L.ml_off + nrec * REC_ML * 4
     L.rt = 4 // g
-    L.tiles = _ceil(max_q_len * g, TILE_ROWS)
-    L.subtiles = L.tiles * 8
+    L.tiles = _ceil(max_q_len * g, L.rows)
+    L.subtiles = L.tiles * L.waves
     in_list = S * L.tiles <= LIST_TILES
-    if not in_list and tq * H >= 2 * num_cus * TILE_ROWS:
+    if not in_list and tq * H >= 2 * num_cus * L.rows:
         L.splits = 1
-    whole = min(S * L.tiles, tq * g // TILE_ROWS + S)
+    whole = min(S * L.tiles, tq * g // L.rows + S)
     two = _ceil(2 * num_cus, KV)
     if not in_list:
         L.max_items = L.splits * S * L.tiles
@@ -606,9 +618,9 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
     return L
 
 
-def tile_keys(G: int, t: int, qlen: int, ctx: int) -> int:
+def tile_keys(L: PrefillLaunch, G: int, t: int, qlen: int, ctx: int) -> int:
     """Keys that tile t of a chunk sees."""
-    last = min((t + 1) * TILE_ROWS, qlen * G) - 1
+    last = min((t + 1) * L.rows, qlen * G) - 1
     return max(ctx - qlen + last // G + 1, 0)
 
 
@@ -626,9 +638,9 @@ def prefill_items(L: PrefillLaunch, cu: np.ndarray, ctx_lens: np.ndarray):
                for s in range(L.S)]
         for i in range(tiles):
             c0, ql, cx = seq[i // L.tiles]
-            valid[i] = (i % L.tiles) * TILE_ROWS < ql * G
+            valid[i] = (i % L.tiles) * L.rows < ql * G
             if valid[i]:
-                n[i] = _ceil(tile_keys(G, i % L.tiles, ql, cx), KT)
+                n[i] = _ceil(tile_keys(L, G, i % L.tiles, ql, cx), L.kt)
         tot, nmax, ntiles = int(n.sum()), int(n.max(initial=0)), int(valid.sum())
 
         def cut_of(step):
@@ -680,7 +692,7 @@ def prefill_items(L: PrefillLaunch, cu: np.ndarray, ctx_lens: np.ndarray):
         j, s = divmod(v, L.S)
         q0 = int(cu[s])
         qlen = int(cu[s + 1]) - q0
-        if t * TILE_ROWS >= qlen * G:
+        if t * L.rows >= qlen * G:
             continue
         ctx = min(max(int(ctx_lens[s]), 0), cap)
         items.append((s, t, j, kh, 0, q0, qlen, ctx, L.ks_steps, True))
@@ -696,24 +708,24 @@ def prefill(W: Writes, L: PrefillLaunch, out: Buf, ws: Buf, cu: np.ndarray, ctx_
             continue
         s, t, j, kh, _, q0, qlen, ctx, ks, _ = it
         W.index([s], L.S, "prefill sequence")
-        nkeys = tile_keys(G, t, qlen, ctx)
-        nsteps = _ceil(nkeys, KT)
+        nkeys = tile_keys(L, G, t, qlen, ctx)
+        nsteps = _ceil(nkeys, L.kt)
         nsp = min(max(_ceil(nsteps, ks), 1), L.splits)
         if j >= nsp:
             continue
         base, rm = divmod(nsteps, nsp)   # near-equal parts
         st0 = j * base + min(j, rm)
         st1 = st0 + base + (1 if j < rm else 0)
-        kend = min(st1 * KT, nkeys)
-        seg = max((LIST_BLOCKS - 2) * L.bs // KT, 1)   # steps whose blocks the list holds
+        kend = min(st1 * L.kt, nkeys)
+        seg = max((LIST_BLOCKS - 2) * L.bs // L.kt, 1)   # steps whose blocks the list holds
         for sb in range(st0, st1, seg):
             se = min(sb + seg, st1)
-            blk0 = sb * KT // L.bs
-            nblk = (min(se * KT, kend) - 1) // L.bs + 1 - blk0
+            blk0 = sb * L.kt // L.bs
+            nblk = (min(se * L.kt, kend) - 1) // L.bs + 1 - blk0
             W.index([nblk - 1], LIST_BLOCKS, "prefill block list in LDS")
             W.index([blk0 + nblk - 1], L.max_bps, "prefill block-table column")
-        for wave in range(8):
-            wsub = t * 8 + wave
+        for wave in range(L.waves):
+            wsub = t * L.waves + wave
             f = np.arange(WAVE_ROWS) + wsub * WAVE_ROWS
             f = f[f < qlen * G]
             lo = ((q0 + f // G) * out_stride_token + (kh * G + f % G) * out_stride_head) * 2

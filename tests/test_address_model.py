@@ -449,3 +449,32 @@ def test_bench_names_the_kernel_the_library_runs():
             for bs in (8, 16, 24, 32, 48, 64, 128, 256):
                 w = SimpleNamespace(num_seqs=S, head_dim=D, block_size=bs)
                 assert bench.fast_path(w) == A.use_fast_path(D, bs, S), (S, D, bs)
+
+
+@pytest.mark.parametrize("hd,waves", [(128, 8), (128, 4), (64, 8), (256, 4)])
+def test_prefill_tiles_of_flattened_rows(hd, waves):
+    """Both workgroup sizes and the three head dims: every store inside the
+    output and the workspace the library sizes, every (token, head) row written
+    by exactly one tile, groups that do not divide a tile, one to more than 512
+    tiles, and block lists longer than LDS holds."""
+    rng = np.random.default_rng(hd + waves)
+    for S, h, kv, mq, px, bs in ((1, 7, 1, 1, 0, 16), (3, 12, 2, 130, 900, 16), (2, 5, 5, 300, 9000, 1),
+                                 (40, 8, 2, 700, 50, 32), (600, 3, 1, 40, 1500, 16)):
+        q = rng.integers(1, mq, S, endpoint=True)
+        ctx = q + rng.integers(0, px, S, endpoint=True)
+        cu = np.concatenate([[0], np.cumsum(q)])
+        mb = int(-(-ctx.max() // bs))
+        T, g = int(cu[-1]), h // kv
+        L = A.prefill_host(S, h, kv, bs, mb, int(q.max()), int(ctx.max()), D=hd, total_q=T,
+                           waves=waves)
+        ws = int(_lib.load().npd_paged_prefill_workspace_size(S, T, h, hd, int(q.max()),
+                                                              int(ctx.max())))
+        assert L.total <= ws
+        W = A.Writes()
+        A.prefill(W, L, A.Buf("out", T * h * hd * 2), A.Buf("ws", ws), cu, ctx, h * hd, hd, D=hd)
+        W.check()
+        tiles = [it[:4] for it in A.prefill_items(L, cu, ctx)]
+        assert len(set(tiles)) == len(tiles)
+        rows = {(s, t, kh) for s, t, _, kh in tiles}
+        assert rows == {(s, t, kh) for s in range(S) for kh in range(kv)
+                        for t in range(-(-int(q[s]) * g // L.rows))}
