@@ -398,6 +398,24 @@ int npd_pack_metadata(const int32_t* seq_desc, const int32_t* flat_tables,
                       int32_t* slot_mapping, int32_t* token_seq,
                       void* stream);
 
+/*
+ * Residual add + RMSNorm of a decoder layer: with delta (null: none) x becomes
+ * x + delta, rounded to the dtype and stored back; then
+ * out = x * rsqrt(mean(x^2) + eps) * weight per row, fp32 inside, rounded once.
+ * All [rows, width] contiguous (weight [width]), 16-byte aligned, width a
+ * multiple of 8 up to 8192. out must not overlap x or delta.
+ */
+int npd_add_rms_norm(void* out, void* x, const void* delta, const void* weight, int64_t rows,
+                     int64_t width, float eps, int32_t dtype, void* stream);
+
+/*
+ * SwiGLU product: out[rows, width] = silu(gate) * up for gate_up rows
+ * [gate (width) | up (width)], silu rounded to the dtype before the product.
+ * Contiguous, 16-byte aligned, width a multiple of 8.
+ */
+int npd_silu_mul(void* out, const void* gate_up, int64_t rows, int64_t width, int32_t dtype,
+                 void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -57,6 +57,8 @@ SIGNATURES = {
     "npd_qk_norm_rope_store_fp8": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                                                   _I64, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                                                   _F, _I32, _P]),
+    "npd_add_rms_norm": (ctypes.c_int, [_P, _P, _P, _P, _I64, _I64, _F, _I32, _P]),
+    "npd_silu_mul": (ctypes.c_int, [_P, _P, _I64, _I64, _I32, _P]),
     "npd_pack_metadata": (ctypes.c_int, [_P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P,
                                          _P, _P]),
 }

@@ -693,6 +693,42 @@ def qk_norm_rope_store(q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
               qkv.stride(0), q_out.stride(0), float(eps), code, _stream(dev))
 
 
+def _rows_16(*ts: torch.Tensor) -> bool:
+    """Contiguous 2-byte tensors that start on 16 bytes, with whole 16-byte rows."""
+    return all(t.is_cuda and t.dtype in _DTYPES and t.dtype == ts[0].dtype and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts)
+
+
+def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tensor,
+                 eps: float) -> torch.Tensor:
+    """RMSNorm over the last dim of x + delta, which is left in ``x`` (delta
+    None: of x). The sum is rounded to the dtype, the norm once after fp32.
+    2-byte CUDA tensors of up to 8192 columns run as one launch, others as the
+    torch operations."""
+    if (x.dim() == 2 and x.size(1) <= 8192 and _rows_16(x, weight)
+            and (delta is None or (delta.shape == x.shape and _rows_16(x, delta)))):
+        out = torch.empty_like(x)
+        _lib.call("npd_add_rms_norm", out.data_ptr(), x.data_ptr(),
+                  None if delta is None else delta.data_ptr(), weight.data_ptr(), x.size(0),
+                  x.size(1), float(eps), _DTYPES[x.dtype], _stream(x.device))
+        return out
+    if delta is not None:
+        x += delta
+    return torch.nn.functional.rms_norm(x, (x.size(-1),), weight, eps)
+
+
+def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of rows [gate | up] (one launch for 2-byte CUDA tensors,
+    the torch operations otherwise)."""
+    n = gate_up.size(-1) // 2
+    if gate_up.dim() == 2 and n % 8 == 0 and _rows_16(gate_up):
+        out = torch.empty(gate_up.size(0), n, dtype=gate_up.dtype, device=gate_up.device)
+        _lib.call("npd_silu_mul", out.data_ptr(), gate_up.data_ptr(), gate_up.size(0), n,
+                  _DTYPES[gate_up.dtype], _stream(gate_up.device))
+        return out
+    return torch.nn.functional.silu(gate_up[:, :n]) * gate_up[:, n:]
+
+
 class BatchMetadata(NamedTuple):
     cu_seqlens_q: torch.Tensor   # int32 [S + 1]
     seq_lens: torch.Tensor       # int32 [S], context after the step

@@ -239,16 +239,20 @@ class PagedQwen3:
         x = F.embedding(b.input_ids, self.embed)
         q = torch.empty(T, H, D, dtype=self.dtype, device=self.device)
         attn = torch.empty(T, H, D, dtype=self.dtype, device=self.device)
+        h = pk.add_rms_norm(x, None, self.layers[0]["in_norm"], cfg.rms_eps)
         for li, w in enumerate(self.layers):
-            h = F.rms_norm(x, (E,), w["in_norm"], cfg.rms_eps)
             qkv = F.linear(h, w["qkv"], w["qkv_bias"])
             self._prologue(li, w, qkv, q, b, rope)
             kc, vc = self.k_cache[li], self.v_cache[li]
             self.attention(li, q, kc, vc, b, attn)
-            x = x + attn.view(T, H * D) @ w["o"].t()
-            h = F.rms_norm(x, (E,), w["post_norm"], cfg.rms_eps)
-            gu = h @ w["gate_up"].t()
-            x = x + (F.silu(gu[:, : cfg.intermediate]) * gu[:, cfg.intermediate:]) @ w["down"].t()
+            # each residual add joins the norm that follows it (x stays the
+            # residual stream); the last one has the sampled rows' norm after it
+            h = pk.add_rms_norm(x, attn.view(T, H * D) @ w["o"].t(), w["post_norm"], cfg.rms_eps)
+            down = pk.silu_mul(h @ w["gate_up"].t()) @ w["down"].t()
+            if li + 1 < cfg.num_layers:
+                h = pk.add_rms_norm(x, down, self.layers[li + 1]["in_norm"], cfg.rms_eps)
+            else:
+                x = x + down
         if b.sample_rows is not None:
             x = x.index_select(0, b.sample_rows)
         xs = F.rms_norm(x, (E,), self.final_norm, cfg.rms_eps)
