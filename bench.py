@@ -326,7 +326,7 @@ def bench_prefill(args, w) -> dict:
             "prefill_flops": flops,
             "prefill_tokens": tp,
             "decode_seqs": len(w.chunk_lens) - npf,
-            "kernels": "prefill_kernel (MFMA 16x16x32) + kv_store_kernel + decode_fast_kernel",
+            "kernels": "prefill_kernel (MFMA 32x32x16) + kv_store_kernel + decode_fast_kernel",
         },
     }
 

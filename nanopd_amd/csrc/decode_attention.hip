@@ -269,8 +269,15 @@ __device__ __forceinline__ void partition_butterfly(float (&v)[NV], int j) {
 // chunks (D at run time, a multiple of 8 from 32 to 256); lanes j >= CPR of a
 // row hold a zero query and load its last chunk (an address inside the row),
 // so they add nothing to the dot products and store nothing.
-template <class TT, int LPT, int G>
-__global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
+// W: waves of a partition, 1 or 4. Four take a run of its steps each, on their
+// own, and their O rows and (m, l) meet in LDS: that cuts the chain of a launch
+// that does not fill the chip, and of the register-heavy shapes that leave few
+// waves resident (launch_partitions). Merging a unit's partitions in this
+// kernel, by its last one to arrive, was slower than the second launch (64
+// sequences at D 96 120 against 113 us, four of 8k-30k tokens 149 against 131):
+// the partials then go through the device-coherent level.
+template <class TT, int LPT, int G, int W>
+__global__ __launch_bounds__(64 * W) void decode_partition_kernel(DecodeArgs a) {
   static_assert(LPT == 4 || LPT == 8 || LPT == 16 || LPT == 32, "lanes per token row");
   constexpr int TPL = 64 / LPT;          // tokens per load
   constexpr int NL = kStep / TPL;        // loads per step
@@ -281,11 +288,16 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
   constexpr int HELD = NV >> NH;                 // values a lane keeps
   static_assert(TPL * NL == kStep, "step shape");
 
-  __shared__ float s_p[kMaxPartition * GP];      // scores, then probabilities
+  constexpr int WTOK = kMaxPartition / W;        // most tokens of a wave
+  __shared__ float s_pw[W][WTOK * GP];           // scores, then probabilities
   __shared__ int s_blk[kMaxPartition + 1];       // block ids of the partition
-  __shared__ float s_ml[2 * GP];                 // per-head max and sum
+  __shared__ float s_mlw[W][2 * GP];             // per-head max and sum of a wave's tokens
+  __shared__ float s_accw[W][W > 1 ? G * LPT * 8 : 1];   // ... and its O rows
 
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  float* s_p = s_pw[wave];
+  float* s_ml = s_mlw[wave];
   const int r = lane / LPT;   // token row within a load
   const int j = lane % LPT;   // 16-byte chunk of the head row
   const int cpr = a.head_dim / 8;          // chunks per head row
@@ -300,7 +312,7 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
   const int cap = a.max_bps * a.block_size;
   ctx = ctx < cap ? ctx : cap;
   if (ctx <= 0) {
-    if (part == 0 && lane < LPT && live) {
+    if (part == 0 && wave == 0 && lane < LPT && live) {
       const float z[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       for (int h = 0; h < G; ++h)
         store_row8<TT>(a.out + s * a.out_stride_seq + (kh * G + h) * a.out_stride_head + j * 8, z, 0.f);
@@ -309,16 +321,22 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
   }
   const int nparts = (ctx + a.partition - 1) / a.partition;
   if (part >= nparts) return;
-  const int t0 = part * a.partition;
-  const int ntok = (ctx - t0) < a.partition ? (ctx - t0) : a.partition;
-  const int nsteps = (ntok + kStep - 1) / kStep;
+  const int p0 = part * a.partition;
+  const int ptok = (ctx - p0) < a.partition ? (ctx - p0) : a.partition;
   const int bs = a.block_size;
-  const int b0 = t0 / bs;
-  const int nb = (t0 + ntok - 1) / bs - b0 + 1;
+  const int b0 = p0 / bs;
+  const int nb = (p0 + ptok - 1) / bs - b0 + 1;
+  // this wave's tokens: a run of whole steps, equal but for the last (none
+  // where the partition is short)
+  const int wsteps = ((ptok + kStep - 1) / kStep + W - 1) / W;
+  const int t0 = p0 + wave * wsteps * kStep;
+  int ntok = p0 + ptok - t0;
+  if (W > 1) ntok = ntok < 0 ? 0 : (ntok < wsteps * kStep ? ntok : wsteps * kStep);
+  const int nsteps = (ntok + kStep - 1) / kStep;
 
   // Block ids of this partition -> LDS, clamped into the pool.
   const int32_t* bt_row = a.block_tables + (int64_t)s * a.max_bps;
-  for (int e = lane; e < nb; e += 64) {
+  for (int e = threadIdx.x; e < nb; e += 64 * W) {
     int b = bt_row[b0 + e];
     b = b < 0 ? 0 : (b >= a.num_blocks ? a.num_blocks - 1 : b);
     s_blk[e] = b;
@@ -405,7 +423,8 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
 #pragma unroll
   for (int b = 0; b < R; ++b)
     if (b < nsteps) load_rows(a.v_cache, vb[b], b);
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the wave's own LDS scores
+  __builtin_amdgcn_wave_barrier();
 
   // ---------------- pass 2: softmax over the partition ----------------
   {
@@ -414,9 +433,12 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
     for (int idx = lane; idx < n; idx += 64) m = fmaxf(m, s_p[idx]);
 #pragma unroll
     for (int mask = GP; mask < 64; mask <<= 1) m = fmaxf(m, shfl_xor(m, mask));
+    // a wave whose tokens all score -inf (or that has none) keeps m = -inf: its
+    // probabilities are zeros, which the other waves' maxima outweigh
+    const float mr = W > 1 && m == -INFINITY ? 0.f : m;
     float l = 0.f;
     for (int idx = lane; idx < n; idx += 64) {
-      const float p = exp2f(s_p[idx] - m);
+      const float p = exp2f(s_p[idx] - mr);
       s_p[idx] = p;
       l += p;
     }
@@ -427,7 +449,8 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
       s_ml[GP + lane] = l;
     }
   }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 
   // ---------------- pass 3: probabilities x V ----------------
   // (units of more than 8 heads keep O only in the MFMA accumulators and
@@ -484,28 +507,76 @@ __global__ __launch_bounds__(64) void decode_partition_kernel(DecodeArgs a) {
 #pragma unroll
       for (int d = 0; d < 8; ++d) acc[h][d] += shfl_xor(acc[h][d], mask);
 
-  if (lane >= LPT || !live) return;
-  const int D = a.head_dim;
-  if (nparts == 1) {
+  if constexpr (W == 1) {
+    if (lane >= LPT || !live) return;
+    const int D = a.head_dim;
+    if (nparts == 1) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      const float l = s_ml[GP + h];
-      store_row8<TT>(a.out + s * a.out_stride_seq + (kh * G + h) * a.out_stride_head + j * 8,
-                     acc[h], 1.f / l);
+      for (int h = 0; h < G; ++h) {
+        const float l = s_ml[GP + h];
+        store_row8<TT>(a.out + s * a.out_stride_seq + (kh * G + h) * a.out_stride_head + j * 8,
+                       acc[h], 1.f / l);
+      }
+    } else {
+      const int64_t base = (int64_t)unit * a.max_parts + part;
+#pragma unroll
+      for (int h = 0; h < G; ++h) {
+        f32x4* dst = reinterpret_cast<f32x4*>(a.part_acc + ((base * G + h) * D + j * 8));
+        dst[0] = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+        dst[1] = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+      }
+      // (m, l) of every head: the row's live lanes take heads j, j + cpr, ...
+      // (cpr may be below G at small head dims)
+      for (int h = j; h < G; h += cpr) {
+        a.part_ml[(base * G + h) * 2] = s_ml[h];
+        a.part_ml[(base * G + h) * 2 + 1] = s_ml[GP + h];
+      }
     }
   } else {
-    const int64_t base = (int64_t)unit * a.max_parts + part;
+    // The waves' O rows and (m, l) meet in LDS; the log-sum-exp rule over them
+    // gives the partition's.
+    if (lane < LPT) {
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
-      f32x4* dst = reinterpret_cast<f32x4*>(a.part_acc + ((base * G + h) * D + j * 8));
-      dst[0] = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-      dst[1] = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+      for (int h = 0; h < G; ++h) {
+        f32x4* dst = reinterpret_cast<f32x4*>(&s_accw[wave][(h * LPT + j) * 8]);
+        dst[0] = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+        dst[1] = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+      }
     }
-    // (m, l) of every head: the row's live lanes take heads j, j + cpr, ...
-    // (cpr may be below G at small head dims)
-    for (int h = j; h < G; h += cpr) {
-      a.part_ml[(base * G + h) * 2] = s_ml[h];
-      a.part_ml[(base * G + h) * 2 + 1] = s_ml[GP + h];
+    __syncthreads();
+    const int D = a.head_dim;
+    // one (head, chunk) of the group per thread: at most 8 * 32
+    static_assert(W == 1 || (G <= 8 && 8 * LPT <= 64 * W), "a thread per (head, chunk)");
+    const int h = threadIdx.x / LPT;
+    if (h >= G || !live) return;
+    float m = s_mlw[0][h];   // the first wave has tokens
+#pragma unroll
+    for (int w = 1; w < W; ++w) m = fmaxf(m, s_mlw[w][h]);
+    float l = 0.f, o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float mw = s_mlw[w][h];
+      const float x = mw == -INFINITY ? 0.f : exp2f(mw - m);   // a wave without tokens adds nothing
+      l += s_mlw[w][GP + h] * x;
+      const f32x4* src = reinterpret_cast<const f32x4*>(&s_accw[w][(h * LPT + j) * 8]);
+      const f32x4 u = src[0], v = src[1];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        o[d] = fmaf(u[d], x, o[d]);
+        o[4 + d] = fmaf(v[d], x, o[4 + d]);
+      }
+    }
+    if (nparts == 1) {
+      store_row8<TT>(a.out + s * a.out_stride_seq + (kh * G + h) * a.out_stride_head + j * 8, o, 1.f / l);
+    } else {
+      const int64_t base = ((int64_t)unit * a.max_parts + part) * G + h;
+      f32x4* dst = reinterpret_cast<f32x4*>(a.part_acc + (base * D + j * 8));
+      dst[0] = f32x4{o[0], o[1], o[2], o[3]};
+      dst[1] = f32x4{o[4], o[5], o[6], o[7]};
+      if (j == 0) {
+        a.part_ml[base * 2] = m;
+        a.part_ml[base * 2 + 1] = l;
+      }
     }
   }
 }
@@ -1823,18 +1894,32 @@ int dispatch_fp8(int g, const DecodeArgs& a, int64_t units, hipStream_t st) {
 
 // Generic path: any head dim (a multiple of 8 from 32 to 256), block size and
 // batch; a wave's lanes per token row are the next power of two above D / 8.
+// Four waves per partition where that measured faster than one (us, one /
+// four, 32 / 8 heads unless given): launches of at most 1024 partitions, less
+// than a wave per SIMD (3 sequences of 12 / 2 heads at D 96 42.4 / 20.5), more
+// than 16 chunks per row (64 sequences at D 160 237 / 188) and groups above 4
+// heads (200 sequences of 64 / 8 heads at D 96 168 / 155). Not the rest: 64
+// sequences at D 96 113 / 117, at D 128 with blocks of 8 119 / 129, 24 at D 96
+// 47.5 / 48.3.
+template <class TT, int LPT, int G>
+void launch_partitions(const DecodeArgs& a, int64_t units, hipStream_t st) {
+  const dim3 grid((unsigned)units, (unsigned)a.max_parts);
+  if constexpr (LPT <= 16 && G <= 4) {
+    if (units * a.max_parts > 1024) {
+      hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 1>), grid, dim3(64), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 4>), grid, dim3(256), 0, st, a);
+}
+
 template <class TT, int G>
 int launch_generic(const DecodeArgs& a, int64_t units, hipStream_t st) {
-  const dim3 grid((unsigned)units, (unsigned)a.max_parts);
   const int cpr = a.head_dim / 8;
-  if (cpr <= 4)
-    hipLaunchKernelGGL((decode_partition_kernel<TT, 4, G>), grid, dim3(64), 0, st, a);
-  else if (cpr <= 8)
-    hipLaunchKernelGGL((decode_partition_kernel<TT, 8, G>), grid, dim3(64), 0, st, a);
-  else if (cpr <= 16)
-    hipLaunchKernelGGL((decode_partition_kernel<TT, 16, G>), grid, dim3(64), 0, st, a);
-  else
-    hipLaunchKernelGGL((decode_partition_kernel<TT, 32, G>), grid, dim3(64), 0, st, a);
+  if (cpr <= 4) launch_partitions<TT, 4, G>(a, units, st);
+  else if (cpr <= 8) launch_partitions<TT, 8, G>(a, units, st);
+  else if (cpr <= 16) launch_partitions<TT, 16, G>(a, units, st);
+  else launch_partitions<TT, 32, G>(a, units, st);
   if (a.max_parts > 1)
     hipLaunchKernelGGL((merge_partitions_kernel<TT, G>), dim3((unsigned)units), dim3(256), 0, st, a);
   return npd::check_launch("npd_paged_attention");

@@ -179,3 +179,33 @@ def test_prefill_fp8_pool_any_head_dim(device, hd, dtype):
     case = _fp8_prefill_case(device, [0, 100, 1500, 77], [64, 37, 200, 1], 8, 2, dtype,
                              seed=hd, D=hd)
     _prefill_run_and_check(device, *case, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd,G,S", [(96, 4, 1), (96, 4, 40), (40, 8, 3), (160, 3, 5), (224, 8, 2)])
+def test_decode_generic_waves_per_partition(device, dtype, hd, G, S):
+    """The generic decode kernel with four waves per partition (few partitions,
+    rows of more than 16 chunks, groups above 4 heads) and with one (40
+    sequences of 2048-token tables at D 96): contexts that leave waves without
+    a token, and a run of tokens whose scores are all -inf."""
+    print(f"decode generic waves D={hd} G={G} S={S} dtype={dtype}", flush=True)
+    g = torch.Generator().manual_seed(hd + S)
+    kvh, bs, mb = 4, 16, 128
+    ctx = ([1, 15, 16, 17, 64, 65, 255, 256, 257, 300, 2047, 2048] * 4)[:S] if S > 1 else [770]
+    kc = (torch.randn(S * mb, kvh, bs, hd, generator=g) * 0.5).to(dtype)
+    vc = (torch.randn(S * mb, kvh, bs, hd, generator=g) * 0.5).to(dtype)
+    q = (torch.rand(S, kvh * G, hd, generator=g) + 0.1).to(dtype)
+    bt = torch.randperm(S * mb, generator=g).to(torch.int32).view(S, mb)
+    if S == 1:   # tokens 64 .. 127: q . k overflows to -inf in bf16, is very low in fp16
+        for blk in bt[0, 4:8].tolist():
+            kc[blk] = torch.finfo(dtype).min
+    sl = torch.tensor(ctx, dtype=torch.int32)
+    kd, vd, qd, out = kc.to(device), vc.to(device), q.to(device), torch.empty_like(q, device=device)
+    pk.paged_attention_forward(out, qd, kd, vd, bt.to(device), sl.to(device), 0.1, bs, mb)
+    for s, n in enumerate(ctx):
+        k = kc[bt[s].long()].permute(0, 2, 1, 3).reshape(-1, kvh, hd)[:n].double()
+        v = vc[bt[s].long()].permute(0, 2, 1, 3).reshape(-1, kvh, hd)[:n].double()
+        sc = torch.einsum("kgd,nkd->kgn", q[s].double().view(kvh, G, hd), k) * 0.1
+        want = torch.einsum("kgn,nkd->kgd", sc.softmax(-1), v).reshape(kvh * G, hd)
+        got = out[s].double().cpu()
+        assert (got - want).abs().max().item() <= (1e-2 if dtype == torch.bfloat16 else 2e-3), (s, n)
