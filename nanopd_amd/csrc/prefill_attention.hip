@@ -707,12 +707,15 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
   //   interval       2i                2i + 1
   //   waves 0-3   QK(i), PV(i-1)     softmax(i)
   //   waves 4-7   softmax(i-1)       QK(i), PV(i-1)
-  // Each wave starts its share of tile i + 3 before softmax(i), in interval
-  // 2i + 1 at the earliest, into the buffers of K tile i - 1 and V tile i - 2
-  // (4 K, 5 V buffers), last read in interval 2i - 1. Its share of tile i + 2
+  // Each wave starts its share of tile i + 3 before softmax(i) (over an FP8
+  // pool at head dim 64, where the MFMAs are the shorter half and the share is
+  // conversions too, before those of step i: 1684 + 994 tokens 47.5 against
+  // 48.7 us; 2-byte pools gain nothing), in interval 2i at the earliest, into the buffers of K tile i - 1 and V tile i - 2 (4 K, 5 V
+  // buffers), last read in interval 2i - 1. Its share of tile i + 2
   // has landed when its softmax(i) is done (interval 2i + 1 or 2i + 2), so the
   // whole tile has when a wave reads its first K operands ahead of step i + 2,
   // at the end of interval 2i + 3 or 2i + 4.
+  constexpr bool kLoadFirst = D == 64 && kF8;
   const bool late = NW == 8 && wave >= NW / 2;
   const int list_steps = (int)((int64_t)(kListBlocks - 2) * bs / KT);   // steps the list covers
   const int seg = list_steps < 1 ? 1 : list_steps;
@@ -784,6 +787,8 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
           if constexpr (kF8) fetch(raw);
         }
       }
+    };
+    auto advance = [&]() {   // to step i + 1's buffers
       kb = (kb + 1) & 3;
       kb3 = (kb3 + 1) & 3;
       vp = vb;
@@ -797,20 +802,24 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
     int i = 0;
     for (; i < nact; ++i) {
       f32x16 sacc[NS];   // S^T[key = n*32 + 8*(i/4) + 4 hf + i%4][row c32]
+      if (kLoadFirst) next_tile(i);
       __builtin_amdgcn_s_setprio(1);
       qk(kb, kpre, sacc);
       pv(vp, pb);
       interleave();
       wait_and_barrier<63>();
       __builtin_amdgcn_s_setprio(0);
-      next_tile(i);
+      if (!kLoadFirst) next_tile(i);
+      advance();
       softmax(sb + i, sacc, pb);
       softmax_done(i);
     }
     pv(vp, pb);
     for (; i < n; ++i) {
+      if (kLoadFirst) next_tile(i);
       wait_and_barrier<63>();
-      next_tile(i);
+      if (!kLoadFirst) next_tile(i);
+      advance();
       softmax_done(i);
     }
     if (!late) wait_and_barrier<63>();   // as many barriers as waves 4-7
