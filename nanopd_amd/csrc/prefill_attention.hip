@@ -28,8 +28,8 @@
 //                        exp2; the row sum is a v_dot2 of the rounded P pair
 //                        with (1, 1). No maximum is taken in the usual step:
 //                        whether the reference must move is read off the packed
-//                        P values (past_bound), and only then the maxima are
-//                        taken, O rescaled and P formed again;
+//                        P values or their sum (Bound), and only then the
+//                        maxima are taken, O rescaled and P formed again;
 //     O^T += V^T . P^T -- P^T is the S^T accumulator, already in B-operand
 //                        layout (packed with v_cvt_pk_bf16_f32); V stays
 //                        row-major in LDS like K, and the V^T A operand is two
@@ -156,38 +156,33 @@ struct Mfma<npd::F16> {
 // maximum it was taken from, P is <= 2^-7 then, and a P of 2 or more (bit 14 of
 // any packed half; also inf and NaN) asks for a new one: one v_or3 per two
 // pairs. fp16 keeps its reference at the maximum (a bias would cost small P
-// their bits) and asks at P >= 2^8, by packed integer maxima. Either way a
-// reference moves when a score passed it by 2^8 and P stays exact enough: fp32
+// their bits) and asks where a lane's P of the step, which are summed anyway,
+// come to kPast = 2^8: one compare, and every P is below 2^8 where none asks.
+// (A packed integer maximum over the 16 registers instead: 291 against 266 us
+// for three chunks of 300-1000 tokens of 64 / 8 heads on prefixes to 4096, FP8
+// pool.) The lane's up to 32 P of such a step have one of 2^3 or more, so that
+// its row moves (kMove). Either way P stays exact enough between moves: fp32
 // sums, relative rounding of the pair.
 template <class TT>
 struct Bound;
 template <>
 struct Bound<npd::BF16> {
-  static constexpr float kBias = 7.f, kMove = 0.f;
+  static constexpr float kBias = 7.f, kMove = 0.f, kPast = 0.f;
 };
 template <>
 struct Bound<npd::F16> {
-  static constexpr float kBias = 0.f, kMove = 7.f;
+  static constexpr float kBias = 0.f, kMove = 2.f, kPast = 256.f;
 };
-template <class TT, int KB>
-__device__ __forceinline__ bool past_bound(const u32x4 (&pb)[KB]) {
-  if constexpr (std::is_same<TT, npd::BF16>::value) {
-    uint32_t o = 0;
+// bf16: any P of 2 or more
+template <int KB>
+__device__ __forceinline__ bool past_two(const u32x4 (&pb)[KB]) {
+  uint32_t o = 0;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      o = o | pb[kb][0] | pb[kb][1];
-      o = o | pb[kb][2] | pb[kb][3];
-    }
-    return (o & 0x40004000u) != 0;
-  } else {
-    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
-    us2 m = __builtin_bit_cast(us2, pb[0][0]);   // P >= 0: ordered as integers
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, pb[kb][i]));
-    return m.x >= 0x5c00u || m.y >= 0x5c00u;   // 2^8
+  for (int kb = 0; kb < KB; ++kb) {
+    o = o | pb[kb][0] | pb[kb][1];
+    o = o | pb[kb][2] | pb[kb][3];
   }
+  return (o & 0x40004000u) != 0;
 }
 
 // Max / sum over the 4 key groups of a query row (lanes l, l^16, l^32, l^48).
@@ -637,10 +632,29 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
               TT::pack2(__builtin_amdgcn_exp2f(fmaf(sacc[n][i], c2, nmref)),
                         __builtin_amdgcn_exp2f(fmaf(sacc[n][i + 1], c2, nmref)));
     };
+    // sum of this lane's P of the step on top of x
+    auto sum_p = [&](float x) {
+      float ps[4] = {x, 0.f, 0.f, 0.f};   // four short chains
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ps[i] = TT::dot2(pb[kb][i], TT::kOne2, ps[i]);
+      return (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    };
     expo();
     // The reference moves only when an exponential grew past a bound, read off
-    // the packed values: the maximum is taken in that rare case only.
-    if (__builtin_expect(__ballot(past_bound<TT, KB>(pb)) != 0, 0)) {
+    // the packed values or their sum: the maximum is taken in that rare case
+    // only.
+    constexpr bool kBySum = std::is_same<TT, npd::F16>::value;
+    float st = 0.f;
+    bool past;
+    if constexpr (kBySum) {
+      st = sum_p(0.f);
+      past = st >= Bound<TT>::kPast;
+    } else {
+      past = past_two(pb);
+    }
+    if (__builtin_expect(__ballot(past) != 0, 0)) {
       float mx = fmaxf(fmaxf(sacc[0][0], sacc[0][1]), sacc[0][2]);
 #pragma unroll
       for (int e = 3; e + 1 < 16 * NS; e += 2)
@@ -655,13 +669,10 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
       mref = mnew;
       nmref = mnew == -INFINITY ? kNoRef : -mnew;
       expo();
+      if constexpr (kBySum) st = sum_p(0.f);
     }
-    float ps[4] = {lsum, 0.f, 0.f, 0.f};   // four short chains
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ps[i] = TT::dot2(pb[kb][i], TT::kOne2, ps[i]);
-    lsum = (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    if constexpr (kBySum) lsum += st;
+    else lsum = sum_p(lsum);
   };
   // O^T += V^T . P^T ; A = V^T[d = db*32 + c32][keys as pb's slots]: two
   // transposing reads, in each of which lane i of a group of 16 addresses key

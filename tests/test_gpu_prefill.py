@@ -305,3 +305,35 @@ def test_exponent_reference_moves(device, dtype):
             kc[b, 0, i % bs] = (kc[b, 0, i % bs].float() * 0.2 + r[i]).to(dtype)
     q.copy_((q.float() * 0.2 + 1.0).to(dtype))
     check(run(*args, 0.12), q, kc, vc, bt, cu, ctx, 0.12)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("hd,kvh", [(64, 2), (128, 2), (128, 8), (256, 2)])
+def test_one_late_key_far_above_the_rest(device, dtype, fp8, hd, kvh):
+    """32 sequences, each with one key (the 32 positions of a 32-key block after
+    two steps of near-zero scores) whose score is 46 log2 units above all others:
+    wherever it sits, the exponent reference has to move (P of 2^46 is no fp16
+    number). Head dim 128 by workgroups of 4 waves (2 kv heads) and of 8."""
+    print(f"prefill late key D={hd} {dtype} fp8={fp8} kvh={kvh}", flush=True)
+    g = torch.Generator().manual_seed(hd)
+    args = make_case("cpu", [200] * 32, [3] * 32, H=4 * kvh, kvh=kvh, D=hd, dtype=dtype, seed=hd)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    q.copy_((0.5 + 0.05 * torch.randn(q.shape, generator=g)).to(dtype))
+    kc.copy_((kc.float() * 0.1).to(dtype))
+    for s in range(32):
+        key = 128 + s
+        kc[bt[s, key // 16], :, key % 16] = 64.0 / math.sqrt(hd)
+    scale, ks = 1 / math.sqrt(hd), 1 / 16
+    dev = [x.to(device) for x in (q, kc, vc, bt, cu, ctx)]
+    if fp8:
+        k8, v8 = ((c.float() / ks).to(torch.float8_e4m3fn) for c in (kc, vc))
+        kc, vc = ((c.float() * ks).to(dtype) for c in (k8, v8))   # exact
+        out = torch.full_like(q, float("nan")).to(device)
+        sc = torch.full((kvh,), ks, device=device)
+        pk.paged_prefill_attention_fp8(out, dev[0], k8.to(device), v8.to(device), *dev[3:], scale,
+                                       16, mb, mq, sc, sc)
+        torch.cuda.synchronize()
+    else:
+        out = run(*dev, mb, mq, scale)
+    check(out, q, kc, vc, bt, cu, ctx, scale)
