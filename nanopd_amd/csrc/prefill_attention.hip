@@ -11,10 +11,10 @@
 //
 // MI355X design (gfx950, v_mfma_f32_32x32x16_{bf16,f16}, wave64):
 //   head dim D = 64, 128 or 256 (prefill_kernel<.., D, ..>; the other multiples
-//   of 32 up to 224 run prefill_generic_kernel below);
+//   of 32 up to 224, and 256 over an FP8 pool, run prefill_generic_kernel below);
 //   workgroup = 8 waves = one (sequence, kv-head, tile of 256 rows, key part)
 //   -- 4 waves and 128 rows, without the half-step shift below, at head dim 256
-//   (32 keys per step, no key parts) and for few tiles at 128.
+//   (no key parts) and for few tiles at 128.
 //   Rows are (token, head) pairs of the kv head's G query heads, flattened as
 //   token * G + head: any G fills its tiles, and a wave's 32 rows span 32 / G
 //   tokens, so its causal range ends with the tile's. With 8
@@ -78,9 +78,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kWaveRows = 32;    // flattened (token, head) rows per wave
 constexpr int tile_rows(int nw) { return nw * kWaveRows; }   // ... and per workgroup of nw waves
 constexpr int kKT = 64;          // keys per step
-// ... of prefill_kernel at head dim d: 32 at 256, so that its tiles (16 KB) and
-// accumulators fit
-constexpr int step_keys(int d) { return d == 256 ? 32 : kKT; }
 constexpr int kBufK = 4;         // K tiles in LDS
 constexpr int kBufV = 5;         // V tiles in LDS
 constexpr int kListBlocks = 2048;     // blocks of the key range listed in LDS at a time (8 KB)
@@ -152,7 +149,7 @@ struct Mfma<npd::F16> {
   }
 };
 
-// When a row's reference moves. bf16: the reference sits kBias above the
+// When a row's reference moves (head dims 64 and 128). bf16: the reference sits kBias above the
 // maximum it was taken from, P is <= 2^-7 then, and a P of 2 or more (bit 14 of
 // any packed half; also inf and NaN) asks for a new one: one v_or3 per two
 // pairs. fp16 keeps its reference at the maximum (a bias would cost small P
@@ -428,8 +425,8 @@ __device__ __forceinline__ void wait_and_barrier() {
 // scales go into the score scale and the output.
 template <class TT, int D, int NW, bool kOff32, bool kF8>
 __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
-  static_assert(D == 64 || D == 128 || D == 256, "head dims of this kernel");
-  constexpr int KT = step_keys(D);                     // keys per step
+  static_assert(D == 64 || D == 128 || (D == 256 && !kF8), "head dims of this kernel");
+  constexpr int KT = kKT;                              // keys per step
   constexpr int NT = 64 * NW;                          // threads
   constexpr int RB = 2 * D;                            // bytes of a tile row
   constexpr int TB = KT * RB;                         // bytes of a K or V tile
@@ -439,9 +436,18 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
   constexpr int KB = KT / 16;                         // 16-key blocks of PV
   constexpr int DB = D / 32;                           // 32-dim blocks of O
   constexpr int kRecO = rec_o(D);
+  // Head dim 256 keeps the running maximum of a row as its reference, so that
+  // the largest P is 1 and exact: one that lags leaves 3 to 9% more error in the
+  // output where few keys dominate a row. The 128 accumulators of O are rescaled
+  // in most of the first steps then (one of 32 rows has a new maximum), so steps
+  // are of 64 keys (of 32: 127 against 103 us for three chunks of 300 to 700
+  // tokens of 16 / 8 heads on prefixes to 1500; a lagging reference 88), and two
+  // tiles of 32 KB each are what fits: the next one loads during the step.
+  constexpr bool kExactMax = D == 256;
+  constexpr int NBK = kExactMax ? 2 : kBufK, NBV = kExactMax ? 2 : kBufV;
   static_assert(NI * 1024 * NW == TB, "tile shape");
-  __shared__ __attribute__((aligned(1024))) char s_k[kBufK * TB];
-  __shared__ __attribute__((aligned(1024))) char s_v[kBufV * TB];
+  __shared__ __attribute__((aligned(1024))) char s_k[NBK * TB];
+  __shared__ __attribute__((aligned(1024))) char s_v[NBV * TB];
   __shared__ int s_row[kListBlocks];   // first K/V row of each block of the key range
   __shared__ int s_ticket;
   __shared__ Item s_item;
@@ -641,6 +647,33 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
         for (int i = 0; i < 4; ++i) ps[i] = TT::dot2(pb[kb][i], TT::kOne2, ps[i]);
       return (ps[0] + ps[1]) + (ps[2] + ps[3]);
     };
+    // the row's scaled maximum of the step
+    auto row_max = [&]() {
+      float mx = fmaxf(fmaxf(sacc[0][0], sacc[0][1]), sacc[0][2]);
+#pragma unroll
+      for (int e = 3; e + 1 < 16 * NS; e += 2)
+        mx = fmaxf(fmaxf(mx, sacc[e >> 4][e & 15]), sacc[(e + 1) >> 4][(e + 1) & 15]);
+      return npd::half_max(fmaxf(mx, sacc[NS - 1][15])) * c2;
+    };
+    // a row whose maximum passed its reference by `move` takes it, plus `bias`,
+    // as the new one
+    auto move_ref = [&](float mx, float move, float bias) {
+      const bool nd = mx > mref + move;
+      const float mnew = nd ? mx + bias : mref;
+      const float alpha = nd ? __builtin_amdgcn_exp2f(mref - mnew) : 1.f;   // 0 from -inf
+#pragma unroll
+      for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
+      lsum *= alpha;
+      mref = mnew;
+      nmref = mnew == -INFINITY ? kNoRef : -mnew;
+    };
+    if constexpr (kExactMax) {
+      const float mx = row_max();
+      if (__ballot(mx > mref) != 0) move_ref(mx, 0.f, 0.f);
+      expo();
+      lsum = sum_p(lsum);
+      return;
+    }
     expo();
     // The reference moves only when an exponential grew past a bound, read off
     // the packed values or their sum: the maximum is taken in that rare case
@@ -655,19 +688,7 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
       past = past_two(pb);
     }
     if (__builtin_expect(__ballot(past) != 0, 0)) {
-      float mx = fmaxf(fmaxf(sacc[0][0], sacc[0][1]), sacc[0][2]);
-#pragma unroll
-      for (int e = 3; e + 1 < 16 * NS; e += 2)
-        mx = fmaxf(fmaxf(mx, sacc[e >> 4][e & 15]), sacc[(e + 1) >> 4][(e + 1) & 15]);
-      mx = npd::half_max(fmaxf(mx, sacc[NS - 1][15])) * c2;
-      const bool nd = mx > mref + Bound<TT>::kMove;
-      const float mnew = nd ? mx + Bound<TT>::kBias : mref;
-      const float alpha = nd ? __builtin_amdgcn_exp2f(mref - mnew) : 1.f;   // 0 from -inf
-#pragma unroll
-      for (int db = 0; db < DB; ++db) oacc[db] *= alpha;
-      lsum *= alpha;
-      mref = mnew;
-      nmref = mnew == -INFINITY ? kNoRef : -mnew;
+      move_ref(row_max(), Bound<TT>::kMove, Bound<TT>::kBias);
       expo();
       if constexpr (kBySum) st = sum_p(0.f);
     }
@@ -747,17 +768,41 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
     // the loop would cover the tile loads too
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
     __syncthreads();
-    // P of the step before the segment: none. Its V tile (the last buffer) is
-    // zeroed too, so that the first interval's PV adds nothing.
-    u32x4 pb[KB];
-#pragma unroll
-    for (int e = 0; e < KB; ++e) pb[e] = u32x4{0, 0, 0, 0};
-    for (int e = tid; e < TB / 16; e += NT)
-      *reinterpret_cast<u32x4*>(s_v + (kBufV - 1) * TB + e * 16) = u32x4{0, 0, 0, 0};
     // steps in which some row of this wave sees a key (the causal mask only
     // ever ends a wave's steps): later ones it spends in the barriers
     int nact = wpos1 < sb * KT ? 0 : wpos1 / KT - sb + 1;
     nact = nact < n ? nact : n;
+    u32x4 pb[KB];
+    if constexpr (kExactMax) {
+      // One wave per SIMD: QK, softmax and PV of a step in turn, one barrier
+      // per step. Past it tile i has landed and every wave has left step i - 1,
+      // whose buffers tile i + 1 loads into.
+      find_rows(sb);
+      load(0, 0);
+      for (int i = 0; i < n; ++i) {
+        const int b = i & 1;
+        wait_and_barrier<0>();
+        if (i + 1 < n) {
+          find_rows(sb + i + 1);
+          load(b ^ 1, b ^ 1);
+        }
+        if (i >= nact) continue;
+        f32x16 sacc[NS];
+        u32x4 kpre[kAhead];
+#pragma unroll
+        for (int x = 0; x < kAhead; ++x) kpre[x] = read_k(b, x);
+        qk(b, kpre, sacc);
+        softmax(sb + i, sacc, pb);
+        pv(b, pb);
+      }
+      continue;
+    }
+    // P of the step before the segment: none. Its V tile (the last buffer) is
+    // zeroed too, so that the first interval's PV adds nothing.
+#pragma unroll
+    for (int e = 0; e < KB; ++e) pb[e] = u32x4{0, 0, 0, 0};
+    for (int e = tid; e < TB / 16; e += NT)
+      *reinterpret_cast<u32x4*>(s_v + (kBufV - 1) * TB + e * 16) = u32x4{0, 0, 0, 0};
     Raw raw;   // FP8: the bytes of the tile stashed next
     if constexpr (kF8) {
       Raw r1, r2;
@@ -898,7 +943,7 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
 }
 
 // The head dims whose rows are not a power of two of 16-byte chunks (32, 96,
-// 160, 192, 224). One workgroup of 4 waves per
+// 160, 192, 224), and 256 over an FP8 pool. One workgroup of 4 waves per
 // (sequence, query head, 64-row query tile); wave w owns query rows
 // 16w .. 16w + 15 of the tile. Per step of 64 keys the workgroup copies the kv
 // head's K and V rows into LDS (keys past the visible range clamped to the
@@ -923,7 +968,7 @@ __global__ __launch_bounds__(256, 2) void prefill_generic_kernel(PrefillArgs a) 
   constexpr int NPASS = kKT * CPR / kGT;        // chunks of the 64-key tile per thread
   constexpr int NC = D / 32;                    // head-dim chunks of QK
   constexpr int NB = D / 16;                    // 16-dim blocks of O
-  static_assert(D % 32 == 0 && D >= 32 && D < 256, "head dims of this kernel");
+  static_assert(D % 32 == 0 && D >= 32 && D <= 256, "head dims of this kernel");
   static_assert(NPASS * kGT == kKT * CPR && RW % 8 == 0, "tile shape");
   __shared__ __attribute__((aligned(16))) uint16_t s_k[kKT * RW];
   __shared__ __attribute__((aligned(16))) uint16_t s_v[kKT * RW];
@@ -1120,7 +1165,14 @@ int launch_generic(int64_t head_dim, const PrefillArgs& a, int64_t grid, hipStre
     case 160: hipLaunchKernelGGL((prefill_generic_kernel<TT, 160, kF8>), g, b, 0, st, a); break;
     case 192: hipLaunchKernelGGL((prefill_generic_kernel<TT, 192, kF8>), g, b, 0, st, a); break;
     case 224: hipLaunchKernelGGL((prefill_generic_kernel<TT, 224, kF8>), g, b, 0, st, a); break;
-    default: return npd::fail(NPD_E_INVALID, "%s: head_dim %lld", name, (long long)head_dim);
+    default:
+      if constexpr (kF8) {
+        if (head_dim == 256) {
+          hipLaunchKernelGGL((prefill_generic_kernel<TT, 256, kF8>), g, b, 0, st, a);
+          break;
+        }
+      }
+      return npd::fail(NPD_E_INVALID, "%s: head_dim %lld", name, (long long)head_dim);
   }
   return npd::check_launch(name);
 }
@@ -1135,8 +1187,9 @@ void launch_d(bool off32, const PrefillArgs& a, int64_t grid, hipStream_t st) {
 template <class TT, bool kF8>
 int launch_dt(int64_t head_dim, int waves, bool off32, const PrefillArgs& a, int64_t grid,
               hipStream_t st, const char* name) {
-  if (head_dim == 256) launch_d<TT, 256, 4, kF8>(off32, a, grid, st);
-  else if (head_dim == 64) launch_d<TT, 64, 8, kF8>(off32, a, grid, st);
+  if (head_dim == 256) {
+    if constexpr (!kF8) launch_d<TT, 256, 4, false>(off32, a, grid, st);
+  } else if (head_dim == 64) launch_d<TT, 64, 8, kF8>(off32, a, grid, st);
   else if (waves == 8) launch_d<TT, 128, 8, kF8>(off32, a, grid, st);
   else launch_d<TT, 128, 4, kF8>(off32, a, grid, st);
   return npd::check_launch(name);
@@ -1210,8 +1263,10 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
     return fail(NPD_E_INVALID, "%s: head_dim %lld is not a multiple of 32 in [32, 256]", name,
                 (long long)head_dim);
   // head dims 64, 128 and 256: prefill_kernel (256 without key splits: its
-  // callers bring no workspace); every other one: prefill_generic_kernel
-  const bool generic = head_dim != 64 && head_dim != 128 && head_dim != 256;
+  // callers bring no workspace); every other one, and 256 over an FP8 pool
+  // (three chunks of 300 to 700 tokens of 16 / 8 heads on prefixes to 1500:
+  // 100.5 us, prefill_kernel with the exact maximum 121): prefill_generic_kernel
+  const bool generic = head_dim != 64 && head_dim != 128 && (head_dim != 256 || fp8);
   if (num_heads % num_kv_heads != 0)
     return fail(NPD_E_INVALID, "%s: num_heads %lld is not a multiple of num_kv_heads %lld", name,
                 (long long)num_heads, (long long)num_kv_heads);

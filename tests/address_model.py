@@ -584,7 +584,7 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
     if D == 256:
         waves = 4
     L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus, waves=waves,
-                      kt=32 if D == 256 else KT)
+                      kt=KT)
     g = H // KV
     tq = S * max_q_len if total_q is None else total_q
     if D == 256:

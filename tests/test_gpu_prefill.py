@@ -337,3 +337,34 @@ def test_one_late_key_far_above_the_rest(device, dtype, fp8, hd, kvh):
     else:
         out = run(*dev, mb, mq, scale)
     check(out, q, kc, vc, bt, cu, ctx, scale)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("spread", [3.0, 6.0])
+def test_head_dim_256_rounds_no_more_than_an_exact_maximum(device, dtype, spread):
+    """Peaked rows at head dim 256: the error against float64 is that of
+    probabilities relative to the row's maximum (the largest is exactly 1),
+    rounded to the dtype, summed as rounded -- computed here in fp32 from the
+    same inputs. 262144 outputs: their RMS error is known to well below 1%, and
+    a reference that lags the maximum adds 10% and more."""
+    D, H, px, ch = 256, 4, 960, 64
+    scale = 1 / math.sqrt(D)
+    args = make_case(device, [px] * 4, [ch] * 4, H=H, kvh=1, D=D, dtype=dtype, seed=int(spread))
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    q.copy_((q.float() * 4 * spread).to(dtype))   # scores of standard deviation `spread`
+    got = run(*args, scale)
+    see = torch.arange(px + ch, device=device)[None] <= px + torch.arange(ch, device=device)[:, None]
+    err = emu = 0.0
+    for s in range(4):
+        k, v = (c[bt[s].long()].permute(0, 2, 1, 3).reshape(-1, D)[:px + ch].float() for c in (kc, vc))
+        qs = q[s * ch:(s + 1) * ch].float().reshape(ch * H, D)
+        sc = (qs @ k.t().contiguous()) * scale
+        sc.masked_fill_(~see.repeat_interleave(H, 0), -math.inf)
+        want = torch.softmax(sc.double(), -1) @ v.double()
+        p = torch.exp(sc - sc.amax(-1, keepdim=True)).to(dtype).float()
+        e = ((p @ v) / p.sum(-1, keepdim=True)).to(dtype).double()
+        emu += (e - want).pow(2).sum().item()
+        err += (got[s * ch:(s + 1) * ch].reshape(ch * H, D).double() - want).pow(2).sum().item()
+    ratio = math.sqrt(err / emu)
+    print(f"head dim 256 {dtype} spread {spread}: error {ratio:.3f} of the emulation's")
+    assert ratio <= 1.05
