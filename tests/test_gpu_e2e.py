@@ -21,9 +21,12 @@ SMALL = Qwen3Config(num_layers=3, hidden=1024, num_heads=16, num_kv_heads=4, hea
                     intermediate=2048, vocab=4096, init_std=0.05)
 
 
-def torch_attention(layer, q, kc, vc, b: StepBatch, out):
+def torch_attention(layer, q, kc, vc, b: StepBatch, out, p_shift=None):
     """fp32 attention over each sequence's paged context (after the step's
-    store): row i of a q_len-row sequence sits at position ctx - q_len + i."""
+    store): row i of a q_len-row sequence sits at position ctx - q_len + i.
+    p_shift: probabilities relative to the row's maximum less p_shift log2
+    units, rounded to q's dtype and summed as rounded, as the matrix cores take
+    them."""
     m = b.meta
     cu = m.cu_seqlens_q.tolist()
     sl = m.seq_lens.tolist()
@@ -44,7 +47,12 @@ def torch_attention(layer, q, kc, vc, b: StepBatch, out):
         pos = ctx - (e - a) + torch.arange(e - a, device=q.device)
         mask = torch.arange(ctx, device=q.device)[None, :] > pos[:, None]
         sc = sc.masked_fill(mask[None], float("-inf"))
-        out[a:e] = torch.matmul(torch.softmax(sc, dim=-1), V).transpose(0, 1).to(out.dtype)
+        if p_shift is None:
+            o = torch.matmul(torch.softmax(sc, dim=-1), V)
+        else:
+            p = torch.exp(sc - sc.amax(-1, keepdim=True) + p_shift * math.log(2)).to(q.dtype).float()
+            o = torch.matmul(p, V) / p.sum(-1, keepdim=True)
+        out[a:e] = o.transpose(0, 1).to(out.dtype)
 
 
 def _model(device, attention=None, fused_prologue=True):
@@ -163,42 +171,97 @@ def test_serve_reports_throughput(device):
     assert res["tok_per_s"] > 0 and res["wall_s"] > 0
 
 
+def _dequantised(model, layer, kc, vc):
+    return (kc.float() * model.k_scale[layer][None, :, None, None],
+            vc.float() * model.v_scale[layer][None, :, None, None])
+
+
+def _fp8_models(device, count):
+    """The FP8-pool model `count` times, over the same random codes in its pool
+    (uniform over the e4m3 codes: wide, so that the scores are peaked)."""
+    ms = [PagedQwen3(SMALL, num_blocks=512, block_size=16, device=device, seed=3,
+                     kv_cache_dtype="fp8") for _ in range(count)]
+    g = torch.Generator(device=device).manual_seed(9)
+    shape = ms[0].k_cache.shape
+    codes = torch.randint(0, 0x7E, shape, generator=g, device=device,
+                          dtype=torch.int32) | (torch.randint(0, 2, shape, generator=g,
+                                                              device=device, dtype=torch.int32) << 7)
+    for m in ms:
+        m.k_cache.view(torch.uint8).copy_(codes.to(torch.uint8))
+        m.v_cache.view(torch.uint8).copy_(codes.flip(0).to(torch.uint8))
+    return ms
+
+
+def test_fp8_pool_layers_match_torch_attention(device):
+    """Each layer's attention of an FP8-pool model step (prefill and decode ops)
+    against fp32 attention of the same q over the same dequantised pool, so that
+    no layer sees another one's rounding. u = 2^-8 is bf16's unit roundoff.
+    Element by element: the probabilities are rounded (numerator and sum: at
+    most u of sum p |v| / sum p, called A, and u of |o|), then the output (u of
+    |o|); and 1e-4 of A for fp32 scores of magnitude 100. Over a layer: two
+    independent roundings of rms at most u / sqrt(3) each."""
+    (m,) = _fp8_models(device, 1)
+    u = 2.0 ** -8
+    rel = []
+
+    def attend(layer, q, kc, vc, b, out):
+        m._paged_attention(layer, q, kc, vc, b, out)
+        K, V = _dequantised(m, layer, kc, vc)
+        want, A = torch.empty_like(q, dtype=torch.float32), torch.empty_like(q, dtype=torch.float32)
+        torch_attention(layer, q, K, V, b, want)
+        torch_attention(layer, q, K, V.abs(), b, A)
+        err = (out.float() - want).abs()
+        assert (err <= u * 1.01 * (A + 2 * want.abs()) + 1e-4 * A).all(), layer
+        tp = b.num_prefill_tokens
+        for rows in (slice(0, tp), slice(tp, None)):
+            rel.append((err[rows].norm() / want[rows].norm()).item())
+
+    m.attention = attend
+    m.forward(_mixed_batch(m, device))
+    print("fp8 pool, per layer (prefill, decode) relative error: " + " ".join(f"{r:.2e}" for r in rel))
+    assert len(rel) == 2 * SMALL.num_layers and max(rel) <= u * math.sqrt(2 / 3)
+
+
 def test_fp8_pool_step_matches_torch_attention(device):
     """The model with an FP8 (e4m3) KV pool: the fused prologue stores e4m3
     bytes, the FP8 prefill and decode ops read them. Against the same model
     with the fp32 PyTorch attention over the dequantised pool (e4m3 * scale),
-    after identical random prefix/context bytes in both pools: the logits agree
-    as closely as the 2-byte pools' A/B, and the step's own K/V bytes are the
-    same in both pools (layer 0 sees identical inputs)."""
-    def torch_attention_fp8(model):
-        def attend(layer, q, kc, vc, b, out):
-            ks = model.k_scale[layer][None, :, None, None]
-            vs = model.v_scale[layer][None, :, None, None]
-            torch_attention(layer, q, kc.float() * ks, vc.float() * vs, b, out)
-        return attend
+    after identical random prefix/context bytes in both pools. The step's own
+    K/V bytes are the same in both pools (layer 0 sees identical inputs).
 
-    hip = PagedQwen3(SMALL, num_blocks=512, block_size=16, device=device, seed=3,
-                     kv_cache_dtype="fp8")
-    ref = PagedQwen3(SMALL, num_blocks=512, block_size=16, device=device, seed=3,
-                     kv_cache_dtype="fp8")
-    ref.attention = torch_attention_fp8(ref)
-    g = torch.Generator(device=device).manual_seed(9)
-    codes = torch.randint(0, 0x7E, hip.k_cache.shape, generator=g, device=device,
-                          dtype=torch.int32) | (torch.randint(0, 2, hip.k_cache.shape, generator=g,
-                                                              device=device, dtype=torch.int32) << 7)
-    for m in (hip, ref):
-        m.k_cache.view(torch.uint8).copy_(codes.to(torch.uint8))
-        m.v_cache.view(torch.uint8).copy_(codes.flip(0).to(torch.uint8))
-    del codes
+    How far the logits may be apart is taken from the model itself: three bf16
+    layers of peaked attention amplify the last bit of an attention output, and
+    PyTorch attention with its probabilities rounded to bf16 is as far from
+    fp32 attention as the ops are. Over 12 to 24 seeds of this step three
+    attentions (16x16x32 and 32x32x16 MFMA prefill with bf16 probabilities, and
+    one with fp16 probabilities, a third of the error per layer) were all 0.012
+    to 0.028 of the logit range off, 0.018 to 0.019 on average, with a standard
+    deviation of 0.004. So the bound is twice the farthest of four such roundings
+    (references at 0, 1/4, 1/2, 3/4 log2 units from the maximum); the ops
+    themselves are held by the test above."""
+    hip, ref = _fp8_models(device, 2)
     b = _mixed_batch(hip, device)
+    pools = [(c.view(torch.uint8), c.view(torch.uint8).clone()) for c in (ref.k_cache, ref.v_cache)]
+
+    def logits_of(p_shift):
+        for pool, start in pools:
+            pool.copy_(start)
+        ref.attention = lambda layer, q, kc, vc, b, out: torch_attention(
+            layer, q, *_dequantised(ref, layer, kc, vc), b, out, p_shift)
+        return ref.forward(b)
+
     lh = hip.forward(b)
-    lr = ref.forward(b)
+    rounded = [logits_of(f) for f in (0.0, 0.25, 0.5, 0.75)]
+    lr = logits_of(None)
     torch.cuda.synchronize()
     assert torch.isfinite(lh).all()
     err = (lh - lr).abs().max().item()
+    own = [(x - lr).abs().max().item() for x in rounded]
     spread = lr.abs().max().item()
-    print(f"fp8 pool: logits max-abs {err:.3e} (|logits| max {spread:.2f})")
-    assert err <= 2e-2 * max(1.0, spread)
+    print(f"fp8 pool: logits max-abs {err:.3e} (|logits| max {spread:.2f}), PyTorch with rounded "
+          "probabilities " + " ".join(f"{x:.3e}" for x in own))
+    assert 0 < max(own) <= 4e-2 * max(1.0, spread)
+    assert err <= 2 * max(own)
     assert (lh.argmax(-1) == lr.argmax(-1)).float().mean().item() >= 5 / 6
     assert torch.equal(hip.k_cache[0].view(torch.uint8), ref.k_cache[0].view(torch.uint8))
     assert torch.equal(hip.v_cache[0].view(torch.uint8), ref.v_cache[0].view(torch.uint8))
