@@ -694,9 +694,12 @@ def qk_norm_rope_store(q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 
 
 def _rows_16(*ts: torch.Tensor) -> bool:
-    """Contiguous 2-byte tensors that start on 16 bytes, with whole 16-byte rows."""
-    return all(t.is_cuda and t.dtype in _DTYPES and t.dtype == ts[0].dtype and t.is_contiguous()
-               and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts)
+    """Contiguous 2-byte tensors of one dtype and one GPU that start on 16 bytes,
+    with whole 16-byte rows."""
+    t0 = ts[0]
+    return (t0.is_cuda and t0.dtype in _DTYPES
+            and all(t.get_device() == t0.get_device() and t.dtype == t0.dtype and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts))
 
 
 def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tensor,
@@ -704,8 +707,9 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tens
     """RMSNorm over the last dim of x + delta, which is left in ``x`` (delta
     None: of x). The sum is rounded to the dtype, the norm once after fp32.
     2-byte CUDA tensors of up to 8192 columns run as one launch, others as the
-    torch operations."""
-    if (x.dim() == 2 and x.size(1) <= 8192 and _rows_16(x, weight)
+    torch operations, which also refuse what does not fit together (the kernel
+    reads x.size(1) weights and as many deltas as x has elements)."""
+    if (x.dim() == 2 and x.size(1) <= 8192 and weight.shape == x.shape[1:] and _rows_16(x, weight)
             and (delta is None or (delta.shape == x.shape and _rows_16(x, delta)))):
         out = torch.empty_like(x)
         _lib.call("npd_add_rms_norm", out.data_ptr(), x.data_ptr(),
