@@ -695,11 +695,12 @@ def qk_norm_rope_store(q_out: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
 
 def _rows_16(*ts: torch.Tensor) -> bool:
     """Contiguous 2-byte tensors of one dtype and one GPU that start on 16 bytes,
-    with whole 16-byte rows."""
+    with whole 16-byte rows, none empty, none to record a gradient for."""
     t0 = ts[0]
-    return (t0.is_cuda and t0.dtype in _DTYPES
+    return (t0.is_cuda and t0.dtype in _DTYPES and t0.numel() > 0
             and all(t.get_device() == t0.get_device() and t.dtype == t0.dtype and t.is_contiguous()
-                    and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts))
+                    and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
 
 
 def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tensor,

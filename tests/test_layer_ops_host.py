@@ -53,3 +53,18 @@ def test_add_rms_norm_launches_nothing_across_gpus(launches, which):
     w, d = on_gpu(64, gpu=which == "weight"), on_gpu(2, 64, gpu=which == "delta")
     pk.add_rms_norm(x, d, w, 1e-6)   # (the torch operations refuse real tensors of two GPUs)
     assert not launches
+
+
+def test_no_launch_records_a_gradient_or_takes_nothing(launches):
+    w = on_gpu(64).requires_grad_()
+    assert pk.add_rms_norm(on_gpu(2, 64), None, w, 1e-6).requires_grad
+    with torch.no_grad():
+        assert not launches
+        pk.add_rms_norm(on_gpu(2, 64), None, w, 1e-6)
+    assert len(launches) == 1
+    assert pk.add_rms_norm(on_gpu(0, 64), None, w, 1e-6).shape == (0, 64)
+    assert len(launches) == 1
+    with torch.enable_grad():
+        assert pk.silu_mul(on_gpu(2, 64).requires_grad_()).requires_grad
+    assert pk.silu_mul(on_gpu(3, 0)).shape == (3, 0)
+    assert len(launches) == 1
