@@ -723,15 +723,17 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tens
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
-    """silu(gate) * up of rows [gate | up] (one launch for 2-byte CUDA tensors,
-    the torch operations otherwise)."""
-    n = gate_up.size(-1) // 2
+    """silu(gate) * up of rows [gate | up], of any rank (one launch for 2-byte
+    CUDA tensors of two dims, the torch operations otherwise)."""
+    n, odd = divmod(gate_up.size(-1), 2)
+    if odd:
+        _fail(f"gate_up rows of {gate_up.size(-1)}: a gate and an up half of one width are wanted")
     if gate_up.dim() == 2 and n % 8 == 0 and _rows_16(gate_up):
         out = torch.empty(gate_up.size(0), n, dtype=gate_up.dtype, device=gate_up.device)
         _lib.call("npd_silu_mul", out.data_ptr(), gate_up.data_ptr(), gate_up.size(0), n,
                   _DTYPES[gate_up.dtype], _stream(gate_up.device))
         return out
-    return torch.nn.functional.silu(gate_up[:, :n]) * gate_up[:, n:]
+    return torch.nn.functional.silu(gate_up[..., :n]) * gate_up[..., n:]
 
 
 class BatchMetadata(NamedTuple):

@@ -68,3 +68,19 @@ def test_no_launch_records_a_gradient_or_takes_nothing(launches):
         assert pk.silu_mul(on_gpu(2, 64).requires_grad_()).requires_grad
     assert pk.silu_mul(on_gpu(3, 0)).shape == (3, 0)
     assert len(launches) == 1
+
+
+@pytest.mark.parametrize("shape", [(32,), (2, 32), (2, 1, 32), (3, 2, 5, 16), (2, 6)])
+def test_silu_mul_takes_the_halves_of_the_last_dim(shape):
+    gu = torch.randn(*shape, generator=torch.Generator().manual_seed(1))
+    n = shape[-1] // 2
+    gate, up = gu.split(n, dim=-1)
+    got = pk.silu_mul(gu)
+    assert got.shape == shape[:-1] + (n,)
+    assert torch.equal(got, torch.nn.functional.silu(gate) * up)
+
+
+@pytest.mark.parametrize("shape", [(2, 3), (2, 17), (1, 2, 5)])
+def test_silu_mul_refuses_halves_of_two_widths(shape):
+    with pytest.raises(RuntimeError):
+        pk.silu_mul(torch.ones(*shape))
