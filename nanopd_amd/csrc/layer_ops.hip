@@ -80,8 +80,11 @@ __global__ __launch_bounds__(kThreads) void silu_mul_kernel(u32x4* __restrict__ 
   const int64_t src = at + row * chunks;   // row * 2 * chunks + column
   const u32x4 g = gu[src], u = gu[src + chunks];
   auto silu = [](float x) {
-    // x / (1 + e^-x): 0 at -inf's side (e^-x overflows to inf), x at +inf's
-    return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f));
+    // x / (1 + e^-x): 0 at -inf's side (e^-x overflows to inf), x at +inf's. Of
+    // a quarter of the divisor, whose reciprocal is a normal number: below -87.3
+    // that of the divisor itself is not, and v_rcp_f32 would make it 0.
+    const float e = __builtin_amdgcn_exp2f(x * -1.4426950408889634f);
+    return x * 0.25f * __builtin_amdgcn_rcpf(fmaf(e, 0.25f, 0.25f));
   };
   u32x4 y;
 #pragma unroll

@@ -52,3 +52,15 @@ def test_silu_mul(device, dtype, rows, width):
     assert (err <= U[dtype] * 2.01 * want.abs()[fin] + half * 1.01 * (up.abs()[fin] + 1)).all()
     nan = torch.full((1, 16), float("nan"), dtype=dtype, device=device)
     assert pk.silu_mul(nan).isnan().all()
+
+
+def test_silu_of_far_negative_gates(device):
+    """Gates down to -88.5, where 1 / (1 + e^88) is no normal fp32 number but
+    silu(-88) = -5.3e-37 is a bf16 one: two roundings, as above."""
+    g = torch.arange(-88.5, -80.0, 0.5, device=device)[:16].to(torch.bfloat16)
+    gu = torch.cat([g, torch.ones_like(g)]).view(1, 32)
+    got = pk.silu_mul(gu)[0].double()
+    want = g.double() * torch.sigmoid(g.double())
+    assert (got != 0).all()
+    # (and fp32's exponential of 128 log2 units: 128 * 2^-24 * ln 2 of the value)
+    assert ((got - want).abs() <= (U[torch.bfloat16] * 2.01 + 1e-5) * want.abs()).all()
