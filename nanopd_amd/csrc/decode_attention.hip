@@ -1895,22 +1895,31 @@ int dispatch_fp8(int g, const DecodeArgs& a, int64_t units, hipStream_t st) {
 // Generic path: any head dim (a multiple of 8 from 32 to 256), block size and
 // batch; a wave's lanes per token row are the next power of two above D / 8.
 // Four waves per partition where that measured faster than one (us, one /
-// four, 32 / 8 heads unless given): launches of at most 1024 partitions, less
-// than a wave per SIMD (3 sequences of 12 / 2 heads at D 96 42.4 / 20.5), more
-// than 16 chunks per row (64 sequences at D 160 237 / 188) and groups above 4
-// heads (200 sequences of 64 / 8 heads at D 96 168 / 155). Not the rest: 64
+// four): launches of at most 1024 partitions of the tables, less than a wave
+// per SIMD (3 sequences of 12 / 2 heads at D 96 42.4 / 20.5). Shapes whose
+// registers leave few waves resident (more than 16 chunks per row, groups above
+// 4 heads) up to 2048 partitions (130 sequences of 64 / 8 heads at D 96, tables
+// of 256 tokens, 43.4 / 35.3), and beyond that while a partition is long enough
+// to share and the units do not fill the chip many times over by themselves (64
+// sequences of 32 / 8 heads at D 160 on up to 4096 tokens 241 / 197, 260 of 8 /
+// 8 heads on 256 46 / 39; but 400 of 32 / 8 heads on 64 36 / 45, and of 64 / 8
+// at D 96 33.6 / 51.9; 520 of 64 / 8 on 1024 337 / 366). Not the rest: 64
 // sequences at D 96 113 / 117, at D 128 with blocks of 8 119 / 129, 24 at D 96
 // 47.5 / 48.3.
+constexpr int64_t kFewPartitions = 1024, kManyUnits = 4096;
+constexpr int kSharedTokens = 256;
 template <class TT, int LPT, int G>
 void launch_partitions(const DecodeArgs& a, int64_t units, hipStream_t st) {
   const dim3 grid((unsigned)units, (unsigned)a.max_parts);
-  if constexpr (LPT <= 16 && G <= 4) {
-    if (units * a.max_parts > 1024) {
-      hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 1>), grid, dim3(64), 0, st, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 4>), grid, dim3(256), 0, st, a);
+  constexpr bool kHeavy = LPT > 16 || G > 4;
+  const int64_t parts = units * a.max_parts;
+  const bool four = parts <= (kHeavy ? 2 * kFewPartitions : kFewPartitions) ||
+                    (kHeavy && units < kManyUnits &&
+                     (int64_t)a.max_bps * a.block_size >= kSharedTokens);
+  if (four)
+    hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 4>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((decode_partition_kernel<TT, LPT, G, 1>), grid, dim3(64), 0, st, a);
 }
 
 template <class TT, int G>

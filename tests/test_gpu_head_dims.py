@@ -209,3 +209,26 @@ def test_decode_generic_waves_per_partition(device, dtype, hd, G, S):
         want = torch.einsum("kgn,nkd->kgd", sc.softmax(-1), v).reshape(kvh * G, hd)
         got = out[s].double().cpu()
         assert (got - want).abs().max().item() <= (1e-2 if dtype == torch.bfloat16 else 2e-3), (s, n)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hd,G", [(160, 4), (96, 8), (224, 3), (40, 5)])
+def test_decode_generic_one_wave_for_many_short_tables(device, dtype, hd, G):
+    """Long rows and groups above 4 heads with one wave per partition: more than
+    2048 partitions of tables of 64 tokens."""
+    print(f"decode generic one wave D={hd} G={G} dtype={dtype}", flush=True)
+    g = torch.Generator().manual_seed(hd)
+    S, kvh, bs, mb = 520, 4, 16, 4
+    kc = (torch.randn(S * mb, kvh, bs, hd, generator=g) * 0.5).to(dtype)
+    vc = (torch.randn(S * mb, kvh, bs, hd, generator=g) * 0.5).to(dtype)
+    q = (torch.randn(S, kvh * G, hd, generator=g) * 0.5).to(dtype)
+    bt = torch.randperm(S * mb, generator=g).to(torch.int32).view(S, mb)
+    sl = (torch.arange(S) % 65).to(torch.int32)   # 0 .. 64 tokens
+    out = torch.full_like(q, float("nan")).to(device)
+    pk.paged_attention_forward(out, q.to(device), kc.to(device), vc.to(device), bt.to(device),
+                               sl.to(device), 0.1, bs, mb)
+    k, v = (c[bt.long()].permute(0, 2, 1, 3, 4).reshape(S, kvh, mb * bs, hd).double() for c in (kc, vc))
+    sc = torch.matmul(q.double().view(S, kvh, G, hd), k.transpose(2, 3).contiguous()) * 0.1
+    sc.masked_fill_(torch.arange(mb * bs)[None, None, None] >= sl[:, None, None, None], -math.inf)
+    want = torch.matmul(torch.softmax(sc, -1).nan_to_num(0.0), v).reshape(S, kvh * G, hd)
+    assert (out.double().cpu() - want).abs().max().item() <= (1e-2 if dtype == torch.bfloat16 else 2e-3)
