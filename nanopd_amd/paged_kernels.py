@@ -266,11 +266,26 @@ def _decode_workspace(dev: torch.device, stream: int, need: int, kind: str = "de
         return ws
 
 
+# Sizes are remembered by the ints that they depend on (of a prefill's contexts:
+# the key steps of 64; not its total_q), so that the steps of one engine mostly
+# find theirs.
 @functools.lru_cache(maxsize=1024)
-def attention_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
-                              block_size: int, max_num_blocks_per_seq: int) -> int:
+def _attention_ws(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
+                  block_size: int, max_num_blocks_per_seq: int) -> int:
     return int(_lib.load().npd_paged_attention_workspace_size(
         num_seqs, num_heads, num_kv_heads, head_dim, block_size, max_num_blocks_per_seq))
+
+
+@functools.lru_cache(maxsize=1024)
+def _prefill_ws(num_seqs: int, num_heads: int, head_dim: int, max_q_len: int, steps: int) -> int:
+    return int(_lib.load().npd_paged_prefill_workspace_size(
+        num_seqs, 0, num_heads, head_dim, max_q_len, steps * 64))
+
+
+def attention_workspace_bytes(num_seqs: int, num_heads: int, num_kv_heads: int, head_dim: int,
+                              block_size: int, max_num_blocks_per_seq: int) -> int:
+    return _attention_ws(int(num_seqs), int(num_heads), int(num_kv_heads), int(head_dim),
+                         int(block_size), int(max_num_blocks_per_seq))
 
 
 def paged_attention_forward(out: torch.Tensor, query: torch.Tensor, key_cache: torch.Tensor,
@@ -322,7 +337,7 @@ def paged_attention_forward(out: torch.Tensor, query: torch.Tensor, key_cache: t
         _fail("head_dim must be the contiguous dim")
     if s == 0:
         return
-    need = attention_workspace_bytes(s, h, kvh, d, bs, mb)
+    need = _attention_ws(s, h, kvh, d, bs, mb)
     stream = _stream(dev)
     ws_ptr = 0
     if need > 0:
@@ -377,7 +392,7 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
         _fail("head_dim must be the contiguous dim")
     if s == 0:
         return
-    need = attention_workspace_bytes(s, h, kvh, d, bs, mb)
+    need = _attention_ws(s, h, kvh, d, bs, mb)
     stream = _stream(dev)
     ws_ptr = 0
     if need > 0:
@@ -397,11 +412,10 @@ def paged_attention_forward_fp8(out: torch.Tensor, query: torch.Tensor, key_cach
 # Chunked prefill attention
 # ---------------------------------------------------------------------------
 
-@functools.lru_cache(maxsize=1024)
 def prefill_workspace_bytes(num_seqs: int, total_q: int, num_heads: int, head_dim: int,
                             max_q_len: int, max_context_len: int) -> int:
-    return int(_lib.load().npd_paged_prefill_workspace_size(
-        num_seqs, total_q, num_heads, head_dim, max_q_len, max_context_len))
+    return _prefill_ws(int(num_seqs), int(num_heads), int(head_dim), int(max_q_len),
+                       (int(max_context_len) + 63) // 64)
 
 
 def _prefill(out, query, key_cache, value_cache, block_tables, cu_seqlens_q, context_lens, scale,
@@ -449,7 +463,7 @@ def _prefill(out, query, key_cache, value_cache, block_tables, cu_seqlens_q, con
     if ns == 0 or tq == 0:
         return
     mctx = int(max_context_len) if max_context_len is not None else mb * bs
-    need = prefill_workspace_bytes(ns, tq, h, d, int(max_q_len), mctx)
+    need = _prefill_ws(ns, h, d, int(max_q_len), (mctx + 63) // 64)
     stream = _stream(dev)
     ws_ptr = 0
     if need > 0:

@@ -235,8 +235,25 @@ def test_prefill_workspace_size():
     assert lib.npd_paged_prefill_workspace_size(4, 2048, 32, 64, 512, 3584) == \
         split(4, 32, 512, 4, D=64)
     assert lib.npd_paged_prefill_workspace_size(4, 2048, 32, 64, 512, 1024) == 0
-    # head dim 256 runs unsplit (prefill_generic_kernel): no workspace
+    # head dim 256 runs unsplit: no workspace
     assert lib.npd_paged_prefill_workspace_size(2, 1024, 32, 256, 512, 32768) == 0
+
+
+def test_remembered_sizes_are_the_library_s():
+    """The Python layer remembers workspace sizes by what they depend on: equal
+    to the library's for every context of a step of 64 keys, whatever total_q."""
+    lib = _lib.load()
+    for S, H, D, mq in ((1, 32, 128, 512), (7, 12, 64, 33), (3, 16, 256, 100), (2, 8, 96, 64)):
+        for ctx in (0, 1, 63, 64, 65, 1024, 1025, 1088, 1089, 5000, 100000):
+            for tq in (0, 1, S * mq):
+                assert pk.prefill_workspace_bytes(S, tq, H, D, mq, ctx) == \
+                    lib.npd_paged_prefill_workspace_size(S, tq, H, D, mq, ctx), (S, D, ctx)
+    n = torch.tensor(3)   # remembered by value, not by the object
+    first = pk.attention_workspace_bytes(n, 32, 8, 128, 16, 256)
+    n += 5
+    assert first == lib.npd_paged_attention_workspace_size(3, 32, 8, 128, 16, 256)
+    assert pk.attention_workspace_bytes(n, 32, 8, 128, 16, 256) == \
+        lib.npd_paged_attention_workspace_size(8, 32, 8, 128, 16, 256) != first
 
 
 def test_python_mirror_raises_like_torch_check():
