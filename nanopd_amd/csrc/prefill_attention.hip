@@ -402,11 +402,11 @@ constexpr int swz8() { return D == 64 ? 32 : 16; }
 // lds .. lds + 1023, lane i at lds + 16 i. Counts in vmcnt; the caller waits.
 __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t off, const void* base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds), "v"(off), "s"(base) : "memory");
+               :: "s"(lds), "v"(off), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* p) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(lds), "v"(p) : "memory");
+               :: "s"(lds), "v"(p) : "memory", "m0");
 }
 // All but the last L LDS accesses of this wave are done and at most N of its
 // direct-to-LDS loads are still in flight; then the workgroup's barrier.
