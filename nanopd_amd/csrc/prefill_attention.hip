@@ -117,6 +117,7 @@ struct PrefillArgs {
   int tiles_max, subtiles, splits_max;   // subtiles: 32-row subtiles per (sequence, kv head)
   int ks_steps;                          // key steps per split (fixed order)
   int max_items;                         // items per kv head the grid has room for
+  int even_items;                        // ... to be used where no tile outlasts the mean load
   int num_cus;                           // compute units of the device (work-list sizing)
   float scale_log2;
   int64_t q_stride_token, q_stride_head, out_stride_token, out_stride_head;
@@ -264,18 +265,21 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
     // a few steps), ks = nmax / p for the p whose estimated time is least: the
     // longest item where one round of the compute units takes them all, else
     // their mean load plus a share of the longest item (what a greedy
-    // longest-first order leaves uneven; less with every further round). An
-    // item costs kItemSteps steps on top of its own, one that publishes and
-    // merges kMergeSteps more. Over 500 random batches of 1-6 chunks this ends
-    // within 0.2% of the best p's greedy schedule on average. Three rounds of
-    // whole tiles are not cut.
+    // longest-first order leaves uneven; less with every further round, none
+    // from three on). An item costs kItemSteps steps on top of its own, one that
+    // publishes and merges kMergeSteps more. Three rounds of whole tiles are not
+    // cut, unless the longest outlasts the mean load: one long prefix among many
+    // prompts ends the launch by itself (12 chunks of 512 tokens of 32 / 8
+    // heads, one on a prefix of 100000: 2050 us whole, 787 cut).
     auto nsp_of = [&](int k, int step) {
       const int p = small_div(n[k] + step - 1, step);
       return !valid[k] ? 0 : (p < 1 ? 1 : (p > a.splits_max ? a.splits_max : p));
     };
     int ks = nmax < 1 ? 1 : nmax;
     const int units = a.num_cus < per_item ? 1 : small_div(a.num_cus, per_item);
-    if (a.splits_max > 1 && ntiles < 3 * units) {
+    const bool tail = (float)(nmax + kItemSteps) * units > (float)tot + (float)(ntiles * kItemSteps);
+    if (a.splits_max > 1 && (ntiles < 3 * units || tail)) {
+      const int room = tail ? a.max_items : a.even_items;
       float best = 0.f;
       for (int p = 1; p <= a.splits_max; ++p) {
         const int kp = small_div(nmax + p - 1, p);
@@ -288,11 +292,11 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
             sums += npd::wave_sum_i(c + (c > 1 ? c << 16 : 0));
           }
         const int items = sums & 0xffff, cut = sums >> 16;
-        if (p > 1 && items > a.max_items) break;
+        if (p > 1 && items > room) break;
         const float longest = (float)(kp + kItemSteps + (p > 1 ? kMergeSteps : 0));
         const float mean = (float)(tot + items * kItemSteps + cut * kMergeSteps) / units;
         const float est = items <= units ? longest
-                                         : fmaxf(longest, mean + 0.35f * longest * (3 * units - items) / (2 * units));
+                                         : fmaxf(longest, mean + 0.35f * longest * max(3 * units - items, 0) / (2 * units));
         if (p == 1 || est < 0.97f * best) best = est, ks = kp < 1 ? 1 : kp;
       }
     }
@@ -1356,18 +1360,35 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   if (L.total > 0 && num_seqs * tiles * num_kv_heads > kMaxCounters)
     return fail(NPD_E_INVALID, "%s: too many query tiles for the %lld merge counters", name,
                 (long long)kMaxCounters);
+  // Whether the longest context there can be outlasts the mean load of a
+  // compute unit, as far as the host can tell: total_q rows make no fewer than
+  // `rows` tiles, whose steps are least where all chunks are alike and without
+  // a prefix.
+  const int kt = kKT;
+  const int64_t longest = (max_context_len + kt - 1) / kt, rows = total_q * g / tr;
+  const bool tail = (longest + kItemSteps) * device_cus() >
+                    rows * num_kv_heads * (kItemSteps + total_q / num_seqs / (2 * kt));
   // Up to kListTiles (sequence, tile) pairs the kernel cuts key ranges by the
   // work it finds. More run whole, in a fixed order, unless they leave compute
-  // units idle (many short chunks on long prefixes).
+  // units idle (many short chunks on long prefixes) or one may end the launch
+  // by itself (700 chunks of 60 tokens and one of 256 on a prefix of 32512:
+  // 1630 us whole, 1510 cut).
   const bool list = num_seqs * tiles <= kListTiles;
-  const bool whole = !list && total_q * num_heads >= 2LL * device_cus() * tr;
+  const bool whole = !list && !tail && total_q * num_heads >= 2LL * device_cus() * tr;
   const int splits = whole ? 1 : L.splits;
-  // Grid: the tiles there can be, or two rounds of the compute units where the kernel may cut that many parts;
-  // a workgroup without an item ends after the work list.
+  // Grid: the tiles there can be, or two rounds of the compute units where the
+  // kernel may cut that many parts; a workgroup without an item ends after the
+  // work list. Where one of several sequences may outlast the others, its parts
+  // have a further round (parts no shorter than the mean load are no more; with
+  // two or three rounds of room the greedy schedules of 400 random skewed
+  // batches end no sooner).
   const int64_t whole_tiles = tiles_of(tr);
+  const int64_t round = (device_cus() + num_kv_heads - 1) / num_kv_heads;
   const int64_t two_rounds = (2LL * device_cus() + num_kv_heads - 1) / num_kv_heads;
-  const int64_t max_items = !list ? splits * num_seqs * tiles
-                            : splits > 1 && whole_tiles < two_rounds ? two_rounds : whole_tiles;
+  const int64_t even_items = !list ? splits * num_seqs * tiles
+                             : splits > 1 && whole_tiles < two_rounds ? two_rounds : whole_tiles;
+  const int64_t max_items = list && tail && splits > 1 && num_seqs > 1 && whole_tiles + round > even_items
+                                ? whole_tiles + round : even_items;
   const int64_t grid = max_items * num_kv_heads;
   if (grid > INT32_MAX) return fail(NPD_E_INVALID, "%s: too many tiles", name);
 
@@ -1397,6 +1418,7 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   a.splits_max = splits;
   a.ks_steps = L.ks_steps;
   a.max_items = (int)max_items;
+  a.even_items = (int)even_items;
   a.num_cus = device_cus();
   a.scale_log2 = scale * kLog2e;
   a.q_stride_token = q_stride_token;

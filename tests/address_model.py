@@ -564,6 +564,7 @@ class PrefillLaunch:
     total: int = 0
     grid: int = 0
     max_items: int = 0
+    even_items: int = 0
     subtiles: int = 0
     num_cus: int = 256
     waves: int = 8       # per workgroup
@@ -575,18 +576,23 @@ class PrefillLaunch:
 
 
 def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
-                 D: int = 128, total_q: int | None = None, waves: int = 8) -> PrefillLaunch:
+                 D: int = 128, total_q: int | None = None,
+                 waves: int | None = None) -> PrefillLaunch:
     """prefill_layout and prefill_impl (prefill_attention.hip), head dims 64,
-    128 and 256 (prefill_kernel). total_q: S * max_q_len unless given; waves:
-    per workgroup, 8, or 4 (head dim 256, and 128 where 256-row tiles take half
-    the compute units at most)."""
+    128 and 256 (prefill_kernel). total_q: S * max_q_len unless given; waves per
+    workgroup: the library's choice unless given -- 8, or 4 (head dim 256, and
+    128 where 256-row tiles take half the compute units at most)."""
     assert D in (64, 128, 256)
-    if D == 256:
-        waves = 4
-    L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus, waves=waves,
-                      kt=KT)
     g = H // KV
     tq = S * max_q_len if total_q is None else total_q
+
+    def tiles_of(tr):
+        return min(S * _ceil(max_q_len * g, tr), tq * g // tr + S)
+    if waves is None:
+        few = tiles_of(8 * WAVE_ROWS) * KV * 2 <= num_cus
+        waves = 4 if D == 256 or (D == 128 and few) else 8
+    L = PrefillLaunch(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=num_cus, waves=waves,
+                      kt=KT)
     if D == 256:
         L.ks_steps = 1 << 30   # whole key ranges
     elif max_ctx > 0:
@@ -606,14 +612,20 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
     L.tiles = _ceil(max_q_len * g, L.rows)
     L.subtiles = L.tiles * L.waves
     in_list = S * L.tiles <= LIST_TILES
-    if not in_list and tq * H >= 2 * num_cus * L.rows:
+    # the longest context there can be against the mean load of a compute unit
+    tail = (_ceil(max_ctx, KT) + ITEM_STEPS) * num_cus > \
+        tq * g // L.rows * KV * (ITEM_STEPS + tq // max(S, 1) // (2 * KT))
+    if not in_list and not tail and tq * H >= 2 * num_cus * L.rows:
         L.splits = 1
-    whole = min(S * L.tiles, tq * g // L.rows + S)
+    whole = tiles_of(L.rows)
     two = _ceil(2 * num_cus, KV)
     if not in_list:
-        L.max_items = L.splits * S * L.tiles
+        L.even_items = L.splits * S * L.tiles
     else:
-        L.max_items = two if L.splits > 1 and whole < two else whole
+        L.even_items = two if L.splits > 1 and whole < two else whole
+    L.max_items = L.even_items
+    if in_list and tail and L.splits > 1 and S > 1:
+        L.max_items = max(L.even_items, whole + _ceil(num_cus, KV))
     L.grid = L.max_items * KV
     return L
 
@@ -648,20 +660,22 @@ def prefill_items(L: PrefillLaunch, cu: np.ndarray, ctx_lens: np.ndarray):
 
         ks = max(nmax, 1)
         units = max(L.num_cus // L.KV, 1)
-        if L.splits > 1 and ntiles < 3 * units:
+        tail = (nmax + ITEM_STEPS) * units > tot + ntiles * ITEM_STEPS
+        if L.splits > 1 and (ntiles < 3 * units or tail):
             best = 0.0
+            room = L.max_items if tail else L.even_items
             for p in range(1, L.splits + 1):
                 kp = _ceil(nmax, p)
                 if p > 1 and kp < MIN_PART:
                     break
                 c = cut_of(max(kp, 1))
                 cnt, cut = int(c.sum()), int(c[c > 1].sum())
-                if p > 1 and cnt > L.max_items:
+                if p > 1 and cnt > room:
                     break
                 longest = kp + ITEM_STEPS + (MERGE_STEPS if p > 1 else 0)
                 mean = (tot + cnt * ITEM_STEPS + cut * MERGE_STEPS) / units
                 est = longest if cnt <= units else max(
-                    longest, mean + 0.35 * longest * (3 * units - cnt) / (2 * units))
+                    longest, mean + 0.35 * longest * max(3 * units - cnt, 0) / (2 * units))
                 if p == 1 or est < 0.97 * best:
                     best, ks = est, max(kp, 1)
         cut = cut_of(ks)
@@ -775,7 +789,8 @@ def prefill_generic(W: Writes, S: int, H: int, KV: int, bs: int, max_bps: int, n
                     max_q_len: int, out: Buf, cu: np.ndarray, ctx_lens: np.ndarray,
                     out_stride_token: int, out_stride_head: int, tables: np.ndarray,
                     D: int) -> None:
-    """prefill_generic_kernel (head dim 256): one workgroup per
+    """prefill_generic_kernel (the other head dims, and 256 over an FP8 pool):
+    one workgroup per
     (sequence, head, 64-row tile), grouped by (sequence, kv head) on one XCD;
     every K/V row it reads and every output row it writes."""
     tiles = _ceil(max_q_len, 64)

@@ -161,7 +161,7 @@ def check_eager_step(W, pre, decs, fp8):
                BS, H * D, fp8)
     max_sl = max(q + c for q, c, _ in seqs)
     if pre:
-        L = A.prefill_host(1, H, KV, BS, mb, tp, max_sl)
+        L = A.prefill_host(1, H, KV, BS, mb, tp, max_sl, total_q=tp)
         ws = A.Buf("prefill workspace", _prefill_ws(1, tp, tp, max_sl))
         assert ws.nbytes == L.total
         A.prefill(W, L, A.Buf("attn[:tp]", tp * H * D * 2), ws, np.array([0, tp]),
@@ -205,7 +205,7 @@ def test_configs_1_to_4_and_large_batches():
     pre = [0, 512, 1536, 3072]
     cu = np.array([0, 512, 1024, 1536, 2048])
     ctx = np.array([p + 512 for p in pre])
-    L = A.prefill_host(4, H, KV, BS, 224, 512, 3584)
+    L = A.prefill_host(4, H, KV, BS, 224, 512, 3584, total_q=2048)
     A.prefill(W, L, A.Buf("out", 2048 * H * D * 2), A.Buf("ws", _prefill_ws(4, 2048, 512, 3584)),
               cu, ctx, H * D, D)
     # a wide batch of prefills (fixed-grid path): 70 chunks of 1..300 rows
@@ -213,13 +213,13 @@ def test_configs_1_to_4_and_large_batches():
     cu = np.concatenate([[0], np.cumsum(q)])
     c = q + rng.integers(0, 3000, 70)
     mb = int((c.max() + BS - 1) // BS)
-    L = A.prefill_host(70, H, KV, BS, mb, int(q.max()), int(c.max()))
+    L = A.prefill_host(70, H, KV, BS, mb, int(q.max()), int(c.max()), total_q=int(cu[-1]))
     assert 70 * L.tiles > 64
     A.prefill(W, L, A.Buf("out", int(cu[-1]) * H * D * 2),
               A.Buf("ws", _prefill_ws(70, int(cu[-1]), int(q.max()), int(c.max()))), cu, c, H * D, D)
     # other head groupings of prefill (G = 6 -> 2 heads per workgroup, G = 1)
     for h, kv in ((12, 2), (8, 8)):
-        L = A.prefill_host(2, h, kv, BS, 64, 300, 1000)
+        L = A.prefill_host(2, h, kv, BS, 64, 300, 1000, total_q=600)
         A.prefill(W, L, A.Buf("out", 600 * h * D * 2),
                   A.Buf("ws", _prefill_ws(2, 600, 300, 1000, h=h)), np.array([0, 300, 600]),
                   np.array([1000, 300]), h * D, D)
@@ -272,7 +272,7 @@ def test_planted_mistakes_are_reported():
         W.check()
     # a prefill output one token short
     W = A.Writes()
-    L = A.prefill_host(1, H, KV, BS, 64, 512, 1024)
+    L = A.prefill_host(1, H, KV, BS, 64, 512, 1024, total_q=512)
     A.prefill(W, L, A.Buf("out", 511 * H * D * 2), A.Buf("ws", _prefill_ws(1, 512, 512, 1024)),
               np.array([0, 512]), np.array([1024]), H * D, D)
     with pytest.raises(A.OutOfBounds, match="prefill output"):
@@ -290,7 +290,7 @@ def test_head_dims_64_and_256():
     """The fused prologue (4, 8 or 16 lanes a row, eight rotate-half pairs
     per lane at D 256) and prefill at those head dims (prefill_kernel at 64,
     with its partials in the workspace the library sizes; the generic kernel
-    at 256): every K/V row read and every store inside its buffer, over
+    at 256, which an FP8 pool runs there): every K/V row read and every store inside its buffer, over
     ragged chunks on paged prefixes, an empty chunk, a chunk longer than its
     context (rows before position 0) and block tables at their full width; a
     planted wrong row stride is caught."""
@@ -313,7 +313,7 @@ def test_head_dims_64_and_256():
         out = A.Buf("out", int(cu[-1]) * h * d * 2)
         if d == 64:
             mctx = int(ctx.max())
-            L = A.prefill_host(len(q), h, kv, bs, mb, int(q.max()), mctx, D=d)
+            L = A.prefill_host(len(q), h, kv, bs, mb, int(q.max()), mctx, D=d, total_q=int(cu[-1]))
             ws_bytes = int(_lib.load().npd_paged_prefill_workspace_size(
                 len(q), int(cu[-1]), h, d, int(q.max()), mctx))
             assert ws_bytes == L.total > 0
@@ -335,7 +335,7 @@ def test_head_dims_64_and_256():
 @pytest.mark.parametrize("S,H,KV,mq", [(4, 32, 8, 512), (3, 12, 2, 130), (5, 6, 1, 64),
                                         (1, 16, 16, 700), (64, 8, 2, 65), (70, 4, 4, 64)])
 def test_prefill_generic_grid_covers_every_tile_once(S, H, KV, mq):
-    """Head dim 256: the XCD-grouped grid of prefill_generic_kernel runs every
+    """The XCD-grouped grid of prefill_generic_kernel runs every
     (sequence, 64-row tile, query head) exactly once (tied and clamped
     contexts included), the workgroups of one (sequence, kv head) all go to
     one XCD, and up to 64 sequences start longest context first."""
@@ -399,10 +399,10 @@ def test_prefill_work_list_covers_every_part_once(case):
     cu = np.concatenate([[0], np.cumsum(q)])
     ctx = np.array(q) + np.array(p)
     max_bps = int(np.ceil(ctx.max() / BS))
-    L = A.prefill_host(S, h, kv, BS, max_bps, max(q), int(ctx.max()))
+    L = A.prefill_host(S, h, kv, BS, max_bps, max(q), int(ctx.max()), total_q=int(cu[-1]))
     assert L.S * L.tiles <= 64
     items = [it for it in A.prefill_items(L, cu, ctx) if it is not None]
-    TR = 64 * L.rt
+    TR = L.rows // (h // kv)
     seen = set()
     parts = {}
     for s, t, j, kh, hg, q0, qlen, cx, ks, eq in items:
@@ -478,3 +478,38 @@ def test_prefill_tiles_of_flattened_rows(hd, waves):
         rows = {(s, t, kh) for s, t, _, kh in tiles}
         assert rows == {(s, t, kh) for s in range(S) for kh in range(kv)
                         for t in range(-(-int(q[s]) * g // L.rows))}
+
+
+@pytest.mark.parametrize("q,prefix", [
+    ([512] * 12, [0] * 11 + [100000]),            # one long document among fresh prompts
+    ([1024] * 7 + [64], [0] * 7 + [131072]),
+    ([60] * 100 + [256], [0] * 100 + [32512]),    # more than three rounds of tiles
+    ([700] * 30 + [300], [500] * 30 + [60000]),   # 341 (sequence, tile) pairs
+    ([60] * 700 + [256], [0] * 700 + [32512]),    # past the work list: the fixed order
+])
+def test_a_long_tile_in_a_full_launch_is_cut(q, prefix):
+    """32 / 8 heads on 256 compute units: where one sequence's tiles outlast the
+    mean load of a unit they run in parts, as long as the mean load or an eighth
+    of the tile (the most parts there are) within 1.3, and every part once."""
+    q, ctx = np.array(q), np.array(q) + np.array(prefix)
+    cu = np.concatenate([[0], np.cumsum(q)])
+    L = A.prefill_host(len(q), H, KV, BS, int(-(-ctx.max() // BS)), int(q.max()), int(ctx.max()),
+                       total_q=int(cu[-1]))
+    items = A.prefill_items(L, cu, ctx)
+    assert None not in items
+    units, steps, parts, longest = L.num_cus // KV, {}, {}, 0
+    for s, t, j, kh, _, q0, qlen, cx, ks, _ in items:
+        n = -(-A.tile_keys(L, H // KV, t, qlen, cx) // A.KT)
+        nsp = min(max(-(-n // ks), 1), L.splits)
+        if j >= nsp:
+            continue   # (the fixed order's workgroups of parts that are not there)
+        assert j not in parts.setdefault((s, t, kh), set())
+        parts[(s, t, kh)].add(j)
+        steps[(s, t)] = n
+        longest = max(longest, -(-n // nsp))
+    assert len(parts) == KV * sum(-(-int(x) * (H // KV) // L.rows) for x in q)
+    for (s, t, _), js in parts.items():
+        assert js == set(range(len(js)))
+    mean, nmax = sum(steps.values()) / units, max(steps.values())
+    assert nmax > 1.3 * mean   # whole tiles would be the launch
+    assert longest <= 1.3 * max(mean, nmax / 8)
