@@ -116,6 +116,7 @@ struct PrefillArgs {
   int num_seqs, num_kv_heads, group, block_size, bs_shift, num_blocks, max_bps;
   int tiles_max, subtiles, splits_max;   // subtiles: 32-row subtiles per (sequence, kv head)
   int ks_steps;                          // key steps per split (fixed order)
+  bool list;                             // items by the work list (else in the fixed order)
   int max_items;                         // items per kv head the grid has room for
   int even_items;                        // ... to be used where no tile outlasts the mean load
   int num_cus;                           // compute units of the device (work-list sizing)
@@ -226,7 +227,7 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
   const int cap = a.max_bps * a.block_size;
   const int per_item = a.num_kv_heads;   // workgroups per (sequence, tile, part)
   const int tiles = a.num_seqs * a.tiles_max;
-  if (tiles <= kListTiles) {
+  if (a.list) {
     // Work list in longest-processing-time order, derived from the sequence
     // lengths. Slot (k, lane) stands for tile index i = 64 k +
     // lane: sequence i / tiles_max, tile i % tiles_max, n key steps. The
@@ -256,10 +257,14 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
         cx[k] = cx[k] < 0 ? 0 : (cx[k] < cap ? cx[k] : cap);
         valid[k] = valid[k] && lt * TR < ql[k] * a.group;
         if (valid[k]) n[k] = (tile_keys<TR>(a, lt, ql[k], cx[k]) + KT - 1) / KT;
-        tot += npd::wave_sum_i(n[k]);   // DPP, wave-uniform
-        nmax = max(nmax, npd::wave_max_i(n[k]));
+        tot += n[k];
+        nmax = max(nmax, n[k]);
         ntiles += __popcll(__ballot(valid[k]));
       }
+    // a lane adds up its slots before the wave does: one DPP reduction, not one
+    // per slot row (300 chunks of 60 tokens of 32 / 8 heads 264 -> 246 us)
+    tot = npd::wave_sum_i(tot);   // wave-uniform
+    nmax = npd::wave_max_i(nmax);
     // Parts per tile: a tile of n steps runs as nsp = ceil(n / ks) near-equal
     // parts (a short tail part would pay a whole item's prologue and merge for
     // a few steps), ks = nmax / p for the p whose estimated time is least: the
@@ -289,8 +294,9 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
         for (int k = 0; k < kSlots; ++k)
           if (64 * k < tiles) {
             const int c = nsp_of(k, kp < 1 ? 1 : kp);
-            sums += npd::wave_sum_i(c + (c > 1 ? c << 16 : 0));
+            sums += c + (c > 1 ? c << 16 : 0);
           }
+        sums = npd::wave_sum_i(sums);
         const int items = sums & 0xffff, cut = sums >> 16;
         if (p > 1 && items > room) break;
         const float longest = (float)(kp + kItemSteps + (p > 1 ? kMergeSteps : 0));
@@ -310,17 +316,18 @@ __device__ __forceinline__ bool prefill_item(const PrefillArgs& a, int lane, Ite
       if (64 * k < tiles) {
         cut[k] = nsp_of(k, ks);
         if (valid[k]) len[k] = small_div(n[k] + cut[k] - 1, cut[k]);
-        lenmax = max(lenmax, npd::wave_max_i(len[k]));
+        lenmax = max(lenmax, len[k]);
       }
     }
+    lenmax = npd::wave_max_i(lenmax);
     // items in buckets >= b, non-increasing in b; item id is in the last
     // bucket b with from(b) > id (binary search over DPP wave sums)
     auto from = [&](int b) -> int {
       int c = 0;
 #pragma unroll
       for (int k = 0; k < kSlots; ++k)
-        if (64 * k < tiles) c += npd::wave_sum_i(len[k] >= b ? cut[k] : 0);
-      return c * per_item;
+        if (64 * k < tiles) c += len[k] >= b ? cut[k] : 0;
+      return npd::wave_sum_i(c) * per_item;
     };
     int id = blockIdx.x;
     if (id >= from(0)) return false;   // past the last item
@@ -1373,7 +1380,13 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   // units idle (many short chunks on long prefixes) or one may end the launch
   // by itself (700 chunks of 60 tokens and one of 256 on a prefix of 32512:
   // 1630 us whole, 1510 cut).
-  const bool list = num_seqs * tiles <= kListTiles;
+  // Three rounds or more of tiles that cannot be cut and are nearly all there
+  // need no list either, which costs an item 2 us and more (16 chunks of 512
+  // tokens of 32 / 8 heads 150 us by the list, 130 in the fixed order; 300 of 60
+  // tokens 246, 206; 4 of 2048 169, 160).
+  const bool even = L.splits == 1 && num_seqs * tiles * num_kv_heads >= 3LL * device_cus() &&
+                    4 * num_seqs * tiles <= 5 * rows;
+  const bool list = num_seqs * tiles <= kListTiles && !even;
   const bool whole = !list && !tail && total_q * num_heads >= 2LL * device_cus() * tr;
   const int splits = whole ? 1 : L.splits;
   // Grid: the tiles there can be, or two rounds of the compute units where the
@@ -1417,6 +1430,7 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   a.subtiles = (int)(tiles * waves);
   a.splits_max = splits;
   a.ks_steps = L.ks_steps;
+  a.list = list;
   a.max_items = (int)max_items;
   a.even_items = (int)even_items;
   a.num_cus = device_cus();

@@ -565,6 +565,7 @@ class PrefillLaunch:
     grid: int = 0
     max_items: int = 0
     even_items: int = 0
+    work_list: bool = True
     subtiles: int = 0
     num_cus: int = 256
     waves: int = 8       # per workgroup
@@ -611,10 +612,12 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
     L.rt = 4 // g
     L.tiles = _ceil(max_q_len * g, L.rows)
     L.subtiles = L.tiles * L.waves
-    in_list = S * L.tiles <= LIST_TILES
+    rows = tq * g // L.rows
+    even = L.splits == 1 and S * L.tiles * KV >= 3 * num_cus and 4 * S * L.tiles <= 5 * rows
+    in_list = L.work_list = S * L.tiles <= LIST_TILES and not even
     # the longest context there can be against the mean load of a compute unit
     tail = (_ceil(max_ctx, KT) + ITEM_STEPS) * num_cus > \
-        tq * g // L.rows * KV * (ITEM_STEPS + tq // max(S, 1) // (2 * KT))
+        rows * KV * (ITEM_STEPS + tq // max(S, 1) // (2 * KT))
     if not in_list and not tail and tq * H >= 2 * num_cus * L.rows:
         L.splits = 1
     whole = tiles_of(L.rows)
@@ -643,7 +646,7 @@ def prefill_items(L: PrefillLaunch, cu: np.ndarray, ctx_lens: np.ndarray):
     G = L.H // L.KV
     items = []
     tiles = L.S * L.tiles
-    if tiles <= LIST_TILES:
+    if L.work_list:
         n = np.zeros(tiles, np.int64)
         valid = np.zeros(tiles, bool)
         seq = [(int(cu[s]), int(cu[s + 1] - cu[s]), min(max(int(ctx_lens[s]), 0), cap))

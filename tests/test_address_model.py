@@ -513,3 +513,23 @@ def test_a_long_tile_in_a_full_launch_is_cut(q, prefix):
     mean, nmax = sum(steps.values()) / units, max(steps.values())
     assert nmax > 1.3 * mean   # whole tiles would be the launch
     assert longest <= 1.3 * max(mean, nmax / 8)
+
+
+@pytest.mark.parametrize("q,prefix,listed", [
+    ([512] * 16, [500] * 16, False), ([60] * 300, [200] * 300, False),
+    ([512] * 16, [520] * 16, True),             # key ranges that may be cut
+    ([512] + [30] * 60, [0] * 61, True),        # mostly tiles that are not there
+    ([1024] * 4, [0] * 4, True)])               # two rounds
+def test_equal_whole_tiles_run_without_the_list(q, prefix, listed):
+    """32 / 8 heads: three rounds of tiles that cannot be cut and are nearly all
+    there take the fixed order; either way every tile runs once."""
+    q, ctx = np.array(q), np.array(q) + np.array(prefix)
+    cu = np.concatenate([[0], np.cumsum(q)])
+    L = A.prefill_host(len(q), H, KV, BS, int(-(-ctx.max() // BS)), int(q.max()), int(ctx.max()),
+                       total_q=int(cu[-1]))
+    assert L.work_list == listed and L.splits == (2 if prefix[0] == 520 else 1)
+    seen = [it[:4] for it in A.prefill_items(L, cu, ctx)]
+    assert len(set(seen)) == len(seen)
+    assert {(s, t, kh) for s, t, _, kh in seen} == {
+        (s, t, kh) for s in range(len(q)) for kh in range(KV)
+        for t in range(-(-int(q[s]) * (H // KV) // L.rows))}
