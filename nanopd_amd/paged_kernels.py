@@ -711,10 +711,15 @@ def _rows_16(*ts: torch.Tensor) -> bool:
     """Contiguous 2-byte tensors of one dtype and one GPU that start on 16 bytes,
     with whole 16-byte rows, none empty, none to record a gradient for."""
     t0 = ts[0]
-    return (t0.is_cuda and t0.dtype in _DTYPES and t0.numel() > 0
-            and all(t.get_device() == t0.get_device() and t.dtype == t0.dtype and t.is_contiguous()
-                    and t.data_ptr() % 16 == 0 and t.size(-1) % 8 == 0 for t in ts)
-            and not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)))
+    dtype = t0.dtype
+    if not t0.is_cuda or dtype not in _DTYPES or t0.numel() == 0:
+        return False
+    dev, grad = t0.get_device(), torch.is_grad_enabled()
+    for t in ts:
+        if (t.dtype != dtype or t.get_device() != dev or not t.is_contiguous()
+                or t.data_ptr() & 15 or t.size(-1) & 7 or (grad and t.requires_grad)):
+            return False
+    return True
 
 
 def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tensor,
@@ -724,8 +729,9 @@ def add_rms_norm(x: torch.Tensor, delta: torch.Tensor | None, weight: torch.Tens
     2-byte CUDA tensors of up to 8192 columns run as one launch, others as the
     torch operations, which also refuse what does not fit together (the kernel
     reads x.size(1) weights and as many deltas as x has elements)."""
-    if (x.dim() == 2 and x.size(1) <= 8192 and weight.shape == x.shape[1:] and _rows_16(x, weight)
-            and (delta is None or (delta.shape == x.shape and _rows_16(x, delta)))):
+    if (x.dim() == 2 and x.size(1) <= 8192 and weight.shape == x.shape[1:]
+            and (_rows_16(x, weight) if delta is None
+                 else delta.shape == x.shape and _rows_16(x, weight, delta))):
         out = torch.empty_like(x)
         _lib.call("npd_add_rms_norm", out.data_ptr(), x.data_ptr(),
                   None if delta is None else delta.data_ptr(), weight.data_ptr(), x.size(0),
