@@ -752,9 +752,11 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
   //   waves 4-7   softmax(i-1)       QK(i), PV(i-1)
   // Each wave starts its share of tile i + 3 before softmax(i) (over an FP8
   // pool at head dim 64, where the MFMAs are the shorter half and the share is
-  // conversions too, before those of step i: 1684 + 994 tokens 47.5 against
-  // 48.7 us; 2-byte pools gain nothing), in interval 2i at the earliest, into the buffers of K tile i - 1 and V tile i - 2 (4 K, 5 V
-  // buffers), last read in interval 2i - 1. Its share of tile i + 2
+  // conversions too, before those of step i: 32 / 8 heads, 1684 + 994 tokens
+  // 43.0 against 44.5 us, 6000 on a prefix of 2000 314 against 324, 8 chunks of
+  // 200 on 3000 72 against 75, 4 of 1024 in fp16 73.3 against 72.7; 2-byte pools
+  // gain nothing), in interval 2i at the earliest, into the buffers of K tile
+  // i - 1 and V tile i - 2 (4 K, 5 V buffers), last read in interval 2i - 1. Its share of tile i + 2
   // has landed when its softmax(i) is done (interval 2i + 1 or 2i + 2), so the
   // whole tile has when a wave reads its first K operands ahead of step i + 2,
   // at the end of interval 2i + 3 or 2i + 4.

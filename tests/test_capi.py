@@ -239,6 +239,31 @@ def test_prefill_workspace_size():
     assert lib.npd_paged_prefill_workspace_size(2, 1024, 32, 256, 512, 32768) == 0
 
 
+def test_layer_ops_argument_checks():
+    """npd_add_rms_norm and npd_silu_mul refuse, before any launch: dtypes,
+    widths off 8 (the norm: above 8192), null and misaligned pointers, a negative
+    or NaN eps; no rows are a no-op."""
+    lib = _lib.load()
+    norm, silu = lib.npd_add_rms_norm, lib.npd_silu_mul
+    a = 4096   # a 16-byte aligned address that nothing reads
+    assert norm(a, a, a, a, 0, 64, 1e-6, 1, None) == 0 and silu(a, a, 0, 64, 1, None) == 0
+    for args in [(a, a, a, a, 2, 64, 1e-6, 7, None), (a, a, a, a, -1, 64, 1e-6, 1, None),
+                 (a, a, a, a, 2, 0, 1e-6, 1, None), (a, a, a, a, 2, 12, 1e-6, 1, None),
+                 (a, a, a, a, 2, 8200, 1e-6, 1, None), (a, a, a, a, 2, 64, -1e-6, 1, None),
+                 (a, a, a, a, 2, 64, float("nan"), 1, None), (None, a, a, a, 2, 64, 1e-6, 1, None),
+                 (a, None, a, a, 2, 64, 1e-6, 1, None), (a, a, a, None, 2, 64, 1e-6, 1, None),
+                 (a + 8, a, a, a, 2, 64, 1e-6, 1, None), (a, a, a + 2, a, 2, 64, 1e-6, 1, None),
+                 (a, a, a, a + 8, 2, 64, 1e-6, 1, None), (a, a, a, a, 2**31, 64, 1e-6, 1, None)]:
+        assert norm(*args) < 0, args
+        assert b"npd_add_rms_norm" in lib.npd_last_error()
+    for args in [(a, a, 2, 64, 7, None), (a, a, -1, 64, 1, None), (a, a, 2, 0, 1, None),
+                 (a, a, 2, 12, 1, None), (None, a, 2, 64, 1, None), (a, None, 2, 64, 1, None),
+                 (a + 8, a, 2, 64, 1, None), (a, a + 2, 2, 64, 1, None),
+                 (a, a, 2**62, 64, 1, None)]:
+        assert silu(*args) < 0, args
+        assert b"npd_silu_mul" in lib.npd_last_error()
+
+
 def test_remembered_sizes_are_the_library_s():
     """The Python layer remembers workspace sizes by what they depend on: equal
     to the library's for every context of a step of 64 keys, whatever total_q."""

@@ -368,3 +368,88 @@ def test_head_dim_256_rounds_no_more_than_an_exact_maximum(device, dtype, spread
     ratio = math.sqrt(err / emu)
     print(f"head dim 256 {dtype} spread {spread}: error {ratio:.3f} of the emulation's")
     assert ratio <= 1.05
+
+
+def _fp8_pool(kc, vc, ks):
+    """e4m3 bytes of a pool and the values they stand for, in the pool's dtype."""
+    k8, v8 = ((c.float() / ks).clamp(-448, 448).to(torch.float8_e4m3fn) for c in (kc, vc))
+    return k8, v8, (k8.float() * ks).to(kc.dtype), (v8.float() * ks).to(vc.dtype)
+
+
+@pytest.mark.parametrize("hd,fp8", [(64, False), (64, True), (128, True), (256, False)])
+def test_block_list_in_segments_of_every_loop(device, hd, fp8):
+    """Blocks of one token (test_block_list_in_segments above: head dim 128, a
+    2-byte pool) where tiles come from registers, and at head dim 256."""
+    args = make_case(device, [4500, 0], [33, 20], H=4, kvh=1, D=hd, bs=1, seed=hd + fp8)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    if fp8:
+        k8, v8, kc, vc = _fp8_pool(kc, vc, 1 / 16)
+        out, sc = torch.full_like(q, float("nan")), torch.full((1,), 1 / 16, device=device)
+        pk.paged_prefill_attention_fp8(out, q, k8, v8, bt, cu, ctx, 0.1, 1, mb, mq, sc, sc)
+        torch.cuda.synchronize()
+    else:
+        out = run(*args, 0.1)
+    check(out, q, kc, vc, bt, cu, ctx, 0.1)
+
+
+@pytest.mark.parametrize("hd,fp8", [(64, False), (128, False), (128, True), (256, False)])
+def test_pools_past_4_gib(device, hd, fp8):
+    """The gather with 64-bit offsets: the blocks of a small pool at the end of
+    one of more than 4 GiB give the same bits."""
+    kvh, bs = 8, 16
+    args = make_case(device, [700, 0, 130], [100, 70, 1], H=16, kvh=kvh, D=hd, bs=bs, seed=hd)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    sc = torch.full((kvh,), 1 / 16, device=device)
+    if fp8:
+        kc, vc = (c.view(torch.uint8) for c in _fp8_pool(kc, vc, 1 / 16)[:2])
+
+    def attend(k, v, tables):
+        out = torch.full_like(q, float("nan"))
+        if fp8:
+            pk.paged_prefill_attention_fp8(out, q, k, v, tables, cu, ctx, 0.1, bs, mb, mq, sc, sc)
+        else:
+            pk.paged_prefill_attention(out, q, k, v, tables, cu, ctx, 0.1, bs, mb, mq)
+        return out
+
+    want = attend(kc, vc, bt)
+    n = kc.size(0)
+    total = (1 << 32) // (kvh * bs * hd * kc.element_size()) + 2 * n
+    big = [torch.empty(total, kvh, bs, hd, dtype=kc.dtype, device=device) for _ in range(2)]
+    for b, c in zip(big, (kc, vc)):
+        b[total - n:] = c
+    got = attend(*big, bt + (total - n))
+    torch.cuda.synchronize()
+    assert big[0].numel() * big[0].element_size() > 1 << 32
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+def test_equal_tiles_in_the_fixed_order(device):
+    """110 chunks of 58 to 64 tokens of 32 / 8 heads: three rounds of tiles that
+    cannot be cut and are all there, in the fixed order."""
+    rng = np.random.default_rng(2)
+    chunks = [64] + [int(x) for x in rng.integers(58, 65, 109)]
+    args = make_case(device, [int(x) for x in rng.integers(0, 200, 110)], chunks, seed=2)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    out = torch.full_like(q, float("nan"))
+    pk.paged_prefill_attention(out, q, kc, vc, bt, cu, ctx, 0.1, 16, mb, mq, int(ctx.max()))
+    torch.cuda.synchronize()
+    check(out, q, kc, vc, bt, cu, ctx, 0.1)
+
+
+@pytest.mark.parametrize("S,chunk,prefix", [(30, 512, 30000), (220, 60, 20000), (150, 60, 20000)])
+def test_one_long_prefix_in_a_full_launch(device, S, chunk, prefix):
+    """One chunk of 40 tokens on a long prefix among many prompts: its tile is cut
+    where three rounds of whole tiles are not (30 x 8 and 220 x 1 (sequence, tile)
+    pairs by the list), and, with one chunk of 300 more (150 x 5), in the fixed
+    order."""
+    chunks = [chunk] * (S - 2) + [300 if S == 150 else chunk, 40]
+    args = make_case(device, [0] * (S - 1) + [prefix], chunks, H=16, kvh=4, seed=S)
+    q, kc, vc, bt, cu, ctx, mb, mq = args
+    out = torch.full_like(q, float("nan"))
+    pk.paged_prefill_attention(out, q, kc, vc, bt, cu, ctx, 0.1, 16, mb, mq, int(ctx.max()))
+    torch.cuda.synchronize()
+    first, last = int(cu[-2]), int(cu[-1])
+    check(out[first:last], q[first:last], kc, vc, bt[-1:], cu[-2:] - cu[-2], ctx[-1:], 0.1)
+    few = int(cu[4])
+    check(out[:few], q[:few], kc, vc, bt[:4], cu[:5], ctx[:4], 0.1)
+    assert torch.isfinite(out).all()
