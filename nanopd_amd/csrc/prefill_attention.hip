@@ -17,8 +17,8 @@
 //   (no key parts) and for few tiles at 128.
 //   Rows are (token, head) pairs of the kv head's G query heads, flattened as
 //   token * G + head: any G fills its tiles, and a wave's 32 rows span 32 / G
-//   tokens, so its causal range ends with the tile's. With 8
-//   waves, two share a SIMD, 256 VGPRs each. All 8 waves read the 64-key K/V tiles that the workgroup
+//   tokens, so its causal range ends with the tile's. With 8 waves, two share a
+//   SIMD, 256 VGPRs each. All waves read the 64-key K/V tiles that the workgroup
 //   gathers from the pool into LDS (GQA and row reuse).
 //   per step of 64 keys, each wave:
 //     S^T = K . Q^T   -- A = K rows from LDS, B = the wave's query rows, kept
@@ -29,7 +29,8 @@
 //                        with (1, 1). No maximum is taken in the usual step:
 //                        whether the reference must move is read off the packed
 //                        P values or their sum (Bound), and only then the
-//                        maxima are taken, O rescaled and P formed again;
+//                        maxima are taken, O rescaled and P formed again (head
+//                        dim 256: the maximum of every step, kExactMax);
 //     O^T += V^T . P^T -- P^T is the S^T accumulator, already in B-operand
 //                        layout (packed with v_cvt_pk_bf16_f32); V stays
 //                        row-major in LDS like K, and the V^T A operand is two
@@ -47,12 +48,12 @@
 //
 // What bounds it: power, then issue. 12000 tokens of 32 / 8 heads run at 3009
 // cycles per step against 2048 of MFMA, at 1.8 GHz (all-zero inputs, which draw
-// less, hold 2.4 GHz and take 0.76x the time): 1071 us = 1.10 PFLOP/s of useful
-// work, where a plain 8192^3 product reaches 1.47. Before (16x16x32 MFMAs, K/V
-// through a register ring, maxima in every step): 1383 us. A step without the
-// tile loads takes the same cycles at a higher clock; more operand reads ahead
-// (6 to 12) change nothing; the dot2 row sums cost 11 cycles each under the
-// other wave's MFMAs, 4 alone.
+// less, hold 2.4 GHz and take 0.76x the time): 1027 to 1071 us over several
+// boxes = 1.10 to 1.15 PFLOP/s of useful work, where a plain 8192^3 product
+// reaches 1.47. Before (16x16x32 MFMAs, K/V through a register ring, maxima in
+// every step): 1328 to 1383 us. A step without the tile loads takes the same
+// cycles at a higher clock; more operand reads ahead (6 to 12) change nothing;
+// the dot2 row sums cost 11 cycles each under the other wave's MFMAs, 4 alone.
 //
 // Key splits: tiles are cut into nsp <= splits_max near-equal key parts run by
 // separate workgroups where that shortens the launch (prefill_item; in the
@@ -468,7 +469,10 @@ __global__ __launch_bounds__(64 * NW) void prefill_kernel(PrefillArgs a) {
   const int hf = lane >> 5, c32 = lane & 31;
 
   // The first wave derives the item: eight waves sharing the SIMDs for the same
-  // answer took 5.1 us where this takes 4.4 (32 tiles, four part counts tried).
+  // answer took 5.1 us where this takes 4.4 (32 tiles, four part counts tried;
+  // 3 us where none is, 1.1 in the fixed order). Block ids, queries and the
+  // first tiles follow one after another in 4 us; asking for the block ids ahead
+  // of the queries gave nothing and cost FP8 pools 15%.
   if (wave == 0) {
     Item it{};
     it.nsp = 0;
