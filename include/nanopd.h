@@ -208,8 +208,9 @@ int64_t npd_paged_prefill_workspace_size(int64_t num_seqs, int64_t total_q,
  * Rows with p < 0 (context shorter than the chunk) get zeros. scale must be
  * positive and finite.
  * max_q_len: host-known upper bound on the chunk lengths (grid size).
- * head_dim: a multiple of 32 from 32 to 256 (64 and 128 have the tuned
- * kernel; the reference's SDPA takes any, nanoPD/engine/model_runner.py:166-168).
+ * head_dim: a multiple of 32 from 32 to 256 (64, 128 and, over 2-byte pools,
+ * 256 have the tuned kernel; the reference's SDPA takes any,
+ * nanoPD/engine/model_runner.py:166-168).
  * max_context_len: host-known upper bound on context_lens; at head dims 64
  * and 128 key ranges longer than 1024 keys are split over up to 8 workgroups
  * when it allows (<= 0: no split; other head dims never split). It sizes the

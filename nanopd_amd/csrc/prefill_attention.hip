@@ -48,8 +48,8 @@
 //
 // What bounds it: power, then issue. 12000 tokens of 32 / 8 heads run at 3009
 // cycles per step against 2048 of MFMA, at 1.8 GHz (all-zero inputs, which draw
-// less, hold 2.4 GHz and take 0.76x the time): 1027 to 1071 us over several
-// boxes = 1.10 to 1.15 PFLOP/s of useful work, where a plain 8192^3 product
+// less, hold 2.4 GHz and take 0.76x the time): 1027 to 1122 us over several
+// boxes = 1.05 to 1.15 PFLOP/s of useful work, where a plain 8192^3 product
 // reaches 1.47. Before (16x16x32 MFMAs, K/V through a register ring, maxima in
 // every step): 1328 to 1383 us. A step without the tile loads takes the same
 // cycles at a higher clock; more operand reads ahead (6 to 12) change nothing;
@@ -88,6 +88,7 @@ constexpr int kWaitVm0 = 0x0f70;       // s_waitcnt vmcnt(0), the other counters
 constexpr float kNoRef = 3.402823466e38f;     // exponent offset of a row without a reference
 constexpr int kSplitSteps = 16;       // a key range longer than this many steps is split
 constexpr int kMaxSplits = 8;
+constexpr int kFixedSplits = 4;       // parts in the fixed order of a full launch
 constexpr int kAhead = 4;             // LDS operand reads ahead of their MFMA
 constexpr int kSlots = 8;             // tiles per lane of the work list
 constexpr int kListTiles = 64 * kSlots;
@@ -1384,8 +1385,12 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   // Up to kListTiles (sequence, tile) pairs the kernel cuts key ranges by the
   // work it finds. More run whole, in a fixed order, unless they leave compute
   // units idle (many short chunks on long prefixes) or one may end the launch
-  // by itself (700 chunks of 60 tokens and one of 256 on a prefix of 32512:
-  // 1630 us whole, 1510 cut).
+  // by itself. Then a part there is not costs an empty workgroup of 1 us, so
+  // these are at most kFixedSplits (32 / 8 heads, whole / 2 / 4 / 8 parts: 700
+  // chunks of 60 tokens and one of 256 on a prefix of 32512 1625 / 1358 / 1340 /
+  // 1509 us, 16 of 2048 and one of 64 on 131072 3302 / 1941 / 1309 / 1169, 40 of
+  // 100 and one of 2048 on 30000, whose tiles fill the chip whole, 952 / 979 /
+  // 1024 / 1148).
   // Three rounds or more of tiles that cannot be cut and are nearly all there
   // need no list either, which costs an item 2 us and more (16 chunks of 512
   // tokens of 32 / 8 heads 150 us by the list, 130 in the fixed order; 300 of 60
@@ -1393,8 +1398,9 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   const bool even = L.splits == 1 && num_seqs * tiles * num_kv_heads >= 3LL * device_cus() &&
                     4 * num_seqs * tiles <= 5 * rows;
   const bool list = num_seqs * tiles <= kListTiles && !even;
-  const bool whole = !list && !tail && total_q * num_heads >= 2LL * device_cus() * tr;
-  const int splits = whole ? 1 : L.splits;
+  const bool full = !list && total_q * num_heads >= 2LL * device_cus() * tr;
+  const int splits = !full ? L.splits : !tail ? 1 : L.splits < kFixedSplits ? L.splits : kFixedSplits;
+  const int ks_steps = splits == L.splits ? L.ks_steps : (int)((longest + splits - 1) / splits);
   // Grid: the tiles there can be, or two rounds of the compute units where the
   // kernel may cut that many parts; a workgroup without an item ends after the
   // work list. Where one of several sequences may outlast the others, its parts
@@ -1435,7 +1441,7 @@ int prefill_impl(void* out, const void* query, const void* key_cache, const void
   a.tiles_max = (int)tiles;
   a.subtiles = (int)(tiles * waves);
   a.splits_max = splits;
-  a.ks_steps = L.ks_steps;
+  a.ks_steps = ks_steps;
   a.list = list;
   a.max_items = (int)max_items;
   a.even_items = (int)even_items;

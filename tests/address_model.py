@@ -86,6 +86,7 @@ def ring_of(D: int, G: int = 1, fp8: bool = False) -> int:
 KT = 64
 SPLIT_STEPS = 16
 MAX_SPLITS = 8
+FIXED_SPLITS = 4
 LIST_TILES = 512       # kListTiles: tiles the in-kernel work list orders
 LIST_BLOCKS = 2048     # kListBlocks: blocks listed in LDS at a time
 MIN_PART, ITEM_STEPS, MERGE_STEPS = 4, 4, 4
@@ -618,8 +619,10 @@ def prefill_host(S, H, KV, bs, max_bps, max_q_len, max_ctx, num_cus=256,
     # the longest context there can be against the mean load of a compute unit
     tail = (_ceil(max_ctx, KT) + ITEM_STEPS) * num_cus > \
         rows * KV * (ITEM_STEPS + tq // max(S, 1) // (2 * KT))
-    if not in_list and not tail and tq * H >= 2 * num_cus * L.rows:
-        L.splits = 1
+    if not in_list and tq * H >= 2 * num_cus * L.rows:
+        splits = min(L.splits, FIXED_SPLITS) if tail else 1
+        if splits < L.splits:
+            L.splits, L.ks_steps = splits, _ceil(_ceil(max_ctx, KT), splits)
     whole = tiles_of(L.rows)
     two = _ceil(2 * num_cus, KV)
     if not in_list:

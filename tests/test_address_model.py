@@ -490,7 +490,8 @@ def test_prefill_tiles_of_flattened_rows(hd, waves):
 def test_a_long_tile_in_a_full_launch_is_cut(q, prefix):
     """32 / 8 heads on 256 compute units: where one sequence's tiles outlast the
     mean load of a unit they run in parts, as long as the mean load or an eighth
-    of the tile (the most parts there are) within 1.3, and every part once."""
+    of the tile (a quarter in the fixed order: the most parts there are) within
+    1.3, and every part once."""
     q, ctx = np.array(q), np.array(q) + np.array(prefix)
     cu = np.concatenate([[0], np.cumsum(q)])
     L = A.prefill_host(len(q), H, KV, BS, int(-(-ctx.max() // BS)), int(q.max()), int(ctx.max()),
@@ -512,7 +513,7 @@ def test_a_long_tile_in_a_full_launch_is_cut(q, prefix):
         assert js == set(range(len(js)))
     mean, nmax = sum(steps.values()) / units, max(steps.values())
     assert nmax > 1.3 * mean   # whole tiles would be the launch
-    assert longest <= 1.3 * max(mean, nmax / 8)
+    assert longest <= 1.3 * max(mean, nmax / (8 if L.work_list else 4))
 
 
 @pytest.mark.parametrize("q,prefix,listed", [

@@ -13,7 +13,7 @@ multiple of 32 up to 1024 (PA/csrc/attention/paged_attention_kernel.cu:16-20,
   / 1e-2 (bf16) of the float64 oracle, split partitions and the merge
   included;
 * chunked prefill takes multiples of 32 from 32 to 256 (the generic MFMA
-  kernel at every head dim but 64 and 128): same tolerance, paged prefixes,
+  kernel at every head dim but 64, 128 and, over 2-byte pools, 256): same tolerance, paged prefixes,
   ragged chunks, decode rows, rows before position 0, and the FP8 pool.
 """
 import math
